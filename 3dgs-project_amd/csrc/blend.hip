@@ -13,6 +13,7 @@
 // sequence (the purpose of Faster-GS's per-subtile culling, phase1/fastergs_macro.patch:92-104).
 #include <limits.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "gs_host.h"
@@ -60,11 +61,9 @@ __device__ __forceinline__ uint32_t strip_mask(const int4 d, int tile_y0) {
 // the blends' own float32 evaluation of the boundary (the hardware exp2 included), so a strip is
 // dropped only where every pixel has alpha < 1/255: the blends' results do not change. Splats
 // with a condition number above about 4096 keep ymask (det then loses too many bits).
-// Evaluated for the strips in `want` only (a forward wavefront needs its own strip).
-__device__ __forceinline__ uint32_t strip_mask_band(const float* rp, int tile_x0, int tile_y0, uint32_t ymask,
-                                                    uint32_t want = 0xfu) {
-  ymask &= want;
-  const float mx = rp[0], my = rp[1], A = rp[2], B = rp[3], C = rp[4], thr = rp[7];
+// off: the pixel centres' offset (a pixel's centre is at its index + off).
+__device__ __forceinline__ uint32_t strip_mask_ellipse(float mx, float my, float A, float B, float C, float thr,
+                                                       float off, int tile_x0, int tile_y0, uint32_t ymask) {
   const float det = fmaf(A, C, -(B * B));
   const float t = A + C;
   if (ymask == 0u || !(det > 0.0f) || !(A > 0.0f) || !(C > 0.0f) || !(thr > 0.0f) || t * t >= 4096.0f * det)
@@ -74,13 +73,13 @@ __device__ __forceinline__ uint32_t strip_mask_band(const float* rp, int tile_x0
   const float umax = fmaf(__builtin_amdgcn_sqrtf(q * idet), 1.001f, 0.05f);
   const float us = -B * __builtin_amdgcn_sqrtf((thr + thr) * __builtin_amdgcn_rcpf(C) * idet);
   const float iA = __builtin_amdgcn_rcpf(A);
-  const float c0 = (static_cast<float>(tile_x0) + 0.5f) - mx;  // the tile's columns, from the mean
+  const float c0 = (static_cast<float>(tile_x0) + off) - mx;  // the tile's columns, from the mean
   const float c1 = c0 + static_cast<float>(kTile - 1);
   uint32_t m = 0;
 #pragma unroll
   for (int s = 0; s < kStrips; ++s) {
     if (((ymask >> s) & 1u) == 0u) continue;
-    const float ya = (static_cast<float>(tile_y0 + kStripRows * s) + 0.5f) - my;
+    const float ya = (static_cast<float>(tile_y0 + kStripRows * s) + off) - my;
     const float ua = fmaxf(ya, -umax), ub = fminf(ya + static_cast<float>(kStripRows - 1), umax);
     if (ua > ub) continue;
     const float ur = fminf(fmaxf(us, ua), ub), ul = fminf(fmaxf(-us, ua), ub);
@@ -91,6 +90,38 @@ __device__ __forceinline__ uint32_t strip_mask_band(const float* rp, int tile_x0
     if (fr + mg >= c0 && fl - mg <= c1) m |= 1u << s;
   }
   return m;
+}
+
+// ... of a 3D splat record, for the strips in `want` only.
+__device__ __forceinline__ uint32_t strip_mask_band(const float* rp, int tile_x0, int tile_y0, uint32_t ymask,
+                                                    uint32_t want = 0xfu) {
+  return strip_mask_ellipse(rp[0], rp[1], rp[2], rp[3], rp[4], rp[7], 0.5f, tile_x0, tile_y0, ymask & want);
+}
+
+// ln(255 o), rounded up by far more than its error and a kernel's own rounding of the exponent: a
+// 2D splat of opacity o has alpha < 1/255 wherever its exponent is not above -thr (NaN for an
+// opacity that is not positive: no exponent is above that).
+template <typename S>
+__device__ __forceinline__ float alpha_reach(S o) {
+  const float t = __builtin_amdgcn_logf(255.0f * static_cast<float>(o)) * kLn2;
+  return fmaf(fabsf(t), 1e-5f, t + 1e-4f);
+}
+
+// The strips of a tile that a 2D splat (toy2d: conic, phase0: Cholesky factors) can reach, in
+// float32 also for float64 records (the margins cover the difference).
+template <int R, typename S>
+__device__ __forceinline__ uint32_t strip_mask_2d(const Staged<S>& s, float thr, int tile_x0, int tile_y0,
+                                                  uint32_t want = 0xfu) {
+  float A = static_cast<float>(s.s0), B = static_cast<float>(s.s1), C = static_cast<float>(s.s2);
+  if constexpr (R == kRulesPhase0) {  // Q = L L^T of a = l0 dx + l1 dy, b = l2 dy
+    const float l0 = A, l1 = B, l2 = C;
+    A = l0 * l0;
+    B = l0 * l1;
+    C = fmaf(l1, l1, l2 * l2);
+  }
+  if (!(fmaf(A, C, -(B * B)) > 1e-30f)) return want;  // (the approximate reciprocals need a normal range)
+  return strip_mask_ellipse(static_cast<float>(s.mx), static_cast<float>(s.my), A, B, C, thr,
+                            static_cast<float>(Rule<R, S>::pix_off()), tile_x0, tile_y0, want);
 }
 
 template <typename S>
@@ -137,6 +168,19 @@ __device__ __forceinline__ void count_add(unsigned long long* c, uint32_t v) {
   uint32_t s = v;
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   if ((threadIdx.x & 63) == 0 && s) atomicAdd(c, static_cast<unsigned long long>(s));
+}
+
+// Counter increment by a workgroup's sum (one atomic per workgroup; every thread calls it).
+__device__ __forceinline__ void block_count_add(unsigned long long v, unsigned long long* c) {
+  __shared__ unsigned long long s_w[1024 / kWave];
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < static_cast<int>(blockDim.x) / kWave; ++w) v += s_w[w];
+    if (v) atomicAdd(c, v);
+  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -556,6 +600,138 @@ __global__ __launch_bounds__(4 * kWave) void blend_fwd_strip_kernel(BlendArgs<fl
   }
 }
 
+// Forward of the 2D rule sets: the strip kernel's split (a wavefront per 4-row strip, a pixel per
+// lane, the wavefront staging the tile's list 64 entries at a time in its own LDS and ending on its
+// own 64 pixels), with the rule sets' own arithmetic, decision for decision that of
+// blend_fwd_kernel. The 2D tile lists hold every tile of a splat's rectangle, so most of a list's
+// entries reach few of a tile's pixels: an entry is skipped for a strip its ellipse misses (a
+// scalar bit), and its exponential is not evaluated where no lane's exponent is above
+// -ln(255 o).
+//
+// Checkpoints: with the shared staging a workgroup stopped at the first multiple of 256 entries
+// at which all its pixels had stopped; buckets before that hold the pixels' states, those after
+// it zeros (toy2d) or the final states (phase0). Here the wavefronts end on their own, and the
+// tail of the checkpoints is written once the workgroup's stop is known.
+template <int R, typename S>
+__global__ __launch_bounds__(4 * kWave) void blend_fwd_strip2d_kernel(BlendArgs<S> a) {
+  using Ru = Rule<R, S>;
+  __shared__ Staged<S> s_sp[4][kWave];
+  __shared__ int s_stop[4], s_last[4];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int tile = blockIdx.x;
+  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x;
+  Staged<S>* sw = s_sp[wave];
+  const uint32_t r0 = a.ranges[static_cast<int64_t>(tile) * a.range_stride];
+  const uint32_t r1 = a.ranges[static_cast<int64_t>(tile) * a.range_stride + 1];
+  const int len = static_cast<int>(r1 - r0);
+  const int px = tx * kTile + (lane & 15), py = ty * kTile + kStripRows * wave + (lane >> 4);
+  const bool inside = px < a.W && py < a.H;
+  const S pxf = static_cast<S>(px) + Ru::pix_off(), pyf = static_cast<S>(py) + Ru::pix_off();
+  S* ck = a.ckpt ? a.ckpt + (static_cast<int64_t>(a.bucket_offsets[tile]) * kTilePixels + kWave * wave + lane) * 4
+                 : nullptr;
+  S T = S(1), Cr = S(0), Cg = S(0), Cb = S(0);
+  int last = 0, count = 0, stop_at = 0;  // stop_at: list entries up to the pixel's stop
+  bool done = !inside;
+  auto store_ck = [&](int q, S c0, S c1, S c2, S c3) {
+    S* c = ck + static_cast<int64_t>(q) * kTilePixels * 4;
+    if constexpr (sizeof(S) == 4) {
+      *reinterpret_cast<float4*>(c) = make_float4(c0, c1, c2, c3);
+    } else {
+      reinterpret_cast<double2*>(c)[0] = make_double2(c0, c1);
+      reinterpret_cast<double2*>(c)[1] = make_double2(c2, c3);
+    }
+  };
+  auto store_state = [&](int q) {
+    if constexpr (Ru::kCkptTFirst) store_ck(q, T, Cr, Cg, Cb);
+    else store_ck(q, Cr, Cg, Cb, T);
+  };
+  int written = 0;  // buckets whose checkpoints are written
+  bool stopped = __ballot(done ? 0 : 1) == 0ull;
+  for (int b0 = 0; b0 < len && !stopped; b0 += kWave) {
+    wave_sync();  // every lane is done with the previous batch
+    const int j = b0 + lane;
+    uint32_t hit = 0;
+    if (j < len) {
+      Staged<S> sp = Ru::stage(a.rec + static_cast<int64_t>(a.point_list[r0 + j]) * kRecFloats);
+      const float thr = alpha_reach(sp.o);
+      sp.n0 = static_cast<S>(-thr);
+      sw[lane] = sp;
+      hit = strip_mask_2d<R, S>(sp, thr, tx * kTile, ty * kTile, 1u << wave);
+    }
+    const uint64_t wm = __ballot(hit ? 1 : 0);
+    wave_sync();
+    const int nb = min(kWave, len - b0);
+    for (int c0 = 0; c0 < nb; c0 += kBucket) {
+      if (ck) store_state(written);
+      ++written;
+      uint32_t cm = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(wm >> c0));
+      const Staged<S>* bp = sw + c0;
+      while (cm != 0u) {
+        const int k = __builtin_ctz(cm);
+        cm &= cm - 1u;
+        const Staged<S>& sp = bp[k];
+        Eval<S> e;
+        const S pw = Ru::exponent(sp, pxf, pyf, e);
+        const bool reach = !done && Ru::in_domain(pw) && pw > sp.n0;
+        if (__ballot(reach ? 1 : 0) == 0ull) continue;  // wave-uniform
+        Ru::alpha_of(sp, pw, e);
+        if (reach && e.alpha >= Ru::alpha_min()) {
+          if (Ru::kStopBefore && T * (S(1) - e.alpha) < Ru::t_stop()) {
+            done = true;
+            stop_at = b0 + c0 + k + 1;
+          } else {
+            composite<R, S>(Cr, Cg, Cb, T, sp, e.alpha);
+            last = b0 + c0 + k + 1;
+            ++count;
+            if (!Ru::kStopBefore && T < Ru::t_stop()) {
+              done = true;
+              stop_at = last;
+            }
+          }
+        }
+      }
+      if (__ballot(done ? 0 : 1) == 0ull) {
+        stopped = true;
+        break;
+      }
+    }
+  }
+  if (lane == 0) s_stop[wave] = len;
+  const int wstop = wave_max(stop_at), wlast = wave_max(last);
+  if (lane == 0) {
+    if (stopped) s_stop[wave] = wstop;
+    s_last[wave] = wlast;
+  }
+  __syncthreads();
+  if (ck) {
+    const int stop = max(max(s_stop[0], s_stop[1]), max(s_stop[2], s_stop[3]));
+    const int covered = min(len, (stop + kTilePixels - 1) / kTilePixels * kTilePixels);
+    for (int q = written; q < (len + kBucket - 1) / kBucket; ++q) {
+      if (R == kRulesPhase0 || q * kBucket < covered) store_state(q);
+      else store_ck(q, S(0), S(0), S(0), S(0));
+    }
+  }
+  if (inside) {
+    const int64_t pix = static_cast<int64_t>(py) * a.W + px;
+    if constexpr (Ru::kInterleaved) {
+      a.image[3 * pix] = Cr;
+      a.image[3 * pix + 1] = Cg;
+      a.image[3 * pix + 2] = Cb;
+    } else {
+      const int64_t HW = static_cast<int64_t>(a.H) * a.W;
+      a.image[pix] = fma(T, a.bg0, Cr);
+      a.image[HW + pix] = fma(T, a.bg1, Cg);
+      a.image[2 * HW + pix] = fma(T, a.bg2, Cb);
+    }
+    a.final_T[pix] = T;
+    if (a.n_contrib) a.n_contrib[pix] = Ru::kCountContrib ? count : last;
+    if (a.last_contrib) a.last_contrib[pix] = last;
+  }
+  if (threadIdx.x == 0 && a.tile_max)
+    a.tile_max[tile] = static_cast<uint32_t>(max(max(s_last[0], s_last[1]), max(s_last[2], s_last[3])));
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
@@ -596,7 +772,7 @@ __device__ __forceinline__ void wave_reduce12(const float* v, float& u0, float& 
 }
 
 template <int CTRL>
-__device__ __forceinline__ double dpp64(double v) {
+__device__ __forceinline__ double dpp(double v) {
   const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
   const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(u & 0xffffffffu), CTRL,
                                                                           0xf, 0xf, false));
@@ -615,7 +791,37 @@ __device__ __forceinline__ double f64_of(uint32_t lo, uint32_t hi) {
   return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
 }
 
-// Reduction of one bucket-splat step of the 3D backward without the |dL/dmean2d| sums. In: the
+// a + b of the pair that v_permlane32_swap (v_permlane16_swap) leaves in each lane: the lower half
+// (the even rows) sums a with its partner's a, the upper half (the odd rows) b with its partner's b.
+__device__ __forceinline__ float swap32_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap16_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double swap32_add(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane32_swap(lo32(a), lo32(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(hi32(a), hi32(b), false, false);
+  return f64_of(l[0], h[0]) + f64_of(l[1], h[1]);
+}
+__device__ __forceinline__ double swap16_add(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane16_swap(lo32(a), lo32(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi32(a), hi32(b), false, false);
+  return f64_of(l[0], h[0]) + f64_of(l[1], h[1]);
+}
+
+// Lane 16's value in every lane.
+__device__ __forceinline__ float read_lane16(float v) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 16));
+}
+__device__ __forceinline__ double read_lane16(double v) {
+  return f64_of(__builtin_amdgcn_readlane(lo32(v), 16), __builtin_amdgcn_readlane(hi32(v), 16));
+}
+
+// Reduction of one bucket-splat step (the 3D backward without the |dL/dmean2d| sums, and the 2D
+// rule sets). In: the
 // lane's sums over its 4 pixels (one column) of h, h dy, h dy^2 and the three colour sums, and
 // the column's dx. The 4 lanes of a column (lane ^ 16, ^ 32) are summed first, transposing: xor
 // 32 with v_permlane32_swap over the pairs (h, red), (h dy, green), (h dy^2, blue), leaving the
@@ -628,33 +834,15 @@ __device__ __forceinline__ double f64_of(uint32_t lo, uint32_t hi) {
 //   g 0: (sum h dx, sum h dy)          g 1: (sum h dx^2, sum h dx dy)
 //   g 2: (sum h, sum h dy^2)           g 4: (red, green)       g 6: (red, blue)
 // (g 3, 5, 7 hold repeats). 27 instructions, the dx products included.
-__device__ __forceinline__ void wave_reduce_cols(float sh, float shy, float shyy, float cr, float cg, float cb,
-                                                 float dx, bool row0, float& u0, float& u1) {
+template <typename S>
+__device__ __forceinline__ void wave_reduce_cols(S sh, S shy, S shyy, S cr, S cg, S cb, S dx, bool row0, S& u0,
+                                                 S& u1) {
   const int lane = threadIdx.x & 63;
-  float s0, s1, s2;
-  {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(sh), __float_as_uint(cr), false, false);
-    s0 = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(shy), __float_as_uint(cg), false, false);
-    s1 = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(shyy), __float_as_uint(cb), false, false);
-    s2 = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-  float t0, t1;
-  {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s0), __float_as_uint(s0), false, false);
-    t0 = __uint_as_float(r[0]) + __uint_as_float(r[1]);  // every row: its quarter's first sum
-  }
-  {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s1), __float_as_uint(s2), false, false);
-    t1 = __uint_as_float(r[0]) + __uint_as_float(r[1]);  // even rows s1, odd rows s2
-  }
-  const float f = row0 ? dx : 1.0f;
-  const float v0 = t0 * f, v1 = v0 * f, v3 = t1 * f;
+  const S s0 = swap32_add(sh, cr), s1 = swap32_add(shy, cg), s2 = swap32_add(shyy, cb);
+  const S t0 = swap16_add(s0, s0);  // every row: its quarter's first sum
+  const S t1 = swap16_add(s1, s2);  // even rows s1, odd rows s2
+  const S f = row0 ? dx : S(1);
+  const S v0 = t0 * f, v1 = v0 * f, v3 = t1 * f;
   const bool b3 = (lane & 8) != 0;
   u0 = (b3 ? v1 : v0) + dpp<0x128>(b3 ? v0 : v1);  // row_ror:8 = partner lane ^ 8
   u1 = (b3 ? v3 : t1) + dpp<0x128>(b3 ? t1 : v3);
@@ -683,67 +871,6 @@ __device__ __forceinline__ void wave_reduce12(const double* v, double& u0, doubl
   }
 }
 
-// Raw per-pair sums of the bucketed backward (the splat-constant factors are applied once
-// per splat in finish_grad): [0] sum h dx (phase0: h a), [1] sum h dy (phase0: h b),
-// [2] sum h dx dx (h a dx), [3] sum h dx dy (h a dy), [4] sum h dy dy (h b dy), [5] sum G dL/dalpha,
-// [6..8] colour, [9..10] |dL/dmean| (3D); h = alpha dL/dalpha = dL/dpower.
-template <int R, typename S>
-__device__ __forceinline__ void pair_sums(const Staged<S>& s, const Eval<S>& e, S dLda, S* acc) {
-  if (e.clamped) return;
-  acc[5] = fma(e.G, dLda, acc[5]);
-  const S h = e.alpha * dLda;
-  S hx, hy;
-  if constexpr (R == kRulesPhase0) {
-    hx = h * e.a;
-    hy = h * e.b;
-    acc[2] = fma(hx, e.dx, acc[2]);
-    acc[3] = fma(hx, e.dy, acc[3]);
-    acc[4] = fma(hy, e.dy, acc[4]);
-  } else {
-    hx = h * e.dx;
-    hy = h * e.dy;
-    acc[2] = fma(hx, e.dx, acc[2]);
-    acc[3] = fma(hx, e.dy, acc[3]);
-    acc[4] = fma(hy, e.dy, acc[4]);
-    if constexpr (R == kRules3D) {
-      acc[9] += fabs(fma(s.n0, hx, s.n1 * hy));
-      acc[10] += fabs(fma(s.n1, hx, s.nat2 * hy));
-    }
-  }
-  acc[0] += hx;
-  acc[1] += hy;
-}
-
-// Final gradient of value index k from its total u (u0, u1: totals of indices 0 and 1).
-template <int R, typename S>
-__device__ __forceinline__ S finish_grad(const Staged<S>& s, int k, S u, S u0, S u1) {
-  if constexpr (R == kRulesPhase0) {
-    // power = -(a^2 + b^2) / 2 with a = l0 dx + l1 dy, b = l2 dy, d = pixel - mean
-    if (k == 0) return s.s0 * u0;
-    if (k == 1) return fma(s.s1, u0, s.s2 * u1);
-    if (k >= 2 && k <= 4) return -u;
-    if (k == 5) return u * s.o * (S(1) - s.o);  // dL/dlogit = dL/do o (1 - o)
-    return u;
-  } else {
-    S A, B, C;
-    if constexpr (R == kRules3D) {
-      A = s.n0;
-      B = s.n1;
-      C = s.nat2;
-    } else {
-      A = s.s0;
-      B = s.s1;
-      C = s.s2;
-    }
-    // power = -1/2 (A dx^2 + 2 B dx dy + C dy^2), d = mean - pixel
-    if (k == 0) return -fma(A, u0, B * u1);
-    if (k == 1) return -fma(B, u0, C * u1);
-    if (k == 2 || k == 4) return S(-0.5) * u;
-    if (k == 3) return -u;
-    return u;
-  }
-}
-
 // ---------------------------------------------------------------------------------------
 // Bucketed backward
 // ---------------------------------------------------------------------------------------
@@ -767,11 +894,12 @@ static_assert(sizeof(Staged<float>) == 48 && offsetof(Staged<float>, n0) == 36 &
 // kAbs (3D): also accumulate |dL/dmean2d| (grad2d slots 9-10) for densification by absolute
 // gradient, as Faster-GS's compute_abs_grad instantiation does; without it those slots are
 // left untouched.
-// One bucket b, by one wavefront (whose LDS slots are s_sp, s_m, s_id).
-template <int R, typename S, bool kCount, bool kAbs>
-__device__ __forceinline__ void bwd_bucket(const BlendArgs<S>& a, int64_t b, Staged<S>* s_sp, uint32_t* s_m,
-                                           uint32_t* s_id, float* s_c, uint32_t& evals, uint32_t& atomics) {
-  using Ru = Rule<R, S>;
+// One bucket b, by one wavefront (whose LDS slots are s_sp, s_id and s_c): 3D.
+template <bool kCount, bool kAbs>
+__device__ __forceinline__ void bwd_bucket_3d(const BlendArgs<float>& a, int64_t b, Staged<float>* s_sp,
+                                              uint32_t* s_id, float* s_c, uint32_t& evals, uint32_t& atomics) {
+  using S = float;
+  using Ru = Rule<kRules3D, S>;
   constexpr int NV = Ru::kGradVals;
   // (opaque: in the striding kernel the lane's constants are then formed per bucket instead of
   // being hoisted out of its loop and held in registers across it)
@@ -787,21 +915,13 @@ __device__ __forceinline__ void bwd_bucket(const BlendArgs<S>& a, int64_t b, Sta
   if (bsize <= 0) return;
   const int tx = static_cast<int>(tile) % a.tiles_x, ty = static_cast<int>(tile) / a.tiles_x;
 
-  uint32_t mk_lane = 0;  // the strip mask of this lane's staged splat (3D)
+  uint32_t mk_lane = 0;  // the strip mask of this lane's staged splat
   if (lane < bsize) {
     const uint32_t g = a.point_list[r0 + bstart + lane];
     const S* rp = a.rec + static_cast<int64_t>(g) * kRecFloats;
     s_sp[lane] = Ru::stage(rp);
-    if constexpr (Ru::kStrips) {
-      uint32_t mk = strip_mask(reinterpret_cast<const int4*>(rp)[3], ty * kTile);
-      if constexpr (R == kRules3D) {
-        mk = strip_mask_band(rp, tx * kTile, ty * kTile, mk);
-        if (a.conic64 && elongated(rp)) mk |= kElongBit;
-        mk_lane = mk;
-      } else {
-        s_m[lane] = mk;
-      }
-    }
+    mk_lane = strip_mask_band(rp, tx * kTile, ty * kTile, strip_mask(reinterpret_cast<const int4*>(rp)[3], ty * kTile));
+    if (a.conic64 && elongated(rp)) mk_lane |= kElongBit;
     s_id[lane] = g;
   }
 
@@ -823,13 +943,381 @@ __device__ __forceinline__ void bwd_bucket(const BlendArgs<S>& a, int64_t b, Sta
     lim[r] = 0;
     if (px < a.W && py < a.H) {
       const int64_t pix = static_cast<int64_t>(py) * a.W + px;
-      // phase0 without a limit table: every inside pixel replays the bucket and stops by the
-      // T < 1e-4 rule (phase0/csrc/macrotile/splat2d_bwd_splat.cu:69)
-      const int32_t* lp = a.last_contrib ? a.last_contrib : a.n_contrib;
-      const int used = lp ? lp[pix] - bstart : kBucket;
+      const int used = a.n_contrib[pix] - bstart;
       if (used > 0) {
         lim[r] = used;
         lim_max = max(lim_max, used);
+        Gr[r] = a.grad_image[pix];
+        Gg[r] = a.grad_image[HW + pix];
+        Gb[r] = a.grad_image[2 * HW + pix];
+        const S* c = a.ckpt + (b * kTilePixels + kWave * r + lane) * 4;
+        T[r] = c[3];
+        // rho = G . (image - C): the colour still to come (background included)
+        rho[r] = Gr[r] * (a.image[pix] - c[0]) + Gg[r] * (a.image[HW + pix] - c[1]) +
+                 Gb[r] * (a.image[2 * HW + pix] - c[2]);
+        // alpha = 1 - T_final output: its gradient enters like a background term
+        if (a.grad_alpha) rho[r] -= a.grad_alpha[pix] * a.final_T[pix];
+      }
+    }
+  }
+  if constexpr (!kAbs) {
+    // the coefficient pair of each lane's gradient, g = -(c0 u0 + c1 u1) of the reduction's totals
+    // (u0, u1); lanes 0 and 1 read theirs, the splat's (A, B) and (B, C), from the staged splat,
+    // lane l >= 2 reads (t[l], t[l + 1]) of this table (consecutive words: no bank conflicts): the
+    // owners' pairs are lane 8 (1/2, 0), 9 (0, 1), 16 (-1, 0), 17 (0, 1/2), 32 (-1, 0), 33 (0, -1),
+    // 49 (0, -1), all others (0, 0)
+    float* kt = reinterpret_cast<float*>(s_sp + kBucket);
+    kt[lane] = lane == 8 || lane == 18 ? 0.5f
+               : lane == 10            ? 1.0f
+               : (lane == 16 || lane == 32 || lane == 34 || lane == 50) ? -1.0f
+                                                                       : 0.0f;
+    if (lane == 0) kt[kWave] = 0.0f;
+  }
+  // (scalar: the splat loop is uniform over the wavefront)
+  const int jmax = __builtin_amdgcn_readfirstlane(min(bsize, wave_max(lim_max)));
+  wave_sync();
+
+  // value index k owned by this lane after wave_reduce12 (lo = 0 or 1 within the 8-lane group)
+  const int grp = lane >> 3, lo = lane & 7;
+  const int kidx = 6 * (grp >> 2) + 3 * ((grp >> 1) & 1) + 2 * (grp & 1) + lo;
+  const bool owner = lo < 2 && (2 * (grp & 1) + lo) < 3 && kidx < NV;
+  // The lane's 4 pixels share a column: the column terms of the power and of the mean
+  // gradient are computed once per splat, and per pixel only dy-dependent sums are kept;
+  // the dx factors are applied in the reduction, once per column. Pixel r of every
+  // lane lies in strip r, so the strip test and the wavefront's largest limit of row r are
+  // scalar; inside, the pixel body has no branches: a lane past its limit or below the
+  // alpha threshold blends alpha = 0, which leaves its T, rho and every sum unchanged.
+  // dL/dopacity = sum G dL/dalpha = (sum alpha dL/dalpha) / o: the sum h is reduced instead.
+  int lim_row[kPixPerLane];
+#pragma unroll
+  for (int r = 0; r < kPixPerLane; ++r) lim_row[r] = __builtin_amdgcn_readfirstlane(wave_max(lim[r]));
+  // the staged splats' strip bits and elongation bit as scalar bit planes (bit j: splat j), so
+  // the per-splat tests below are scalar bit tests with no LDS read
+  uint64_t plane[kPixPerLane + 1];
+#pragma unroll
+  for (int r = 0; r < kPixPerLane; ++r) plane[r] = __ballot(((mk_lane >> r) & 1u) ? 1 : 0);
+  plane[kPixPerLane] = __ballot((mk_lane & kElongBit) ? 1 : 0);
+  // With |dL/dmean2d| (kAbs) the 12 sums are reduced by wave_reduce12 and the final gradient of
+  // the lane's value index k is c0 u0 + c1 u1 + c u (u = its own total): k 0, 1 (mean2d):
+  // -(A u0 + B u1), -(B u0 + C u1); k 2, 4: -u/2; k 3: -u; k 5 (opacity): u; colour and
+  // |dL/dmean2d|: u. Without, wave_reduce_cols leaves two totals (u0, u1) in each 8-lane group
+  // and the gradient of a lane is -(c0 u0 + c1 u1): lanes 0 and 1 the mean2d values from
+  // (sum h dx, sum h dy), with (c0, c1) = (A, B) and (B, C) read from the staged splat; lanes 8
+  // and 9 the conic A and B (-u0/2, -u1), lanes 16 and 17 the opacity (u0) and the conic C
+  // (-u1/2), lanes 32, 33 and 49 the colour, their pairs read from a table of constants.
+  // The opacity column holds sum h = sum alpha dL/dalpha = opacity dL/dopacity: the preprocess
+  // backward divides by the opacity once per Gaussian (in float64) instead of every
+  // bucket-splat step here. The lane-constant parts are chosen here.
+  const bool k0 = kidx == 0, k1 = kidx == 1;  // (kAbs) the lanes of the two mean2d values
+  int kslot;  // the grad2d column of the lane's gradient (-1: none)
+  float kc = 0.0f;
+  if constexpr (kAbs) {
+    kslot = owner ? kidx : -1;
+    kc = (kslot == 2 || kslot == 4) ? -0.5f : kslot == 3 ? -1.0f : kslot >= 5 ? 1.0f : 0.0f;
+  } else {
+    kslot = lane == 0    ? 0
+            : lane == 1  ? 1
+            : lane == 8  ? 2
+            : lane == 9  ? 3
+            : lane == 16 ? 5
+            : lane == 17 ? 4
+            : lane == 32 ? 6
+            : lane == 33 ? 7
+            : lane == 49 ? 8
+                         : -1;
+  }
+  // (without kAbs) the float index of the lane's coefficient pair in s_sp, j * m01 + cidx:
+  // lanes 0 and 1 in staged splat j, the others in the table after the staged splats
+  constexpr int kStagedFloats = static_cast<int>(sizeof(Staged<S>) / sizeof(S));
+  const int m01 = lane < 2 ? kStagedFloats : 0;
+  const int cidx = lane < 2 ? static_cast<int>(offsetof(Staged<S>, n0) / sizeof(S)) + lane
+                            : kBucket * kStagedFloats + lane;
+  const bool row0 = lane < 16;
+  const bool live_owner = kslot >= 0;
+  const bool conic_owner = kslot >= 2 && kslot <= 4;
+  const int64_t kofs = kslot;
+  for (int j = 0; j < jmax; ++j) {
+    const Staged<S> sp = s_sp[j];
+    const typename Ru::Col cl = Ru::col(sp, pxf);
+    const float n0dx = sp.n0 * cl.dx, n1dx = sp.n1 * cl.dx;
+    // zeros the compiler cannot see through: each sum then lives in one register from its
+    // zero to its last update, instead of being re-zeroed on every path that skips a pixel
+    float sh, shy, shyy, cr, cg, cb;
+    opaque_zero2(sh, shy);
+    opaque_zero2(shyy, cr);
+    opaque_zero2(cg, cb);
+    float ab0 = 0.0f, ab1 = 0.0f;
+    if constexpr (kAbs) {
+      ab0 = opaque_zero();
+      ab1 = opaque_zero();
+    }
+    uint64_t used = 0;  // the lanes that blended the splat (a lane mask: scalar)
+#pragma unroll
+    for (int r = 0; r < kPixPerLane; ++r) {
+      if (((plane[r] >> j) & 1u) == 0u || j >= lim_row[r]) continue;  // wave-uniform
+      const bool live = j < lim[r];
+      if constexpr (kCount) evals += live ? 1u : 0u;
+      const float dy = sp.my - pyf[r];
+      const float G = Ru::falloff(Ru::power(sp, cl, dy));
+      const float a_raw = sp.o * G;
+      const bool above = a_raw >= kAlphaMin;
+      const bool take = live && above;
+      // (the masks of the two compares themselves: a ballot of their conjunction would first
+      // turn it into a per-lane value)
+      used |= __builtin_amdgcn_ballot_w64(live) & __builtin_amdgcn_ballot_w64(above);
+      const float alpha = take ? a_raw : 0.0f;
+      const float w = T[r] * alpha;
+      const float dot = fmaf(Gb[r], sp.cb, fmaf(Gg[r], sp.cg, Gr[r] * sp.cr));
+      cr = fmaf(w, Gr[r], cr);
+      cg = fmaf(w, Gg[r], cg);
+      cb = fmaf(w, Gb[r], cb);
+      rho[r] = fmaf(-w, dot, rho[r]);
+      const float oma = 1.0f - alpha;
+      const float dLda = fmaf(T[r], dot, -(rho[r] * __builtin_amdgcn_rcpf(fmaxf(oma, kOneMinusAlphaEps))));
+      const float h = alpha * dLda;  // dL/dpower
+      const float hy = h * dy;
+      sh += h;
+      shy += hy;
+      shyy = fmaf(hy, dy, shyy);
+      if constexpr (kAbs) {
+        ab0 = fmaf(fabsf(h), fabsf(fmaf(sp.n1, dy, n0dx)), ab0);
+        ab1 = fmaf(fabsf(h), fabsf(fmaf(sp.nat2, dy, n1dx)), ab1);
+      }
+      T[r] = T[r] * oma;
+    }
+    if (used == 0) continue;
+    const bool wide = ((plane[kPixPerLane] >> j) & 1u) != 0u;  // wave-uniform
+    if (wide) {
+      // each lane parks the conic sums of its pixels, read back after the float32 reduction
+      const float dxsh = cl.dx * sh;
+      s_c[lane] = cl.dx * dxsh;
+      s_c[kWave + lane] = cl.dx * shy;
+      s_c[2 * kWave + lane] = shyy;
+    }
+    float g;
+    if constexpr (kAbs) {
+      const float dxsh = cl.dx * sh;
+      const float cxx = cl.dx * dxsh, cxy = cl.dx * shy;  // the conic sums of the lane's column
+      const float c0 = k0 ? -sp.n0 : k1 ? -sp.n1 : 0.0f;
+      const float c1 = k0 ? -sp.n1 : k1 ? -sp.nat2 : 0.0f;
+      S acc[12] = {dxsh, shy, cxx, cxy, shyy, sh, cr, cg, cb, ab0, ab1, 0.0f};
+      S u0, u1;
+      wave_reduce12(acc, u0, u1);
+      g = fmaf(c0, u0, fmaf(c1, u1, kc * (lo == 0 ? u0 : u1)));
+    } else {
+      float u0, u1;
+      wave_reduce_cols(sh, shy, shyy, cr, cg, cb, cl.dx, row0, u0, u1);
+      const S* cp = reinterpret_cast<const S*>(s_sp) + (j * m01 + cidx);
+      g = fmaf(-cp[0], u0, -(cp[1] * u1));
+    }
+    // (an elongated splat's conic sums go to the float64 buffer below instead)
+    if (live_owner && !(wide && conic_owner))
+      atomic_add_grad(a.grad_rec + static_cast<int64_t>(s_id[j]) * kGrad2D + kofs, g);
+    if (wide) {  // the conic sums in float64
+      const uint32_t id = __builtin_amdgcn_readfirstlane(s_id[j]);  // wave-uniform
+      wave_sync();  // every lane's parked values
+      // row k of 16 lanes (k < 3) sums value k of the 64 lanes: 4 values per lane in float64
+      // (exactly), then the row's 16 partial sums; A, B, C = -1/2, -1, -1/2 times the sums of
+      // dx^2 h, dx dy h, dy^2 h
+      int ln = lane;
+      asm volatile("" : "+v"(ln));  // formed here, not kept in registers over the whole loop
+      const int k = ln >> 4, r16 = ln & 15;
+      double t = 0.0;
+      if (k < 3) {
+        const float* v = s_c + k * kWave + r16;
+        t = (static_cast<double>(v[0]) + static_cast<double>(v[16])) +
+            (static_cast<double>(v[32]) + static_cast<double>(v[48]));
+      }
+      t += dpp<0x128>(t);  // row_ror:8
+      t += dpp<0x141>(t);  // row_half_mirror
+      t += dpp<0xB1>(t);   // quad_perm [1,0,3,2]
+      t += dpp<0x4E>(t);   // quad_perm [2,3,0,1]
+      if (r16 == 0 && k < 3) atomic_add_grad(a.conic64 + 4 * static_cast<uint64_t>(id) + k, (k == 1 ? -1.0 : -0.5) * t);
+      // marks the splat's row for the preprocess backward, which then adds the float64 sums
+      if (lane == 48) a.grad_rec[static_cast<uint64_t>(id) * kGrad2D + 11] = 1.0f;
+      wave_sync();  // the parked values are read before the next splat parks its own
+    }
+    if constexpr (kCount) atomics += kAbs ? NV : 9;
+  }
+}
+
+// kList 0: wavefront i takes bucket i of the table. With a.bucket_list (3D), the forward's list
+// of the buckets with blended entries: kList 1, wavefront i takes entry i (a wavefront past the
+// list's length only reads that length); kList 2, a bounded grid strides over the list (the
+// loop keeps more registers live, so it is used only when the table is much longer).
+template <bool kCount, bool kAbs, int kList>
+__global__ __launch_bounds__(bwd_waves<kRules3D>() * kWave) void blend_bwd_bucket_kernel(BlendArgs<float> a) {
+  constexpr int kBwdWaves = bwd_waves<kRules3D>();
+  // (the lanes' coefficient table after the wavefront's staged splats)
+  __shared__ Staged<float> s_sp[kBwdWaves][kBucket + kCoefSlots];
+  __shared__ uint32_t s_id[kBwdWaves][kBucket];
+  // an elongated splat's three per-lane conic sums, parked over the float32 reduction
+  __shared__ float s_c[kBwdWaves][3 * kWave];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  float* s_cw = s_c[wave];
+  uint32_t evals = 0, atomics = 0;
+  if constexpr (kList == 1) {
+    // one wavefront per list entry; wavefronts past the list's length leave at once. (One
+    // wavefront per workgroup: workgroup b runs on XCD b % 8, and the k-th workgroup of an XCD
+    // takes entry (k / kXcdRun * 8 + b % 8) * kXcdRun + k % kXcdRun, so that runs of kXcdRun
+    // consecutive entries -- a tile's buckets, which read the same pixels -- share an L2.)
+    int64_t i = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave;
+    if constexpr (kBwdWaves == 1) {
+      const int64_t k = blockIdx.x / 8;
+      i = (k / kXcdRun * 8 + blockIdx.x % 8) * kXcdRun + k % kXcdRun;
+    }
+    if (i < static_cast<int64_t>(a.bucket_list[0]))
+      bwd_bucket_3d<kCount, kAbs>(a, a.bucket_list[kListHeader + i], s_sp[wave], s_id[wave], s_cw, evals,
+                                     atomics);
+  } else if constexpr (kList == 2) {
+    // a bounded grid strides over the list (for bucket tables far longer than the list)
+    const int64_t cnt = a.bucket_list[0];
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kBwdWaves;
+    // the wavefront's index made scalar: the loop state and the LDS slots' addresses then live in
+    // scalar registers (64 VGPRs and 105 SGPRs, 7 wavefronts per SIMD by the SGPRs, against 77
+    // VGPRs and 6)
+    const int wave_s = __builtin_amdgcn_readfirstlane(wave);
+    float* s_cws = s_c[wave_s];
+    if constexpr (kBwdWaves == 1) {
+      // logical entries L = blockIdx.x + t * gridDim.x (gridDim.x a multiple of 8 kXcdRun) taken
+      // through the list walk's XCD runs (a bijection on every aligned group of 8 kXcdRun), so
+      // that a tile's consecutive buckets share an L2 here too
+      const int64_t cnt_r = (cnt + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
+      for (int64_t L = blockIdx.x; L < cnt_r; L += stride) {
+        const int64_t k = L / 8;
+        const int64_t i = (k / kXcdRun * 8 + L % 8) * kXcdRun + k % kXcdRun;
+        if (i < cnt)
+          bwd_bucket_3d<kCount, kAbs>(a, a.bucket_list[kListHeader + i], s_sp[wave_s], s_id[wave_s],
+                                         s_cws, evals, atomics);
+      }
+    } else {
+      for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave_s; i < cnt; i += stride)
+        bwd_bucket_3d<kCount, kAbs>(a, a.bucket_list[kListHeader + i], s_sp[wave_s], s_id[wave_s],
+                                       s_cws, evals, atomics);
+    }
+  } else {
+    int64_t b = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave;
+    if constexpr (kBwdWaves == 1) {  // the table walk takes the same XCD runs as the list walk
+      const int64_t k = blockIdx.x / 8;
+      b = (k / kXcdRun * 8 + blockIdx.x % 8) * kXcdRun + k % kXcdRun;
+    }
+    if (b < a.n_buckets && !(a.n_buckets_dev && b >= static_cast<int64_t>(*a.n_buckets_dev)))
+      bwd_bucket_3d<kCount, kAbs>(a, b, s_sp[wave], s_id[wave], s_cw, evals, atomics);
+  }
+  if constexpr (kCount) {
+    if (lane == 0 && atomics) atomicAdd(a.counters, static_cast<unsigned long long>(atomics));
+    count_add(a.counters + 2, evals);
+  }
+}
+
+// A staged splat of the 2D rule sets with the coefficient pairs of its final gradients: the owner
+// lanes' gradients are -(c0 u0 + c1 u1) of wave_reduce_cols's totals, pair i in co[2 i], co[2 i + 1].
+template <typename S>
+struct alignas(16) Staged2D {
+  S mx, my, s0, s1, s2, o, cr, cg, cb;
+  S cut;     // alpha < 1/255 wherever the exponent is not above this
+  S co[16];  // pairs of lanes 0, 1 (mean), 8, 9, 17 (shape), 16 (opacity), red or green, blue
+};
+
+template <int R, typename S>
+__device__ __forceinline__ Staged2D<S> stage2d(const Staged<S>& r, S cut) {
+  Staged2D<S> s;
+  s.mx = r.mx; s.my = r.my; s.s0 = r.s0; s.s1 = r.s1; s.s2 = r.s2; s.o = r.o;
+  s.cr = r.cr; s.cg = r.cg; s.cb = r.cb;
+  s.cut = cut;
+  S* c = s.co;
+  if constexpr (R == kRulesPhase0) {
+    // power = -(a^2 + b^2) / 2, a = l0 dx + l1 dy, b = l2 dy, d = pixel - mean: with Q = L L^T the mean's
+    // gradient is Q (sum h dx, sum h dy), that of l0 -(l0 sum h dx^2 + l1 sum h dx dy), of l1
+    // -(l0 sum h dx dy + l1 sum h dy^2) (its second part is added apart: another group's total), of
+    // l2 -l2 sum h dy^2; the opacity logit's dL/do o (1 - o) = (1 - o) sum h
+    const S A = r.s0 * r.s0, B = r.s0 * r.s1, C = r.s1 * r.s1 + r.s2 * r.s2;
+    c[0] = -A; c[1] = -B; c[2] = -B; c[3] = -C;
+    c[4] = r.s0; c[5] = r.s1;
+    c[6] = S(0); c[7] = r.s0;
+    c[8] = -(S(1) - r.o); c[9] = S(0);
+    c[10] = S(0); c[11] = r.s2;
+  } else {
+    // power = -1/2 (A dx^2 + 2 B dx dy + C dy^2), d = mean - pixel; dL/do = (sum h) / o, since
+    // h = alpha dL/dalpha and alpha = o G wherever it is not clamped (there h is 0)
+    c[0] = r.s0; c[1] = r.s1; c[2] = r.s1; c[3] = r.s2;
+    c[4] = S(0.5); c[5] = S(0);
+    c[6] = S(0); c[7] = S(1);
+    c[8] = S(-1) / r.o; c[9] = S(0);
+    c[10] = S(0); c[11] = S(0.5);
+  }
+  c[12] = S(-1); c[13] = S(0); c[14] = S(0); c[15] = S(-1);
+  return s;
+}
+
+// a / b rounded as the division instruction sequence rounds it for b in [0.01, 1] (one Newton step
+// on the reciprocal, one correction of the quotient; no scaling needed there): 6 instructions.
+__device__ __forceinline__ float div_unit(float a, float b) {
+  float r = __builtin_amdgcn_rcpf(b);
+  r = fmaf(fmaf(-b, r, 1.0f), r, r);
+  const float q = a * r;
+  return fmaf(fmaf(-b, q, a), r, q);
+}
+__device__ __forceinline__ double div_unit(double a, double b) { return a / b; }
+
+// One bucket b of the 2D rule sets, by one wavefront. As the 3D step (strips of 4 rows that the
+// splat's ellipse misses are skipped by a scalar bit, column terms once per splat, dy-only sums per
+// pixel, wave_reduce_cols) with the rule sets' own arithmetic, so that T replays the forward's bits;
+// a row whose lanes' exponents are all at or below the splat's cut skips the exponential.
+// VALU bound. Against a loop that evaluated every row of every entry and reduced twelve sums per
+// splat with wave_reduce12: toy2d 1024^2, 200k splats 192 -> 104 us; phase0 1080p, 50k splats
+// 247 -> 140 us without the counts, 572 -> 146 + 6.5 us with them.
+// kCount: the bucket's reduced steps and its splat-pixel evaluations (a pixel evaluates every list
+// entry up to its stop) are added, as integers, to slots 9 and 10 of its first splat's gradient
+// record, which fold_counts_kernel sums and clears: one counter that every wavefront adds to costs
+// more than the whole backward (about 10 ns an atomic on one address).
+template <int R, typename S, bool kCount>
+__device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, Staged2D<S>* s_sp, uint32_t* s_id) {
+  using Ru = Rule<R, S>;
+  const int lane = threadIdx.x & 63;
+  const uint32_t tile = a.bucket_to_tile[b];
+  const int bstart = static_cast<int>(b - a.bucket_offsets[tile]) * kBucket;
+  const int tmax = a.tile_max ? static_cast<int>(a.tile_max[tile]) : INT_MAX;
+  if (bstart >= tmax) return;
+  const uint32_t r0 = a.ranges[static_cast<int64_t>(tile) * a.range_stride];
+  const uint32_t r1 = a.ranges[static_cast<int64_t>(tile) * a.range_stride + 1];
+  const int bsize = min(kBucket, min(static_cast<int>(r1 - r0), tmax) - bstart);
+  if (bsize <= 0) return;
+  const int tx = static_cast<int>(tile) % a.tiles_x, ty = static_cast<int>(tile) / a.tiles_x;
+
+  uint32_t mk_lane = 0;  // the strip mask of this lane's staged splat
+  if (lane < bsize) {
+    const uint32_t g = a.point_list[r0 + bstart + lane];
+    const Staged<S> r = Ru::stage(a.rec + static_cast<int64_t>(g) * kRecFloats);
+    const float thr = alpha_reach(r.o);
+    s_sp[lane] = stage2d<R, S>(r, static_cast<S>(-thr));
+    mk_lane = strip_mask_2d<R, S>(r, thr, tx * kTile, ty * kTile);
+    s_id[lane] = g;
+  }
+
+  // per-pixel state: pixel p = 64 r + lane, row 4 r + lane / 16, column lane % 16
+  const int64_t HW = static_cast<int64_t>(a.H) * a.W;
+  const int px = tx * kTile + (lane & 15);
+  const S pxf = static_cast<S>(px) + Ru::pix_off();
+  S T[kPixPerLane], rho[kPixPerLane], Gr[kPixPerLane], Gg[kPixPerLane], Gb[kPixPerLane];
+  S pyf[kPixPerLane];
+  int lim[kPixPerLane];
+#pragma unroll
+  for (int r = 0; r < kPixPerLane; ++r) {
+    const int py = ty * kTile + kStripRows * r + (lane >> 4);
+    pyf[r] = static_cast<S>(py) + Ru::pix_off();
+    T[r] = S(0);
+    rho[r] = S(0);
+    Gr[r] = Gg[r] = Gb[r] = S(0);
+    lim[r] = 0;
+    if (px < a.W && py < a.H) {
+      const int64_t pix = static_cast<int64_t>(py) * a.W + px;
+      // phase0 without a limit table: every inside pixel replays the bucket and stops by the
+      // T < 1e-4 rule (phase0/csrc/macrotile/splat2d_bwd_splat.cu:69)
+      const int used = a.n_contrib ? a.n_contrib[pix] - bstart : kBucket;
+      if (used > 0) {
+        lim[r] = min(used, bsize);
         S img0, img1, img2;
         if constexpr (Ru::kInterleaved) {
           Gr[r] = a.grad_image[3 * pix];
@@ -855,311 +1343,176 @@ __device__ __forceinline__ void bwd_bucket(const BlendArgs<S>& a, int64_t b, Sta
         }
         // rho = G . (image - C): the colour still to come (background included)
         rho[r] = Gr[r] * (img0 - c0) + Gg[r] * (img1 - c1) + Gb[r] * (img2 - c2);
-        // alpha = 1 - T_final output: its gradient enters like a background term
-        if constexpr (R == kRules3D) {
-          if (a.grad_alpha) rho[r] -= a.grad_alpha[pix] * a.final_T[pix];
-        }
+        if constexpr (!Ru::kStopBefore)
+          if (T[r] < Ru::t_stop()) lim[r] = 0;  // stopped before this bucket
       }
     }
   }
-  if constexpr (R == kRules3D && !kAbs) {
-    // the coefficient pair of each lane's gradient, g = -(c0 u0 + c1 u1) of the reduction's totals
-    // (u0, u1); lanes 0 and 1 read theirs, the splat's (A, B) and (B, C), from the staged splat,
-    // lane l >= 2 reads (t[l], t[l + 1]) of this table (consecutive words: no bank conflicts): the
-    // owners' pairs are lane 8 (1/2, 0), 9 (0, 1), 16 (-1, 0), 17 (0, 1/2), 32 (-1, 0), 33 (0, -1),
-    // 49 (0, -1), all others (0, 0)
-    float* kt = reinterpret_cast<float*>(s_sp + kBucket);
-    kt[lane] = lane == 8 || lane == 18 ? 0.5f
-               : lane == 10            ? 1.0f
-               : (lane == 16 || lane == 32 || lane == 34 || lane == 50) ? -1.0f
-                                                                       : 0.0f;
-    if (lane == 0) kt[kWave] = 0.0f;
+  int lim_row[kPixPerLane], jmax = 0;
+  uint64_t plane[kPixPerLane];  // the strip bits as scalar bit planes (bit j: splat j)
+#pragma unroll
+  for (int r = 0; r < kPixPerLane; ++r) {
+    lim_row[r] = __builtin_amdgcn_readfirstlane(wave_max(lim[r]));
+    jmax = max(jmax, lim_row[r]);
+    plane[r] = __ballot(((mk_lane >> r) & 1u) ? 1 : 0);
   }
-  // (scalar: the splat loop is uniform over the wavefront)
-  const int jmax = __builtin_amdgcn_readfirstlane(min(bsize, wave_max(lim_max)));
   wave_sync();
 
-  // value index k owned by this lane after wave_reduce12 (lo = 0 or 1 within the 8-lane group)
-  const int grp = lane >> 3, lo = lane & 7;
-  const int kidx = 6 * (grp >> 2) + 3 * ((grp >> 1) & 1) + 2 * (grp & 1) + lo;
-  const bool owner = lo < 2 && (2 * (grp & 1) + lo) < 3 && kidx < NV;
-  if constexpr (R == kRules3D) {
-    // The lane's 4 pixels share a column: the column terms of the power and of the mean
-    // gradient are computed once per splat, and per pixel only dy-dependent sums are kept;
-    // the dx factors are applied in the reduction, once per column. Pixel r of every
-    // lane lies in strip r, so the strip test and the wavefront's largest limit of row r are
-    // scalar; inside, the pixel body has no branches: a lane past its limit or below the
-    // alpha threshold blends alpha = 0, which leaves its T, rho and every sum unchanged.
-    // dL/dopacity = sum G dL/dalpha = (sum alpha dL/dalpha) / o: the sum h is reduced instead.
-    int lim_row[kPixPerLane];
-#pragma unroll
-    for (int r = 0; r < kPixPerLane; ++r) lim_row[r] = __builtin_amdgcn_readfirstlane(wave_max(lim[r]));
-    // the staged splats' strip bits and elongation bit as scalar bit planes (bit j: splat j), so
-    // the per-splat tests below are scalar bit tests with no LDS read
-    uint64_t plane[kPixPerLane + 1];
-#pragma unroll
-    for (int r = 0; r < kPixPerLane; ++r) plane[r] = __ballot(((mk_lane >> r) & 1u) ? 1 : 0);
-    plane[kPixPerLane] = __ballot((mk_lane & kElongBit) ? 1 : 0);
-    // With |dL/dmean2d| (kAbs) the 12 sums are reduced by wave_reduce12 and the final gradient of
-    // the lane's value index k is c0 u0 + c1 u1 + c u (u = its own total): k 0, 1 (mean2d):
-    // -(A u0 + B u1), -(B u0 + C u1); k 2, 4: -u/2; k 3: -u; k 5 (opacity): u; colour and
-    // |dL/dmean2d|: u. Without, wave_reduce_cols leaves two totals (u0, u1) in each 8-lane group
-    // and the gradient of a lane is -(c0 u0 + c1 u1): lanes 0 and 1 the mean2d values from
-    // (sum h dx, sum h dy), with (c0, c1) = (A, B) and (B, C) read from the staged splat; lanes 8
-    // and 9 the conic A and B (-u0/2, -u1), lanes 16 and 17 the opacity (u0) and the conic C
-    // (-u1/2), lanes 32, 33 and 49 the colour, their pairs read from a table of constants.
-    // The opacity column holds sum h = sum alpha dL/dalpha = opacity dL/dopacity: the preprocess
-    // backward divides by the opacity once per Gaussian (in float64) instead of every
-    // bucket-splat step here. The lane-constant parts are chosen here.
-    const bool k0 = kidx == 0, k1 = kidx == 1;  // (kAbs) the lanes of the two mean2d values
-    int kslot;  // the grad2d column of the lane's gradient (-1: none)
-    float kc = 0.0f;
-    if constexpr (kAbs) {
-      kslot = owner ? kidx : -1;
-      kc = (kslot == 2 || kslot == 4) ? -0.5f : kslot == 3 ? -1.0f : kslot >= 5 ? 1.0f : 0.0f;
-    } else {
-      kslot = lane == 0    ? 0
-              : lane == 1  ? 1
-              : lane == 8  ? 2
-              : lane == 9  ? 3
-              : lane == 16 ? 5
-              : lane == 17 ? 4
-              : lane == 32 ? 6
-              : lane == 33 ? 7
-              : lane == 49 ? 8
-                           : -1;
-    }
-    // (without kAbs) the float index of the lane's coefficient pair in s_sp, j * m01 + cidx:
-    // lanes 0 and 1 in staged splat j, the others in the table after the staged splats
-    constexpr int kStagedFloats = static_cast<int>(sizeof(Staged<S>) / sizeof(S));
-    const int m01 = lane < 2 ? kStagedFloats : 0;
-    const int cidx = lane < 2 ? static_cast<int>(offsetof(Staged<S>, n0) / sizeof(S)) + lane
-                              : kBucket * kStagedFloats + lane;
-    const bool row0 = lane < 16;
-    const bool live_owner = kslot >= 0;
-    const bool conic_owner = kslot >= 2 && kslot <= 4;
-    const int64_t kofs = kslot;
-    for (int j = 0; j < jmax; ++j) {
-      const Staged<S> sp = s_sp[j];
-      const typename Ru::Col cl = Ru::col(sp, pxf);
-      const float n0dx = sp.n0 * cl.dx, n1dx = sp.n1 * cl.dx;
-      // zeros the compiler cannot see through: each sum then lives in one register from its
-      // zero to its last update, instead of being re-zeroed on every path that skips a pixel
-      float sh, shy, shyy, cr, cg, cb;
-      opaque_zero2(sh, shy);
-      opaque_zero2(shyy, cr);
-      opaque_zero2(cg, cb);
-      float ab0 = 0.0f, ab1 = 0.0f;
-      if constexpr (kAbs) {
-        ab0 = opaque_zero();
-        ab1 = opaque_zero();
-      }
-      uint64_t used = 0;  // the lanes that blended the splat (a lane mask: scalar)
-#pragma unroll
-      for (int r = 0; r < kPixPerLane; ++r) {
-        if (((plane[r] >> j) & 1u) == 0u || j >= lim_row[r]) continue;  // wave-uniform
-        const bool live = j < lim[r];
-        if constexpr (kCount) evals += live ? 1u : 0u;
-        const float dy = sp.my - pyf[r];
-        const float G = Ru::falloff(Ru::power(sp, cl, dy));
-        const float a_raw = sp.o * G;
-        const bool above = a_raw >= kAlphaMin;
-        const bool take = live && above;
-        // (the masks of the two compares themselves: a ballot of their conjunction would first
-        // turn it into a per-lane value)
-        used |= __builtin_amdgcn_ballot_w64(live) & __builtin_amdgcn_ballot_w64(above);
-        const float alpha = take ? a_raw : 0.0f;
-        const float w = T[r] * alpha;
-        const float dot = fmaf(Gb[r], sp.cb, fmaf(Gg[r], sp.cg, Gr[r] * sp.cr));
-        cr = fmaf(w, Gr[r], cr);
-        cg = fmaf(w, Gg[r], cg);
-        cb = fmaf(w, Gb[r], cb);
-        rho[r] = fmaf(-w, dot, rho[r]);
-        const float oma = 1.0f - alpha;
-        const float dLda = fmaf(T[r], dot, -(rho[r] * __builtin_amdgcn_rcpf(fmaxf(oma, kOneMinusAlphaEps))));
-        const float h = alpha * dLda;  // dL/dpower
-        const float hy = h * dy;
-        sh += h;
-        shy += hy;
-        shyy = fmaf(hy, dy, shyy);
-        if constexpr (kAbs) {
-          ab0 = fmaf(fabsf(h), fabsf(fmaf(sp.n1, dy, n0dx)), ab0);
-          ab1 = fmaf(fabsf(h), fabsf(fmaf(sp.nat2, dy, n1dx)), ab1);
-        }
-        T[r] = T[r] * oma;
-      }
-      if (used == 0) continue;
-      const bool wide = ((plane[kPixPerLane] >> j) & 1u) != 0u;  // wave-uniform
-      if (wide) {
-        // each lane parks the conic sums of its pixels, read back after the float32 reduction
-        const float dxsh = cl.dx * sh;
-        s_c[lane] = cl.dx * dxsh;
-        s_c[kWave + lane] = cl.dx * shy;
-        s_c[2 * kWave + lane] = shyy;
-      }
-      float g;
-      if constexpr (kAbs) {
-        const float dxsh = cl.dx * sh;
-        const float cxx = cl.dx * dxsh, cxy = cl.dx * shy;  // the conic sums of the lane's column
-        const float c0 = k0 ? -sp.n0 : k1 ? -sp.n1 : 0.0f;
-        const float c1 = k0 ? -sp.n1 : k1 ? -sp.nat2 : 0.0f;
-        S acc[12] = {dxsh, shy, cxx, cxy, shyy, sh, cr, cg, cb, ab0, ab1, 0.0f};
-        S u0, u1;
-        wave_reduce12(acc, u0, u1);
-        g = fmaf(c0, u0, fmaf(c1, u1, kc * (lo == 0 ? u0 : u1)));
-      } else {
-        float u0, u1;
-        wave_reduce_cols(sh, shy, shyy, cr, cg, cb, cl.dx, row0, u0, u1);
-        const S* cp = reinterpret_cast<const S*>(s_sp) + (j * m01 + cidx);
-        g = fmaf(-cp[0], u0, -(cp[1] * u1));
-      }
-      // (an elongated splat's conic sums go to the float64 buffer below instead)
-      if (live_owner && !(wide && conic_owner))
-        atomic_add_grad(a.grad_rec + static_cast<int64_t>(s_id[j]) * kGrad2D + kofs, g);
-      if (wide) {  // the conic sums in float64
-        const uint32_t id = __builtin_amdgcn_readfirstlane(s_id[j]);  // wave-uniform
-        wave_sync();  // every lane's parked values
-        // row k of 16 lanes (k < 3) sums value k of the 64 lanes: 4 values per lane in float64
-        // (exactly), then the row's 16 partial sums; A, B, C = -1/2, -1, -1/2 times the sums of
-        // dx^2 h, dx dy h, dy^2 h
-        int ln = lane;
-        asm volatile("" : "+v"(ln));  // formed here, not kept in registers over the whole loop
-        const int k = ln >> 4, r16 = ln & 15;
-        double t = 0.0;
-        if (k < 3) {
-          const float* v = s_c + k * kWave + r16;
-          t = (static_cast<double>(v[0]) + static_cast<double>(v[16])) +
-              (static_cast<double>(v[32]) + static_cast<double>(v[48]));
-        }
-        t += dpp64<0x128>(t);  // row_ror:8
-        t += dpp64<0x141>(t);  // row_half_mirror
-        t += dpp64<0xB1>(t);   // quad_perm [1,0,3,2]
-        t += dpp64<0x4E>(t);   // quad_perm [2,3,0,1]
-        if (r16 == 0 && k < 3) atomic_add_grad(a.conic64 + 4 * static_cast<uint64_t>(id) + k, (k == 1 ? -1.0 : -0.5) * t);
-        // marks the splat's row for the preprocess backward, which then adds the float64 sums
-        if (lane == 48) a.grad_rec[static_cast<uint64_t>(id) * kGrad2D + 11] = 1.0f;
-        wave_sync();  // the parked values are read before the next splat parks its own
-      }
-      if constexpr (kCount) atomics += kAbs ? NV : 9;
-    }
-  } else
+  const int slot = lane == 0    ? 0
+                   : lane == 1  ? 1
+                   : lane == 8  ? 2
+                   : lane == 9  ? 3
+                   : lane == 16 ? 5
+                   : lane == 17 ? 4
+                   : lane == 32 ? 6
+                   : lane == 33 ? 7
+                   : lane == 49 ? 8
+                                : -1;
+  const bool owner = slot >= 0;
+  // the lane's coefficient pair within a staged splat
+  const int pair = lane == 0    ? 0
+                   : lane == 1  ? 1
+                   : lane == 8  ? 2
+                   : lane == 9  ? 3
+                   : lane == 16 ? 4
+                   : lane == 17 ? 5
+                   : lane == 32 ? 6
+                                : 7;
+  const bool row0 = lane < 16;
+  uint32_t steps = 0;  // reduced splats (scalar)
   for (int j = 0; j < jmax; ++j) {
-    const Staged<S> sp = s_sp[j];
-    uint32_t m = 0xfu;
-    if constexpr (Ru::kStrips) m = s_m[j];
-    S acc[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) acc[k] = S(0);
-    bool used = false;
+    const Staged2D<S>& sp = s_sp[j];
+    const S mx = sp.mx, my = sp.my, s0 = sp.s0, s1 = sp.s1, s2 = sp.s2, o = sp.o, cut = sp.cut;
+    const S fr = sp.cr, fg = sp.cg, fb = sp.cb;
+    // the column's part of the exponent (the products exactly as Rule::exponent forms them)
+    S dx, k0, k1;
+    if constexpr (R == kRulesPhase0) {
+      dx = pxf - mx;
+      k0 = s0 * dx;
+      k1 = S(0);
+    } else {
+      dx = mx - pxf;
+      k0 = (s0 * dx) * dx;
+      k1 = s1 * dx;
+    }
+    S sh = S(0), shy = S(0), shyy = S(0), cr = S(0), cg = S(0), cb = S(0);
+    uint64_t used = 0;
 #pragma unroll
     for (int r = 0; r < kPixPerLane; ++r) {
-      if (((m >> r) & 1u) == 0u) continue;  // wave-uniform
-      if (j >= lim[r]) continue;
+      if (((plane[r] >> j) & 1u) == 0u || j >= lim_row[r]) continue;  // wave-uniform
+      S dy, power;
       if constexpr (R == kRulesPhase0) {
-        if (T[r] < Ru::t_stop()) continue;
-      }
-      Eval<S> e;
-      if constexpr (kCount) ++evals;
-      if (!Ru::eval(sp, pxf, pyf[r], e)) continue;
-      used = true;
-      const S w = T[r] * e.alpha;
-      const S dot = fma(Gb[r], sp.cb, fma(Gg[r], sp.cg, Gr[r] * sp.cr));
-      acc[6] = fma(w, Gr[r], acc[6]);
-      acc[7] = fma(w, Gg[r], acc[7]);
-      acc[8] = fma(w, Gb[r], acc[8]);
-      rho[r] = fma(-w, dot, rho[r]);
-      const S oma = S(1) - e.alpha;
-      S dLda;
-      if constexpr (R == kRules3D) {
-        dLda = fma(T[r], dot, -(rho[r] * __builtin_amdgcn_rcpf(fmaxf(oma, kOneMinusAlphaEps))));
+        dy = pyf[r] - my;
+        const S pa = k0 + s1 * dy, pb = s2 * dy;
+        power = S(-0.5) * (pa * pa + pb * pb);
       } else {
-        dLda = T[r] * dot - rho[r] / oma;
+        dy = my - pyf[r];
+        const S t2 = (s2 * dy) * dy;
+        power = S(-0.5) * (k0 + t2) - k1 * dy;
       }
-      pair_sums<R, S>(sp, e, dLda, acc);
-      T[r] = T[r] * oma;
+      const bool reach = j < lim[r] && Ru::in_domain(power) && power > cut;
+      if (__ballot(reach ? 1 : 0) == 0ull) continue;  // wave-uniform
+      const S raw = o * exp_t(power);
+      const bool clamped = raw > S(0.99);
+      const S alpha = clamped ? S(0.99) : raw;
+      const bool take = reach && alpha >= Ru::alpha_min();
+      used |= __ballot(take ? 1 : 0);
+      if (take) {
+        const S w = T[r] * alpha;
+        const S dot = fma(Gb[r], fb, fma(Gg[r], fg, Gr[r] * fr));
+        cr = fma(w, Gr[r], cr);
+        cg = fma(w, Gg[r], cg);
+        cb = fma(w, Gb[r], cb);
+        rho[r] = fma(-w, dot, rho[r]);
+        const S oma = S(1) - alpha;
+        const S dLda = T[r] * dot - div_unit(rho[r], oma);
+        const S h = clamped ? S(0) : alpha * dLda;  // dL/dpower
+        const S hy = h * dy;
+        sh += h;
+        shy += hy;
+        shyy = fma(hy, dy, shyy);
+        T[r] = T[r] * oma;
+        if constexpr (!Ru::kStopBefore)
+          if (T[r] < Ru::t_stop()) lim[r] = j + 1;  // the pixel stops after this splat
+      }
     }
-    if (__ballot(used ? 1 : 0) == 0) continue;  // wave-uniform
+    if (used == 0) continue;  // wave-uniform
+    ++steps;
     S u0, u1;
-    wave_reduce12(acc, u0, u1);
-    if (owner) {
-      const S u = lo == 0 ? u0 : u1;
-      atomic_add_grad(a.grad_rec + static_cast<int64_t>(s_id[j]) * kGrad2D + kidx,
-                      finish_grad<R, S>(sp, kidx, u, u0, u1));
+    wave_reduce_cols(sh, shy, shyy, cr, cg, cb, dx, row0, u0, u1);
+    S g = fma(-sp.co[2 * pair], u0, -(sp.co[2 * pair + 1] * u1));
+    if constexpr (R == kRulesPhase0) {
+      const S uyy = read_lane16(u1);  // sum h dy^2
+      if (lane == 9) g = fma(-s1, uyy, g);
     }
-    if constexpr (kCount) atomics += NV;
+    if (owner) atomic_add_grad(a.grad_rec + static_cast<int64_t>(s_id[j]) * kGrad2D + slot, g);
+  }
+  if constexpr (kCount) {
+    int ev = 0;
+#pragma unroll
+    for (int r = 0; r < kPixPerLane; ++r) ev += lim[r];
+    const uint32_t evals = static_cast<uint32_t>(wave_sum(static_cast<float>(ev)));  // exact: at most 8192
+    uint32_t* row = reinterpret_cast<uint32_t*>(a.grad_rec + static_cast<int64_t>(s_id[0]) * kGrad2D);
+    constexpr int kW = sizeof(S) / 4;
+    if (lane == 0 && steps) atomicAdd(row + 9 * kW, steps);
+    if (lane == 1 && evals) atomicAdd(row + 10 * kW, evals);
   }
 }
 
-// kList 0: wavefront i takes bucket i of the table. With a.bucket_list (3D), the forward's list
-// of the buckets with blended entries: kList 1, wavefront i takes entry i (a wavefront past the
-// list's length only reads that length); kList 2, a bounded grid strides over the list (the
-// loop keeps more registers live, so it is used only when the table is much longer).
-template <int R, typename S, bool kCount, bool kAbs = true, int kList = 0>
-__global__ __launch_bounds__(bwd_waves<R>() * kWave) void blend_bwd_bucket_kernel(
-    BlendArgs<S> a) {
+// 2D rule sets: a wavefront per bucket of the table. kWaves wavefronts to a workgroup; with one,
+// the workgroups take the table in the list walk's XCD runs.
+template <int R, typename S, bool kCount>
+__global__ __launch_bounds__(bwd_waves<R>() * kWave) void blend_bwd_bucket2d_kernel(BlendArgs<S> a) {
   constexpr int kBwdWaves = bwd_waves<R>();
-  // (3D: the lanes' coefficient table after the wavefront's staged splats)
-  __shared__ Staged<S> s_sp[kBwdWaves][kBucket + (R == kRules3D ? kCoefSlots : 0)];
-  __shared__ uint32_t s_m[kBwdWaves][kBucket];
+  __shared__ Staged2D<S> s_sp[kBwdWaves][kBucket];
   __shared__ uint32_t s_id[kBwdWaves][kBucket];
-  // 3D: an elongated splat's three per-lane conic sums, parked over the float32 reduction
-  __shared__ float s_c[R == kRules3D ? kBwdWaves : 1][3 * kWave];
-  const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  float* s_cw = s_c[R == kRules3D ? wave : 0];
-  uint32_t evals = 0, atomics = 0;
-  if constexpr (kList == 1) {
-    // one wavefront per list entry; wavefronts past the list's length leave at once. (One
-    // wavefront per workgroup: workgroup b runs on XCD b % 8, and the k-th workgroup of an XCD
-    // takes entry (k / kXcdRun * 8 + b % 8) * kXcdRun + k % kXcdRun, so that runs of kXcdRun
-    // consecutive entries -- a tile's buckets, which read the same pixels -- share an L2.)
-    int64_t i = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave;
-    if constexpr (kBwdWaves == 1) {
-      const int64_t k = blockIdx.x / 8;
-      i = (k / kXcdRun * 8 + blockIdx.x % 8) * kXcdRun + k % kXcdRun;
-    }
-    if (i < static_cast<int64_t>(a.bucket_list[0]))
-      bwd_bucket<R, S, kCount, kAbs>(a, a.bucket_list[kListHeader + i], s_sp[wave], s_m[wave], s_id[wave], s_cw, evals,
-                                     atomics);
-  } else if constexpr (kList == 2) {
-    // a bounded grid strides over the list (for bucket tables far longer than the list)
-    const int64_t cnt = a.bucket_list[0];
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kBwdWaves;
-    // the wavefront's index made scalar: the loop state and the LDS slots' addresses then live in
-    // scalar registers (64 VGPRs and 105 SGPRs, 7 wavefronts per SIMD by the SGPRs, against 77
-    // VGPRs and 6)
-    const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-    float* s_cws = s_c[R == kRules3D ? wave_s : 0];
-    if constexpr (kBwdWaves == 1) {
-      // logical entries L = blockIdx.x + t * gridDim.x (gridDim.x a multiple of 8 kXcdRun) taken
-      // through the list walk's XCD runs (a bijection on every aligned group of 8 kXcdRun), so
-      // that a tile's consecutive buckets share an L2 here too
-      const int64_t cnt_r = (cnt + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
-      for (int64_t L = blockIdx.x; L < cnt_r; L += stride) {
-        const int64_t k = L / 8;
-        const int64_t i = (k / kXcdRun * 8 + L % 8) * kXcdRun + k % kXcdRun;
-        if (i < cnt)
-          bwd_bucket<R, S, kCount, kAbs>(a, a.bucket_list[kListHeader + i], s_sp[wave_s], s_m[wave_s], s_id[wave_s],
-                                         s_cws, evals, atomics);
-      }
-    } else {
-      for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave_s; i < cnt; i += stride)
-        bwd_bucket<R, S, kCount, kAbs>(a, a.bucket_list[kListHeader + i], s_sp[wave_s], s_m[wave_s], s_id[wave_s],
-                                       s_cws, evals, atomics);
-    }
-  } else {
-    int64_t b = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave;
-    if constexpr (kBwdWaves == 1) {  // the table walk takes the same XCD runs as the list walk
-      const int64_t k = blockIdx.x / 8;
-      b = (k / kXcdRun * 8 + blockIdx.x % 8) * kXcdRun + k % kXcdRun;
-    }
-    if (b < a.n_buckets && !(a.n_buckets_dev && b >= static_cast<int64_t>(*a.n_buckets_dev)))
-      bwd_bucket<R, S, kCount, kAbs>(a, b, s_sp[wave], s_m[wave], s_id[wave], s_cw, evals, atomics);
+  int64_t b = static_cast<int64_t>(blockIdx.x) * kBwdWaves + wave;
+  if constexpr (kBwdWaves == 1) {
+    const int64_t k = blockIdx.x / 8;
+    b = (k / kXcdRun * 8 + blockIdx.x % 8) * kXcdRun + k % kXcdRun;
   }
-  if constexpr (kCount) {
-    if (lane == 0 && atomics) atomicAdd(a.counters, static_cast<unsigned long long>(atomics));
-    count_add(a.counters + 2, evals);
+  if (b < a.n_buckets) bwd_bucket_2d<R, S, kCount>(a, b, s_sp[wave], s_id[wave]);
+}
+
+// The operation counts that blend_bwd_bucket2d_kernel left in slots 9 and 10 of the gradient
+// records, summed into counters[0] (9 atomic adds per reduced splat) and counters[2], and cleared.
+template <typename S>
+__global__ __launch_bounds__(256) void fold_counts_kernel(S* __restrict__ grad_rec, int64_t n,
+                                                          unsigned long long* __restrict__ counters) {
+  constexpr int kW = sizeof(S) / 4;
+  unsigned long long steps = 0, evals = 0;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n; i += stride) {
+    uint32_t* row = reinterpret_cast<uint32_t*>(grad_rec + i * kGrad2D);
+    const uint32_t c = row[9 * kW], e = row[10 * kW];
+    if (c) row[9 * kW] = 0u;
+    if (e) row[10 * kW] = 0u;
+    steps += c;
+    evals += e;
   }
+  block_count_add(9ull * steps, counters);
+  block_count_add(evals, counters + 2);
+}
+
+// counters[2] += the splat-pixel evaluations of a phase0 forward: a pixel evaluates its tile's list
+// up to the splat after which it stopped (its last, if T ended below 1e-4), else all of it. Four
+// tiles per workgroup at a time: with one, 1080p took 16.5 us of dependent loads.
+constexpr int kCountThreads = 4 * kTilePixels;
+
+template <typename S>
+__global__ __launch_bounds__(kCountThreads) void count_evals_kernel(BlendArgs<S> a) {
+  unsigned long long evals = 0;
+  const int t = threadIdx.x % kTilePixels;
+  for (int tile = 4 * blockIdx.x + static_cast<int>(threadIdx.x) / kTilePixels; tile < a.n_tiles; tile += 4 * gridDim.x) {
+    const int px = tile % a.tiles_x * kTile + (t & 15), py = tile / a.tiles_x * kTile + (t >> 4);
+    if (px >= a.W || py >= a.H) continue;
+    const int64_t pix = static_cast<int64_t>(py) * a.W + px;
+    const uint32_t* rg = a.ranges + static_cast<int64_t>(tile) * a.range_stride;
+    const uint32_t len = rg[1] - rg[0], last = static_cast<uint32_t>(a.last_contrib[pix]);
+    evals += a.final_T[pix] < Rule<kRulesPhase0, S>::t_stop() ? last : len;
+  }
+  block_count_add(evals, a.counters + 2);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1282,21 +1635,21 @@ using namespace gs;
 // ---------------------------------------------------------------------------------------
 namespace {
 
+// The 2D forward. The evaluations of a phase0 forward follow from its outputs (count_evals_kernel);
+// a caller that counts without them, or under the toy2d rules, takes the counting kernel.
+constexpr int kCountBlocks = 512;
+
 template <int R, typename S>
-void launch_fwd(const BlendArgs<S>& a, hipStream_t st) {
-  if constexpr (R == kRules3D && std::is_same<S, float>::value) {
-    // (the 3D forward takes no counters) one pixel per lane, a wavefront per strip, measured
-    // fastest: 114 us at 1M SH3 against 118 with two and 165 with four (a wavefront per tile:
-    // too few wavefronts, and the heaviest tiles run alone), and 120 for the shared-staging
-    // blend_fwd_kernel
-    constexpr int P = 1;
-    constexpr int kTPB = 4 / (kStrips / P);
-    hipLaunchKernelGGL(blend_fwd_strip_kernel<P>, dim3(static_cast<unsigned>((a.n_tiles + kTPB - 1) / kTPB)),
-                       dim3(4 * kWave), 0, st, a);
-  } else if (a.counters) {
+void launch_fwd2d(const BlendArgs<S>& a, hipStream_t st) {
+  if (a.counters && !(R == kRulesPhase0 && a.last_contrib)) {
     hipLaunchKernelGGL((blend_fwd_kernel<R, S, true>), dim3(a.n_tiles), dim3(kTilePixels), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((blend_fwd_kernel<R, S, false>), dim3(a.n_tiles), dim3(kTilePixels), 0, st, a);
+    return;
+  }
+  hipLaunchKernelGGL((blend_fwd_strip2d_kernel<R, S>), dim3(a.n_tiles), dim3(4 * kWave), 0, st, a);
+  if constexpr (R == kRulesPhase0) {
+    if (a.counters)
+      hipLaunchKernelGGL(count_evals_kernel<S>, dim3(static_cast<unsigned>(std::min((a.n_tiles + 3) / 4, kCountBlocks))),
+                         dim3(kCountThreads), 0, st, a);
   }
 }
 
@@ -1305,30 +1658,48 @@ void launch_fwd(const BlendArgs<S>& a, hipStream_t st) {
 constexpr int64_t kBwdListBlocks = 256 * 64;
 constexpr int64_t kBwdStrideFrom = 4 * kBwdListBlocks * 4;
 
-template <int R, typename S, bool kCount, bool kAbs>
-void launch_bwd_bucket_k(const BlendArgs<S>& a, hipStream_t st) {
+template <int R>
+int64_t bwd_blocks(int64_t n_buckets) {
   constexpr int kBwdWaves = bwd_waves<R>();
-  int64_t blocks = (a.n_buckets + kBwdWaves - 1) / kBwdWaves;
+  int64_t blocks = (n_buckets + kBwdWaves - 1) / kBwdWaves;
   // (the walks' XCD runs map workgroups onto entries within whole groups of 8 kXcdRun)
   if (kBwdWaves == 1) blocks = (blocks + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
-  const dim3 block(kBwdWaves * kWave);
-  if (a.bucket_list && blocks > kBwdStrideFrom)
-    hipLaunchKernelGGL((blend_bwd_bucket_kernel<R, S, kCount, kAbs, 2>), dim3(static_cast<unsigned>(kBwdListBlocks)),
-                       block, 0, st, a);
-  else if (a.bucket_list)
-    hipLaunchKernelGGL((blend_bwd_bucket_kernel<R, S, kCount, kAbs, 1>), dim3(static_cast<unsigned>(blocks)), block,
-                       0, st, a);
-  else
-    hipLaunchKernelGGL((blend_bwd_bucket_kernel<R, S, kCount, kAbs, 0>), dim3(static_cast<unsigned>(blocks)), block,
-                       0, st, a);
+  return blocks;
 }
 
-template <int R, typename S, bool kAbs = true>
-void launch_bwd_bucket(const BlendArgs<S>& a, hipStream_t st) {
-  if (a.counters)
-    launch_bwd_bucket_k<R, S, true, kAbs>(a, st);
+template <bool kCount, bool kAbs>
+void launch_bwd_bucket_k(const BlendArgs<float>& a, hipStream_t st) {
+  const int64_t blocks = bwd_blocks<kRules3D>(a.n_buckets);
+  const dim3 block(bwd_waves<kRules3D>() * kWave);
+  if (a.bucket_list && blocks > kBwdStrideFrom)
+    hipLaunchKernelGGL((blend_bwd_bucket_kernel<kCount, kAbs, 2>), dim3(static_cast<unsigned>(kBwdListBlocks)), block,
+                       0, st, a);
+  else if (a.bucket_list)
+    hipLaunchKernelGGL((blend_bwd_bucket_kernel<kCount, kAbs, 1>), dim3(static_cast<unsigned>(blocks)), block, 0, st,
+                       a);
   else
-    launch_bwd_bucket_k<R, S, false, kAbs>(a, st);
+    hipLaunchKernelGGL((blend_bwd_bucket_kernel<kCount, kAbs, 0>), dim3(static_cast<unsigned>(blocks)), block, 0, st,
+                       a);
+}
+
+template <bool kAbs>
+void launch_bwd_bucket(const BlendArgs<float>& a, hipStream_t st) {
+  if (a.counters)
+    launch_bwd_bucket_k<true, kAbs>(a, st);
+  else
+    launch_bwd_bucket_k<false, kAbs>(a, st);
+}
+
+template <int R, typename S>
+void launch_bwd_bucket2d(const BlendArgs<S>& a, int64_t n, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(bwd_blocks<R>(a.n_buckets))), block(bwd_waves<R>() * kWave);
+  if (a.counters) {
+    hipLaunchKernelGGL((blend_bwd_bucket2d_kernel<R, S, true>), grid, block, 0, st, a);
+    hipLaunchKernelGGL(fold_counts_kernel<S>, dim3(static_cast<unsigned>(std::min<int64_t>((n + 255) / 256, kCountBlocks))),
+                       dim3(256), 0, st, a.grad_rec, n, a.counters);
+  } else {
+    hipLaunchKernelGGL((blend_bwd_bucket2d_kernel<R, S, false>), grid, block, 0, st, a);
+  }
 }
 
 template <int R, typename S>
@@ -1411,7 +1782,13 @@ extern "C" int gs_blend_fwd_3d(const float* splat_rec, const uint32_t* ranges,
   a.clear4_n = clear_floats / 4;
   if (bucket_list && !(flags & GS_BLEND_LIST_CLEARED))
     fill_zero_f32(reinterpret_cast<float*>(bucket_list), kListHeader, as_stream(stream));
-  launch_fwd<kRules3D, float>(a, as_stream(stream));
+  // one pixel per lane, a wavefront per strip, measured fastest: 114 us at 1M SH3 against 118 with
+  // two and 165 with four (a wavefront per tile: too few wavefronts, and the heaviest tiles run
+  // alone), and 120 for the shared-staging blend_fwd_kernel
+  constexpr int P = 1;
+  constexpr int kTPB = 4 / (kStrips / P);
+  hipLaunchKernelGGL(blend_fwd_strip_kernel<P>, dim3(static_cast<unsigned>((a.n_tiles + kTPB - 1) / kTPB)),
+                     dim3(4 * kWave), 0, as_stream(stream), a);
   return check_launch("blend_fwd_3d");
 }
 
@@ -1474,9 +1851,9 @@ extern "C" int gs_blend_bwd_3d(const float* splat_rec, const uint32_t* ranges,
   GS_REQUIRE(aligned(bucket_list, 16), GS_ERR_ALIGN, "bucket_list must be 16-byte aligned");
   a.bucket_list = bucket_list;
   if (flags & GS_ABS_GRAD)
-    launch_bwd_bucket<kRules3D, float, true>(a, st);
+    launch_bwd_bucket<true>(a, st);
   else
-    launch_bwd_bucket<kRules3D, float, false>(a, st);
+    launch_bwd_bucket<false>(a, st);
   return check_launch("blend_bwd_3d");
 }
 
@@ -1505,7 +1882,7 @@ extern "C" int gs2d_blend_fwd(int rules, int dtype, const void* rec, const uint3
     a.tile_max = tile_max;
     a.ckpt = static_cast<S*>(ckpt);
     a.counters = counters;
-    launch_fwd<R, S>(a, as_stream(stream));
+    launch_fwd2d<R, S>(a, as_stream(stream));
     rc = check_launch("gs2d_blend_fwd");
   });
   return rc;
@@ -1547,7 +1924,7 @@ extern "C" int gs2d_blend_bwd_bucket(int rules, int dtype, const void* rec, cons
     a.n_buckets = n_buckets;
     a.grad_image = static_cast<const S*>(grad_image);
     a.grad_rec = static_cast<S*>(grad_rec);
-    launch_bwd_bucket<R, S>(a, st);
+    launch_bwd_bucket2d<R, S>(a, n, st);
     rc = check_launch("gs2d_blend_bwd_bucket");
   });
   return rc;

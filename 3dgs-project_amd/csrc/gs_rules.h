@@ -35,7 +35,7 @@ struct alignas(16) Staged {
   S s0, s1, s2;  // 3D forward: conic pre-scaled for exp2; 2D: conic or Cholesky factors
   S o;          // opacity
   S cr, cg, cb;  // colour
-  S n0, n1;     // 3D: natural conic A and B (C is in nat2); 2D: unused
+  S n0, n1;     // 3D: natural conic A and B (C is in nat2); 2D: n0 the exponent's cut, n1 unused
   S nat2;       // 3D: natural conic C
 };
 
@@ -147,17 +147,24 @@ struct Rule<kRulesToy2D, S> {
   }
 
   // power = -0.5 (A dx dx + C dy dy) - B dx dy, skipped if positive; alpha = min(0.99, o G)
-  __device__ static bool eval(const Staged<S>& s, S px, S py, Eval<S>& e) {
+  __device__ static S exponent(const Staged<S>& s, S px, S py, Eval<S>& e) {
     e.dx = s.mx - px;
     e.dy = s.my - py;
     const S t1 = (s.s0 * e.dx) * e.dx;
     const S t2 = (s.s2 * e.dy) * e.dy;
-    const S power = S(-0.5) * (t1 + t2) - (s.s1 * e.dx) * e.dy;
-    if (power > S(0)) return false;
+    return S(-0.5) * (t1 + t2) - (s.s1 * e.dx) * e.dy;
+  }
+  __device__ static bool in_domain(S power) { return !(power > S(0)); }
+  __device__ static void alpha_of(const Staged<S>& s, S power, Eval<S>& e) {
     e.G = exp_t(power);
     const S raw = s.o * e.G;
     e.clamped = raw > S(0.99);
     e.alpha = e.clamped ? S(0.99) : raw;
+  }
+  __device__ static bool eval(const Staged<S>& s, S px, S py, Eval<S>& e) {
+    const S power = exponent(s, px, py, e);
+    if (power > S(0)) return false;
+    alpha_of(s, power, e);
     return e.alpha >= alpha_min();
   }
 };
@@ -179,16 +186,23 @@ struct Rule<kRulesPhase0, S> {
   __device__ static Staged<S> stage(const S* r) { return Rule<kRulesToy2D, S>::stage(r); }
 
   // q = (l0 dx + l1 dy)^2 + (l2 dy)^2, G = exp(-q/2), alpha = min(0.99, o G)
-  __device__ static bool eval(const Staged<S>& s, S px, S py, Eval<S>& e) {
+  __device__ static S exponent(const Staged<S>& s, S px, S py, Eval<S>& e) {
     e.dx = px - s.mx;
     e.dy = py - s.my;
     e.a = s.s0 * e.dx + s.s1 * e.dy;
     e.b = s.s2 * e.dy;
     const S q = e.a * e.a + e.b * e.b;
-    e.G = exp_t(S(-0.5) * q);
+    return S(-0.5) * q;
+  }
+  __device__ static bool in_domain(S) { return true; }
+  __device__ static void alpha_of(const Staged<S>& s, S power, Eval<S>& e) {
+    e.G = exp_t(power);
     const S raw = s.o * e.G;
     e.clamped = raw > S(0.99);
     e.alpha = e.clamped ? S(0.99) : raw;
+  }
+  __device__ static bool eval(const Staged<S>& s, S px, S py, Eval<S>& e) {
+    alpha_of(s, exponent(s, px, py, e), e);
     return e.alpha >= alpha_min();
   }
 };

@@ -472,3 +472,79 @@ def test_fused_activation_matches_the_reference_activation(spread):
         e32 = ((t32 - b).norm() / b.norm()).item()
         bound = 1.5 * e32 + 1e-7 if spread else 1e-5
         assert e < bound, f"grad {name}: {e:.2e} (float32 autograd of activate: {e32:.2e})"
+
+
+def edge_splats(rules, dtype, n=330, W=75, H=53, seed=5):
+    """Splats at the edges of what the blends' strip and exponent tests decide: standard deviations
+    from 0.2 to 200 px with axis ratios to beyond the condition limit of the strip test, means on
+    and outside the image, opacities at, just above and far below 1/255, at 1 and above it (toy2d),
+    and (at the end) non-finite means, shapes and opacities, which no pixel blends."""
+    g = np.random.default_rng(seed)
+    means = np.stack([g.uniform(-0.3 * W, 1.3 * W, n), g.uniform(-0.3 * H, 1.3 * H, n)], 1)
+    s1, s2, th = np.exp(g.uniform(np.log(0.2), np.log(200), n)), np.exp(g.uniform(np.log(0.2), np.log(200), n)), \
+        g.uniform(0, np.pi, n)
+    s1[:8], s2[:8] = 0.4, 180.0  # condition numbers of 2e5
+    o = np.clip(g.uniform(-0.1, 0.6, n), 0.0, 1.0)
+    o[10:20], o[20:30], o[30:34], o[34:40] = 1 / 255, 1.0001 / 255, 1e-30, 1.0
+    c, s = np.cos(th), np.sin(th)
+    ia, ib = 1 / s1 ** 2, 1 / s2 ** 2
+    A, B, C = c * c * ia + s * s * ib, c * s * (ia - ib), s * s * ia + c * c * ib
+    if rules == O2.TOY2D:
+        shape, op = np.stack([A, B, C], 1), o
+        op[40:44] = 1.7
+        shape[44:48, 1] *= 40  # not positive definite: blended where the exponent is not positive
+    else:
+        shape = np.stack([np.sqrt(A), B / np.sqrt(A), np.sqrt(np.maximum(C - B * B / A, 1e-12))], 1)
+        op = np.log(np.maximum(o, 1e-30)) - np.log1p(-np.minimum(o, 1 - 1e-6))
+    means[-6], means[-5, 0], shape[-4], op[-3] = np.nan, np.inf, np.nan, np.nan
+    shape[-2, 2] = np.inf
+    color = g.uniform(0, 1, (n, 3))
+    return [a.astype(dtype) for a in (means, shape, color, op)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rules", [O2.TOY2D, O2.PHASE0])
+def test_blend2d_edge_splats_against_oracle(rules, dtype):
+    """Every splat in every tile's list (330 entries: eleven buckets, the last of 10; two staging
+    rounds of a wavefront's 64 and a remainder), so that the strip and exponent tests decide
+    everything: counts bit-exact, image and gradients at the bars of the other tests."""
+    W, H = 75, 53
+    means, shape, color, op = edge_splats(rules, dtype)
+    n, T = len(means), 5 * 4
+    pl = np.tile(np.arange(n, dtype=np.uint32), T)
+    ranges = np.stack([np.arange(T) * n, (np.arange(T) + 1) * n], 1).astype(np.uint32)
+    nb = (n + 31) // 32
+    boff = (np.arange(T + 1) * nb).astype(np.uint32)
+    ref = O2.forward(rules, means, shape, color, op, pl, ranges, boff, W, H)
+    p = [cuda(a) for a in (means, shape, color, op)]
+    rec = R2.pack(rules, p[0], p[1], p[2], p[3])
+    d_pl, d_rg, d_bo = cuda(pl.astype(np.int32)), cuda(ranges.astype(np.int32)), cuda(boff.astype(np.int32))
+    ctr = torch.zeros(3, dtype=torch.int64, device="cuda")
+    image, fT, nc, last, tmax, ckpt = R2.blend_fwd(rules, rec, d_rg, 2, d_pl, d_bo, nb * T, W, H, counters=ctr)
+    assert np.array_equal(nc.cpu().numpy(), ref["n_contrib"])
+    rlast = ref["last_contrib"] if rules == O2.PHASE0 else ref["n_contrib"]
+    assert np.array_equal(last.cpu().numpy(), rlast)
+    assert rel(image, ref["image"]) < (1e-5 if dtype == np.float32 else 1e-12)
+    assert int(ctr[2]) == ref["evals"]
+    # the uncounted forward is the one most callers take
+    again = R2.blend_fwd(rules, rec, d_rg, 2, d_pl, d_bo, nb * T, W, H)
+    assert torch.equal(again[2], nc) and torch.equal(again[3], last) and torch.equal(again[4], tmax)
+    assert rel(again[0], ref["image"]) < (1e-5 if dtype == np.float32 else 1e-12)
+    gi = np.random.default_rng(1).standard_normal(ref["image"].shape).astype(dtype)
+    g_ref, atomics = O2.backward_bucket(rules, means, shape, color, op, pl, ranges, boff, W, H, ref["image"], gi, rlast,
+                                        ref["ckpt"])
+    b2t = torch.arange(T, device="cuda", dtype=torch.int32).repeat_interleave(nb)
+    ctr.zero_()
+    for counters in (ctr, None):
+        g = R2.blend_bwd_bucket(rules, rec, d_rg, 2, d_pl, d_bo, b2t, nb * T, W, H, image, cuda(gi), last, tmax, ckpt,
+                                counters=counters)
+        for x, y in zip(R2.split_grads(g), (g_ref[:, :2], g_ref[:, 2:5], g_ref[:, 5], g_ref[:, 6:9])):
+            assert rel(x, y) < (1e-4 if dtype == np.float32 else 1e-9)
+        assert not bool((g[:, 9:] != 0).any())
+    assert int(ctr[0]) == atomics and int(ctr[2]) == int(rlast.sum())
+    if rules == O2.PHASE0:  # without the limits each pixel replays up to its stop
+        ctr.zero_()
+        g = R2.blend_bwd_bucket(rules, rec, d_rg, 2, d_pl, d_bo, b2t, nb * T, W, H, image, cuda(gi), None, None, ckpt,
+                                counters=ctr)
+        assert rel(g[:, :9], g_ref[:, :9]) < (1e-4 if dtype == np.float32 else 1e-9)
+        assert int(ctr[0]) == atomics and int(ctr[2]) == ref["evals"]
