@@ -4,8 +4,8 @@
 // The order is that of a stable sort of 64-bit keys (tile << 32 | orderable depth) over
 // instances emitted in Gaussian-index order, obtained in two levels: a stable 32-bit sort of
 // the Gaussians by depth (N keys), emission of the instances in that order, and a stable sort
-// of the instances by tile (M keys, ceil(log2 T) bits). Each sort is LSD radix with 8-bit
-// digits, reduce-then-scan per digit: a histogram kernel, a device-wide exclusive scan of the
+// of the instances by tile (M keys, ceil(log2 T) bits). The first is a bucket sort up to 1M keys
+// (gs_sample_sort.h); otherwise each sort is LSD radix, reduce-then-scan per digit: a histogram kernel, a device-wide exclusive scan of the
 // digit-major histogram table, and a scatter kernel that ranks keys stably inside its
 // workgroup. No kernel waits on another workgroup, so there is no forward-progress
 // requirement.
@@ -569,6 +569,23 @@ static void radix_sort(const K* k, const uint32_t* v, K* k_out, uint32_t* v_out,
   }
 }
 
+// Exclusive prefix sum over the wavefront; `total` receives the sum of all lanes.
+__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_t& total) {
+  uint32_t incl = v;
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t u = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += u;
+  }
+  total = __shfl(incl, kWave - 1, 64);
+  return incl - v;
+}
+
+}  // namespace gs
+
+#include "gs_sample_sort.h"
+
+namespace gs {
+
 // ---------------------------------------------------------------------------------------
 // Two-level binning: (1) stable sort of the Gaussians by depth key (culled ones last);
 // (2) emission of (tile, Gaussian) instances in that order; (3) stable sort by tile.
@@ -641,17 +658,6 @@ struct EmitSetup {
   float mx, my, invA, B, det, tA, vmax, vr;  // 3D band setup (what band_columns reads)
   int4 d;                                 // 3D: pixel bounds; rectangles: clamped tile rectangle
 };
-
-// Exclusive prefix sum over the wavefront; `total` receives the sum of all lanes.
-__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_t& total) {
-  uint32_t incl = v;
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t u = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += u;
-  }
-  total = __shfl(incl, kWave - 1, 64);
-  return incl - v;
-}
 
 // Wavefronts per workgroup of emit_kernel: one. Each takes its own window and shares nothing with
 // the others (1M SH3 key duplication 41.4 -> 40.5 us against four per workgroup).
@@ -1827,7 +1833,7 @@ static PrepLayout prep_layout(int64_t n) {
   L.dsorted = o; o += align_up(n * 4);
   L.khi = o; o += align_up(n * 4);
   L.tmpv = o; o += align_up(n * 4);
-  L.sort = o; o += sort_ws(n);
+  L.sort = o; o += std::max(sort_ws(n), ss_layout(n).end);
   L.scan = o; o += scan_ws(n);
   L.end = o;
   return L;
@@ -1957,9 +1963,15 @@ static void bin_prepare(const SplatRec* rec, const float* depth, const double* d
                          counts, n, dkeys, depth64 ? khi : nullptr);
       keys = dkeys;
     }
-    // the final pass also writes the counts in depth order (into khi, free by then), so the scan
-    // reads them contiguously instead of through the order; the sorted keys themselves are not
-    // needed, so it writes none
+    // Up to kSsMaxKeys 32-bit keys: the bucket sort, which takes the offsets along. Beyond, and for
+    // float64 depths, the radix sort, whose final pass also writes the counts in depth order (into khi, free by then), so the
+    // scan reads them contiguously instead of through the order; the sorted keys themselves are
+    // not needed, so it writes none.
+    if (!depth64 && ss_takes(n)) {
+      sample_sort(keys, counts, n, order, offsets, sort_scratch, st);
+      stage_mark("depth_sort", st);
+      return;
+    }
     uint32_t* sorted_counts = offsets ? khi : nullptr;
     if (depth64) {
       // low key halves first, then stably by the high halves gathered into that order

@@ -606,7 +606,9 @@ __global__ __launch_bounds__(4 * kWave) void blend_fwd_strip_kernel(BlendArgs<fl
 // blend_fwd_kernel. The 2D tile lists hold every tile of a splat's rectangle, so most of a list's
 // entries reach few of a tile's pixels: an entry is skipped for a strip its ellipse misses (a
 // scalar bit), and its exponential is not evaluated where no lane's exponent is above
-// -ln(255 o).
+// -ln(255 o). VALU bound. Against blend_fwd_kernel (256 entries staged by the workgroup, every entry
+// evaluated by every pixel): toy2d 1024^2, 200k splats 132 -> 71 us; phase0 1080p, 50k splats, with
+// the evaluation count 425 -> 102 + 8 us (that kernel adds 32k wavefronts' counts to one address).
 //
 // Checkpoints: with the shared staging a workgroup stopped at the first multiple of 256 entries
 // at which all its pixels had stopped; buckets before that hold the pixels' states, those after

@@ -64,10 +64,41 @@ def test_depth_order_few_key_bits(n, far):
     check_depth_order(n, "culled_mix", 9, near=1.0, far=far)
 
 
-def check_depth_order(n, kind, max_count, near=NEAR, far=FAR):
+# the bucket sort's sizes: one workgroup up to 4096 keys, the larger LDS capacity from 512k on, the
+# radix sort beyond 2^20
+@pytest.mark.parametrize("n", [2048, 2049, 4096, 524_287, 1_048_576, 1_048_577])
+@pytest.mark.parametrize("kind", ["distinct", "culled_mix"])
+def test_depth_order_bucket_sort_sizes(n, kind):
+    check_depth_order(n, kind, 9)
+
+
+@pytest.mark.parametrize("n", [5_000, 70_001, 900_000])
+def test_depth_order_bucket_beyond_lds(n):
+    """Keys chosen against the hashed sample positions: every sampled key lies below all others, so
+    one bucket holds nearly all keys and is sorted through global memory; ties among them."""
+    mean = 1024 if n < 512 << 10 else 2048
+    B = (n + mean - 1) // mean
+    S = 8 * B
+    i = np.arange(S, dtype=np.uint64)
+    step = np.uint64((n << 32) // S)
+    lo, hi = i * step >> np.uint64(32), (i + np.uint64(1)) * step >> np.uint64(32)
+    h = i.astype(np.uint32)
+    h ^= h >> np.uint32(16)
+    h = (h.astype(np.uint64) * np.uint64(0x7feb352d) & np.uint64(0xffffffff)).astype(np.uint32)
+    h ^= h >> np.uint32(15)
+    h = (h.astype(np.uint64) * np.uint64(0x846ca68b) & np.uint64(0xffffffff)).astype(np.uint32)
+    h ^= h >> np.uint32(16)
+    pos = (lo + (h.astype(np.uint64) * (hi - lo) >> np.uint64(32))).astype(np.int64)
+    rng = np.random.default_rng(n)
+    keys = (100_000 + rng.integers(0, max(n // 3, 1), n)).astype(np.uint32)
+    keys[pos] = rng.permutation(S).astype(np.uint32)
+    check_depth_order(n, "beyond_lds", 9, keys=keys)
+
+
+def check_depth_order(n, kind, max_count, near=NEAR, far=FAR, keys=None):
     rng = np.random.default_rng(n + len(kind))
     cull = host_order_key(far) - host_order_key(near)
-    keys = depth_keys(n, kind, rng, cull)
+    keys = depth_keys(n, kind, rng, cull) if keys is None else keys
     counts = rng.integers(0, max_count, n).astype(np.uint32)
     dev = torch.device("cuda")
     kd = torch.from_numpy(keys.view(np.int32)).to(dev)
