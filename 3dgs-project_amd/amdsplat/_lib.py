@@ -41,6 +41,12 @@ GS_CAM_PROPER_ANTIALIASING = 1  # gs_camera.flags bit
 GS_BIN_SPANS, GS_BIN_RADIX = 2, 4  # binning path forced (gs_camera.flags, rect flags)
 BIN_FLAGS = {"auto": 0, "spans": GS_BIN_SPANS, "radix": GS_BIN_RADIX}
 GS_BIN_PATH_RADIX, GS_BIN_PATH_SPANS = 0, 1  # gs_bin_path
+GS_VIEW_BACKWARD, GS_VIEW_KEYS, GS_VIEW_NO_IMAGE = 1, 2, 4  # gs_view_* flags
+# regions of the view arenas (gs_view_plan, gs_view_plan_count)
+(VIEW_REC, VIEW_ORDER, VIEW_OFFSETS, VIEW_RANGES, VIEW_BUCKET_OFFSETS, VIEW_FINAL_T, VIEW_N_CONTRIB,
+ VIEW_TILE_MAX) = range(8)
+VIEW_POINT_LIST, VIEW_BUCKET_TO_TILE, VIEW_BUCKET_LIST, VIEW_CKPT, VIEW_SORTED_KEYS = range(5)
+ViewStateOffsets, ViewListOffsets, ViewSizes = C.c_int64 * 8, C.c_int64 * 5, C.c_int64 * 3
 GS_ADAM_MAX_GROUPS = 8
 
 
@@ -92,6 +98,14 @@ _SIGS = {
     "gs_blend_scores_3d": (_i32, [_vp, _vp, _vp, _i32, _i32, _i64, _vp, _vp]),
     "gs_blend_bwd_3d": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                _vp, _vp, _vp, _i32, _vp, _vp]),
+    "gs_view_plan": (_i32, [_i64, C.POINTER(GsCamera), _i32, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
+    "gs_view_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, C.POINTER(GsCamera), _i32, _vp, _vp, _vp,
+                             _vp]),
+    "gs_view_plan_count": (_i32, [_i64, _i64, C.POINTER(GsCamera), _i32, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
+    "gs_view_finish": (_i32, [_i64, _i64, C.POINTER(GsCamera), _i32, _vp, _vp, _vp, _sz, C.POINTER(C.c_float), _vp, _vp,
+                              _vp, _i64, _vp]),
+    "gs_view_backward": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i64, C.POINTER(GsCamera), _vp, _vp, _vp,
+                                _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gs_preprocess_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, C.POINTER(GsCamera), _vp, _vp,
                                  _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gs_adam_step": (_i32, [C.POINTER(GsAdamGroup), _i32, _i64, _vp, _vp]),
@@ -202,7 +216,7 @@ def make_camera(viewmat, fx: float, fy: float, cx: float, cy: float, width: int,
         flat = [x for row in viewmat for x in row] if viewmat and isinstance(viewmat[0], (list, tuple)) else viewmat
     if len(flat) != 16:
         raise ValueError("viewmat must be 4x4")
-    cam.viewmat[:] = [float(x) for x in flat]
+    cam.viewmat[:] = flat if all(type(x) is float for x in flat) else [float(x) for x in flat]
     cam.fx, cam.fy, cam.cx, cam.cy = float(fx), float(fy), float(cx), float(cy)
     cam.width, cam.height = int(width), int(height)
     cam.near_plane, cam.far_plane = float(near), float(far)

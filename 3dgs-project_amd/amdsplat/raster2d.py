@@ -63,7 +63,7 @@ class RectBins:
 
     point_list: torch.Tensor      # [m]
     ranges: torch.Tensor          # [T, 2] CSR [start, end)
-    tile_offsets: torch.Tensor    # [T + 1]
+    tile_offsets: torch.Tensor | None  # [T + 1] (if asked for)
     bucket_offsets: torch.Tensor  # [T + 1]
     bucket_to_tile: torch.Tensor  # [B]
     order: torch.Tensor | None    # [n] stable argsort of depth (if asked for)
@@ -74,8 +74,17 @@ class RectBins:
 BINNING = "auto"
 
 
+def _host_sum(p: int, n: int, st) -> int:
+    """The sum of n uint32 device values on the host, stored there by its kernel (a wait for that
+    kernel, no copy to enqueue)."""
+    call("gs_count_begin", p, n, 0, st)
+    v = C.c_uint64()
+    call("gs_count_end", C.byref(v))
+    return int(v.value)
+
+
 def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | None, width: int, height: int,
-              want_order: bool = False, binning: str | None = None) -> RectBins:
+              want_order: bool = False, binning: str | None = None, want_tile_offsets: bool = True) -> RectBins:
     """Per-tile lists of the Gaussians whose tile rectangle covers the tile, in stable depth
     order (depth given) or index order. Two host reads: the instance and bucket counts.
     binning: "auto", "spans" or "radix" (default: the module's BINNING); the lists are the same."""
@@ -85,17 +94,10 @@ def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | N
     tx, ty = tiles_of(width, height)
     T = tx * ty
     st = stream(dev)
-    if n > 0:
-        # the instance count, summed on the library's side stream and read without draining st
-        call("gs_count_begin", ptr(counts), n, 0, st)
-        mv = C.c_uint64()
-        call("gs_count_end", C.byref(mv))
-        m = int(mv.value)
-    else:
-        m = 0
+    m = _host_sum(ptr(counts), n, st) if n > 0 else 0
     point_list = torch.empty(m, dtype=torch.int32, device=dev)
     ranges = torch.empty(T, 2, dtype=torch.int32, device=dev)
-    tile_offsets = torch.empty(T + 1, dtype=torch.int32, device=dev)
+    tile_offsets = torch.empty(T + 1, dtype=torch.int32, device=dev) if want_tile_offsets else None
     boff = torch.empty(T + 1, dtype=torch.int32, device=dev)
     order = torch.empty(n, dtype=torch.int32, device=dev) if want_order else None
     d = None
@@ -108,9 +110,11 @@ def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | N
     ws = _u8(_lib.size_call("gs_bin_workspace_size", n, m, tx, ty, flags), dev)
     call("gs_bin_fill_rect", ptr(rects), ptr(d), dcode, ptr(counts), n, tx, ty, m, None, ptr(point_list), ptr(ranges),
          ptr(tile_offsets), ptr(boff), ptr(order), flags, ptr(ws), ws.numel(), st)
-    nb = int(boff[T].item())
-    b2t = torch.empty(max(nb, 1), dtype=torch.int32, device=dev)
-    call("gs_bucket_fill", ptr(boff), T, ptr(b2t), nb, st)
+    # the bucket table is filled to its bound (m + 31 T) / 32 while the host waits for the bucket count
+    bound = (m + (BUCKET - 1) * T) // BUCKET
+    b2t = torch.empty(max(bound, 1), dtype=torch.int32, device=dev)
+    call("gs_bucket_fill", ptr(boff), T, ptr(b2t), bound, st)
+    nb = _host_sum(boff.data_ptr() + 4 * T, 1, st) if m > 0 else 0
     return RectBins(point_list, ranges, tile_offsets, boff, b2t[:nb], order, nb)
 
 

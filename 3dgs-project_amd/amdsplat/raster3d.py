@@ -42,15 +42,6 @@ def _u8(nbytes: int, device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
-def _layout(parts: dict):
-    """Byte offsets (256-byte aligned) of named regions of one allocation, and its size."""
-    offs, total = {}, 0
-    for name, nbytes in parts.items():
-        offs[name] = total
-        total += (int(nbytes) + 255) & ~255
-    return offs, max(total, 1)
-
-
 @dataclass
 class Camera:
     """Pinhole camera: row-major world-to-camera `viewmat` (4x4, OpenCV axes) and intrinsics."""
@@ -133,6 +124,76 @@ class ForwardState:
         return int(self.bucket_offsets[-1].item())
 
 
+class _View:
+    """Device buffers of one forward pass as the operator keeps them: a state arena whose regions do
+    not depend on the instance count and a list arena whose regions do (gs_view_plan and
+    gs_view_plan_count give the offsets). Two allocations, and no tensor object per buffer, which
+    the small views' host time depends on; state() makes the ForwardState of the same buffers."""
+
+    def __init__(self, cam: Camera, ccam, n: int, sh_coeffs: int, sh_degree: int, flags: int, bg: tuple):
+        self.cam, self.ccam = cam, ccam  # ccam: the camera as the C calls take it (built once per forward)
+        self.n, self.sh_coeffs, self.sh_degree, self.bg = n, sh_coeffs, sh_degree, bg
+        self._flags = flags
+        self.m = self.n_buckets_max = 0
+        self.path = _lib.GS_BIN_PATH_RADIX
+        self.touched = self.image = self.alpha = None
+        self.timings: dict = {}
+        self._state = self._lists = self._grads = None
+        self._soff, self._loff = _lib.ViewStateOffsets(), _lib.ViewListOffsets()
+
+    def _view(self, arena, off, count, dtype, *shape):
+        size = count * (8 if dtype in (torch.int64, torch.float64) else 4)
+        return arena[off:off + size].view(dtype).view(*shape)
+
+    def _s(self, region: int, count: int, dtype, *shape):
+        return self._view(self._state, self._soff[region], count, dtype, *shape)
+
+    def _l(self, region: int, count: int, dtype, *shape):
+        return self._view(self._lists, self._loff[region], count, dtype, *shape)
+
+    def state_ptr(self, region: int) -> int:
+        return self._state.data_ptr() + self._soff[region]
+
+    def list_ptr(self, region: int) -> int:
+        return self._lists.data_ptr() + self._loff[region]
+
+    @property
+    def for_backward(self) -> bool:
+        return bool(self._flags & _lib.GS_VIEW_BACKWARD)
+
+    def bucket_offsets(self) -> torch.Tensor:
+        T = self.cam.n_tiles
+        return self._s(_lib.VIEW_BUCKET_OFFSETS, T + 1, torch.int32, T + 1)
+
+    def state(self) -> "ForwardState":
+        n, m, nb, T = self.n, self.m, self.n_buckets_max, self.cam.n_tiles
+        H, W = self.cam.height, self.cam.width
+        i32, f32 = torch.int32, torch.float32
+        back, image = self.for_backward, self.image is not None
+        m_keys = m if self._flags & _lib.GS_VIEW_KEYS else 0
+        grad2d, conic64 = _split_grads2d(self._grads, n) if back else (None, None)
+        return ForwardState(
+            cam=self.cam, n=n, sh_coeffs=self.sh_coeffs, sh_degree=self.sh_degree,
+            rec=self._s(_lib.VIEW_REC, n * REC_FLOATS, f32, n, REC_FLOATS), touched=self.touched,
+            order=self._s(_lib.VIEW_ORDER, n, i32, n),
+            offsets=None if self.path == _lib.GS_BIN_PATH_SPANS else self._s(_lib.VIEW_OFFSETS, n + 1, i32, n + 1),
+            path=self.path, m=m, keys=self._l(_lib.VIEW_SORTED_KEYS, m_keys, torch.int64, m_keys),
+            point_list=self._l(_lib.VIEW_POINT_LIST, m, i32, m), ranges=self._s(_lib.VIEW_RANGES, 2 * T, i32, T, 2),
+            bucket_offsets=self.bucket_offsets(), n_buckets_max=nb,
+            bucket_to_tile=self._l(_lib.VIEW_BUCKET_TO_TILE, nb, i32, nb) if back else None,
+            image=self.image, final_T=self._s(_lib.VIEW_FINAL_T, H * W, f32, H, W) if image else None,
+            n_contrib=self._s(_lib.VIEW_N_CONTRIB, H * W, i32, H, W) if back else None,
+            tile_max=self._s(_lib.VIEW_TILE_MAX, T, i32, T) if back else None,
+            ckpt=self._l(_lib.VIEW_CKPT, 1024 * nb, f32, nb, 256, 4) if back else None,
+            bucket_list=self._l(_lib.VIEW_BUCKET_LIST, 4 + nb, i32, 4 + nb) if back else None, bg=self.bg,
+            timings=self.timings, grad2d=grad2d, grad_conic64=conic64, ccam=self.ccam, alpha=self.alpha)
+
+
+def _split_grads2d(g: torch.Tensor, n: int):
+    """(grad2d [n, 12], conic64 [n, 4] float64) of the buffer that holds both."""
+    return g[:n * GRAD2D_FLOATS].view(n, GRAD2D_FLOATS), g[n * GRAD2D_FLOATS:].view(torch.float64).view(n, 4)
+
+
 class StageTimer:
     """Records torch.cuda events on the current stream between stages (no-op if disabled)."""
 
@@ -211,6 +272,13 @@ def forward_pass(means, log_scales, quats, opacity_logits, sh, cam: Camera, sh_d
     """Runs the forward stages; inputs are contiguous float32 CUDA tensors (raw parameters). sh is
     [N, K, 3] or the (DC [N, 1, 3], rest [N, K - 1, 3]) pair. for_backward=False is the inference
     blend: no bucket table, checkpoints or n_contrib (those fields are None), same image bits."""
+    return _forward(means, log_scales, quats, opacity_logits, sh, cam, sh_degree, bg, timing, keep_keys, for_backward,
+                    _scores).state()
+
+
+def _forward(means, log_scales, quats, opacity_logits, sh, cam: Camera, sh_degree, bg, timing=False, keep_keys=False,
+             for_backward=True, scores=None) -> _View:
+    """forward_pass, without a tensor object per buffer. scores: the pruning scores instead of an image."""
     means, log_scales, quats = means.contiguous(), log_scales.contiguous(), quats.contiguous()
     opacity_logits = opacity_logits.contiguous()
     sh_a, sh_b, K = _sh_parts(sh)
@@ -219,125 +287,118 @@ def forward_pass(means, log_scales, quats, opacity_logits, sh, cam: Camera, sh_d
     dev = means.device
     if sh_degree is None:
         sh_degree = int(round(math.sqrt(K))) - 1
-    ccam = cam.c_struct()
     st = _lib.stream_handle(dev)
     tm = timing if isinstance(timing, StageTimer) else StageTimer(bool(timing))
     tm.mark("start")
-
-    rec = torch.empty(n, REC_FLOATS, dtype=torch.float32, device=dev)
-    touched = torch.empty(n, dtype=torch.int32, device=dev)
-    dkeys = torch.empty(n, dtype=torch.int32, device=dev)
-    n_waves = (n + 63) // 64
-    wave_counts = torch.empty(n_waves, dtype=torch.int32, device=dev)
-    call("gs_preprocess_fwd", ptr(means), ptr(log_scales), ptr(quats), ptr(opacity_logits), ptr(sh_a), ptr(sh_b),
-         n, K, sh_degree, ccam, ptr(rec), ptr(touched), ptr(dkeys), ptr(wave_counts), st)
-    tm.mark("preprocess")
-    # The instance count m (the total of the per-wavefront tile counts) needs only the
-    # preprocess: the library's side stream sums the counts and copies the total to host memory
-    # while the depth sort runs on this stream, so the host sizes the fill's buffers without the
-    # stream draining first.
-    counting = n > 0
-    if counting:
-        call("gs_count_begin", ptr(wave_counts), n_waves, int(COUNT_ON_SIDE_STREAM), st)
+    flags = (_lib.GS_VIEW_BACKWARD if for_backward and scores is None else 0) | \
+        (_lib.GS_VIEW_KEYS if keep_keys else 0) | (_lib.GS_VIEW_NO_IMAGE if scores is not None else 0)
+    ccam = cam.c_struct()
+    fs = _View(cam, ccam, n, K, sh_degree, flags, tuple(bg))
+    sizes = _lib.ViewSizes()
+    call("gs_view_plan", n, ccam, flags, fs._soff, sizes)
+    fs.path = sizes[2]
+    state = fs._state = _u8(sizes[0], dev)
+    scratch = _u8(sizes[1], dev)
+    touched = fs.touched = torch.empty(n, dtype=torch.int32, device=dev)
+    params = (ptr(means), ptr(log_scales), ptr(quats), ptr(opacity_logits), ptr(sh_a), ptr(sh_b), n, K, sh_degree)
+    # The instance count m (the total of the preprocess's per-wavefront tile counts) needs only the
+    # preprocess: its sum goes straight to host memory while the depth sort runs, so the host sizes
+    # the count-dependent buffers without the stream draining first.
+    one_call = n > 0 and not tm.enabled and not COUNT_ON_SIDE_STREAM
+    if one_call:
+        call("gs_view_begin", *params, ccam, flags, state.data_ptr(), touched.data_ptr(), scratch.data_ptr(), st)
+    else:
+        held = _begin_stages(fs, params, scratch, tm, st)  # noqa: F841 (read until the count has ended)
     try:
-        return _forward_rest(means, sh_a, sh_b, K, n, dev, sh_degree, cam, ccam, st, tm, rec, touched, dkeys, bg,
-                             timing, keep_keys, for_backward, _scores, counting)
+        return _forward_rest(fs, dev, st, tm, scratch, timing, keep_keys, scores)
     except BaseException:
-        if counting:
+        if n > 0:
             try:
-                _count_end()  # the side stream's copy is done before any buffer it reads is freed
+                _count_end()  # the count is done before any buffer it reads is freed
             except _lib.AmdSplatError:
                 pass
         raise
 
 
-def _forward_rest(means, sh_a, sh_b, K, n, dev, sh_degree, cam, ccam, st, tm, rec, touched, dkeys, bg, timing,
-                  keep_keys, for_backward, _scores, counting):
-    """forward_pass after the preprocess: the depth ordering, the count, the fill and the blend."""
-    T = cam.n_tiles
-    H, W = cam.height, cam.width
-    # The tile binning's path: the radix path takes the depth order and the instance offsets in
-    # that order; the span binning the depth order alone.
-    path = _lib.lib().gs_bin_path(n, ccam)
-    order = torch.empty(n, dtype=torch.int32, device=dev)
-    offsets = torch.empty(n + 1, dtype=torch.int32, device=dev) if path != _lib.GS_BIN_PATH_SPANS else None
-    ws = _u8(_lib.size_call("gs_bin_prepare_workspace_size", n), dev)
-    call("gs_bin_prepare_3d", ptr(rec), ptr(touched), ptr(dkeys), n, ccam, ptr(order), ptr(offsets), ptr(ws),
-         ws.numel(), st)
+def _begin_stages(fs: _View, params, scratch, tm, st):
+    """gs_view_begin stage by stage: with stage marks between, the count on its side stream, or an
+    empty scene. Returns the wave counts, which the caller holds until the count has ended."""
+    n, ccam = fs.n, fs.ccam
+    rec = fs.state_ptr(_lib.VIEW_REC) if n else None
+    dkeys = scratch.data_ptr() if n else None  # (the scratch's first region)
+    n_waves = (n + 63) // 64
+    waves = torch.empty(n_waves, dtype=torch.int32, device=scratch.device)
+    call("gs_preprocess_fwd", *params, ccam, rec, ptr(fs.touched), dkeys, ptr(waves), st)
+    tm.mark("preprocess")
+    if n > 0:
+        call("gs_count_begin", ptr(waves), n_waves, int(COUNT_ON_SIDE_STREAM), st)
+    try:
+        ws = _u8(_lib.size_call("gs_bin_prepare_workspace_size", n), scratch.device)
+        offsets = None if fs.path == _lib.GS_BIN_PATH_SPANS else fs.state_ptr(_lib.VIEW_OFFSETS)
+        call("gs_bin_prepare_3d", rec, ptr(fs.touched), dkeys, n, ccam, fs.state_ptr(_lib.VIEW_ORDER) if n else None,
+             offsets, ptr(ws), ws.numel(), st)
+    except BaseException:
+        if n > 0:
+            _count_end()
+        raise
     tm.mark("depth_order")
-    # Everything whose size does not depend on the instance count is allocated while the copy
-    # and the depth sort run; after the count arrives the host only carves the count-sized
-    # buffers out of one allocation and launches the fill, before the depth sort ends.
-    ranges = torch.empty(T, 2, dtype=torch.int32, device=dev)
-    bucket_offsets = torch.empty(T + 1, dtype=torch.int32, device=dev)
-    backward_state = for_backward and _scores is None
-    n_contrib = tile_max = grad2d = conic64 = gbuf = image = final_T = alpha = None
-    if backward_state:
-        n_contrib = torch.empty(H, W, dtype=torch.int32, device=dev)
-        tile_max = torch.empty(T, dtype=torch.int32, device=dev)
+    return waves
+
+
+def _forward_rest(fs: _View, dev, st, tm, scratch, timing, keep_keys, scores):
+    """forward_pass after the depth ordering is enqueued: the count, the fill and the blend."""
+    cam, ccam, n, flags = fs.cam, fs.ccam, fs.n, fs._flags
+    H, W = cam.height, cam.width
+    # what does not depend on the instance count is allocated while the depth sort runs
+    grads = None
+    if fs.for_backward:
         # the backward's screen gradients [n, 12] float32 and the elongated splats' float64 conic
         # sums [n, 4], one buffer that the forward blend's workgroups zero
-        gbuf = torch.empty(n * (GRAD2D_FLOATS + 8), dtype=torch.float32, device=dev)
-        grad2d = gbuf[:n * GRAD2D_FLOATS].view(n, GRAD2D_FLOATS)
-        conic64 = gbuf[n * GRAD2D_FLOATS:].view(torch.float64).view(n, 4)
-    if _scores is None:
-        image = torch.empty(3, H, W, dtype=torch.float32, device=dev)
-        final_T = torch.empty(H, W, dtype=torch.float32, device=dev)
-        alpha = torch.empty(H, W, dtype=torch.float32, device=dev)
-    # addresses the calls after the readback take (ctypes conversions done before the wait)
-    p_rec, p_dkeys, p_order, p_offsets = ptr(rec), ptr(dkeys), ptr(order), ptr(offsets)
-    p_ranges, p_boff, bg3 = ptr(ranges), ptr(bucket_offsets), _lib.float3(bg)
-    m = 0
-    if counting:
-        m = _count_end()
-        if m >= 1 << 32:
-            raise _lib.AmdSplatError(f"{m} tile instances exceed the 32-bit instance index")
-    nb_max = (m + (BUCKET - 1) * T) // BUCKET if backward_state else 0  # >= sum over tiles of ceil(len / 32)
+        grads = fs._grads = torch.empty(n * (GRAD2D_FLOATS + 8), dtype=torch.float32, device=dev)
+    if scores is None:
+        fs.image = torch.empty(3, H, W, dtype=torch.float32, device=dev)
+        fs.alpha = torch.empty(H, W, dtype=torch.float32, device=dev)
+    bg3 = _lib.float3(fs.bg)
+    if n > 0:
+        fs.m = _count_end()
+        if fs.m >= 1 << 32:
+            raise _lib.AmdSplatError(f"{fs.m} tile instances exceed the 32-bit instance index")
+    m = fs.m
+    sizes = _lib.ViewSizes()
+    call("gs_view_plan_count", n, m, ccam, flags, fs._loff, sizes)
+    fs.n_buckets_max = sizes[2]
     # the fill's scratch is its own allocation, released when this function returns: nothing the
     # blends or the backward read lives in it (the caching allocator reuses it in stream order)
-    ws_fill = _u8(_lib.lib().gs_bin_fill_3d_workspace_size(n, m, ccam), dev)
-    parts = {"point_list": 4 * m, "keys": 8 * m if keep_keys else 0}
-    if backward_state:
-        parts.update(bucket_to_tile=4 * max(nb_max, 1), blist=4 * (4 + nb_max), ckpt=4096 * max(nb_max, 1))
-    offs, total = _layout(parts)
-    arena = torch.empty(total, dtype=torch.uint8, device=dev)
-    # the kernels are launched from raw addresses; the tensor views are made after the launches,
-    # so that the host reaches the fill while the depth sort still runs
-    base = arena.data_ptr()
-    adr = {k: (base + o if parts[k] > 0 else None) for k, o in offs.items()}
+    ws = _u8(sizes[1], dev)
+    lists = fs._lists = _u8(sizes[0], dev)
+    clear, n_clear = (ptr(grads), grads.numel()) if grads is not None else (None, 0)
+    if scores is None and not keep_keys and not tm.enabled:
+        call("gs_view_finish", n, m, ccam, flags, fs._state.data_ptr(), lists.data_ptr(), ws.data_ptr(), ws.numel(), bg3,
+             fs.image.data_ptr(), fs.alpha.data_ptr(), clear, n_clear, st)
+        return fs
+    back = fs.for_backward
+    rec = fs.state_ptr(_lib.VIEW_REC) if n else None
+    point_list = fs.list_ptr(_lib.VIEW_POINT_LIST) if m else None
+    ranges, boff = fs.state_ptr(_lib.VIEW_RANGES), fs.state_ptr(_lib.VIEW_BUCKET_OFFSETS)
+    blist = fs.list_ptr(_lib.VIEW_BUCKET_LIST) if back else None
     # the fill also clears the bucket list's header for the forward blend
-    call("gs_bin_fill_3d", p_rec, p_dkeys, p_order, p_offsets, n, ccam, m, adr["keys"], adr["point_list"], p_ranges,
-         p_boff, adr.get("blist"), ptr(ws_fill), ws_fill.numel(), st)
+    call("gs_bin_fill_3d", rec, scratch.data_ptr() if n else None, fs.state_ptr(_lib.VIEW_ORDER) if n else None,
+         None if fs.path == _lib.GS_BIN_PATH_SPANS else fs.state_ptr(_lib.VIEW_OFFSETS), n, ccam, m,
+         fs.list_ptr(_lib.VIEW_SORTED_KEYS) if keep_keys and m else None, point_list, ranges, boff, blist, ptr(ws),
+         ws.numel(), st)
     tm.mark("binning")
-    if _scores is None:
-        call("gs_blend_fwd_3d", p_rec, p_ranges, adr["point_list"], p_boff, W, H, bg3, ptr(image), ptr(final_T),
-             ptr(alpha), ptr(n_contrib), ptr(tile_max), adr.get("ckpt"), adr.get("blist"), adr.get("bucket_to_tile"),
-             ptr(gbuf), gbuf.numel() if gbuf is not None else 0,
-             _lib.GS_BLEND_LIST_CLEARED if backward_state else 0, st)
-    else:  # pruning scores: the blend's weights, no image
-        call("gs_blend_scores_3d", p_rec, p_ranges, adr["point_list"], W, H, n, ptr(_scores), st)
-
-    def view(name, dtype):
-        o = offs[name]
-        return arena[o:o + parts[name]].view(dtype)
-
-    point_list = view("point_list", torch.int32)
-    keys = view("keys", torch.int64) if keep_keys else torch.empty(0, dtype=torch.int64, device=dev)
-    if _scores is not None:
+    if scores is not None:  # pruning scores: the blend's weights, no image
+        call("gs_blend_scores_3d", rec, ranges, point_list, W, H, n, ptr(scores), st)
         tm.mark("scores")
-        return ForwardState(cam, n, K, sh_degree, rec, touched, order, offsets, path, m, keys, point_list, ranges,
-                            bucket_offsets, 0, None, None, None, None, None, None, None, tuple(bg),
-                            {} if isinstance(timing, StageTimer) else tm.result())
-    bucket_to_tile = ckpt = blist = None
-    if backward_state:
-        bucket_to_tile = view("bucket_to_tile", torch.int32)
-        blist = view("blist", torch.int32)
-        ckpt = view("ckpt", torch.float32).view(max(nb_max, 1), 256, 4)
-    tm.mark("blend_fwd")
-    return ForwardState(cam, n, K, sh_degree, rec, touched, order, offsets, path, m, keys, point_list, ranges,
-                        bucket_offsets, nb_max, bucket_to_tile, image, final_T, n_contrib, tile_max, ckpt, blist,
-                        tuple(bg),
-                        {} if isinstance(timing, StageTimer) else tm.result(), grad2d, conic64, ccam, None, alpha)
+    else:
+        call("gs_blend_fwd_3d", rec, ranges, point_list, boff, W, H, bg3, ptr(fs.image), fs.state_ptr(_lib.VIEW_FINAL_T),
+             ptr(fs.alpha), fs.state_ptr(_lib.VIEW_N_CONTRIB) if back else None,
+             fs.state_ptr(_lib.VIEW_TILE_MAX) if back else None, fs.list_ptr(_lib.VIEW_CKPT) if back else None, blist,
+             fs.list_ptr(_lib.VIEW_BUCKET_TO_TILE) if back and fs.n_buckets_max else None, clear, n_clear,
+             _lib.GS_BLEND_LIST_CLEARED if back else 0, st)
+        tm.mark("blend_fwd")
+    fs.timings = {} if isinstance(timing, StageTimer) else tm.result()
+    return fs
 
 
 def backward_pass(fs: ForwardState, means, log_scales, quats, opacity_logits, sh, grad_image,
@@ -374,6 +435,17 @@ def backward_pass(fs: ForwardState, means, log_scales, quats, opacity_logits, sh
          ptr(grad2d), ptr(conic64),
          _lib.GS_ACCUMULATE | (_lib.GS_ABS_GRAD if abs_grad else 0), ptr(counters), st)
     tm.mark("blend_bwd")
+    params, (g_means, g_ls, g_q, g_op, g_sh), outs = _backward_args(fs, means, log_scales, quats, opacity_logits, sh)
+    call("gs_preprocess_bwd", *params, fs.ccam if fs.ccam is not None else cam.c_struct(), ptr(fs.touched),
+         ptr(grad2d), ptr(conic64), *outs, st)
+    tm.mark("preprocess_bwd")
+    return g_means, g_ls, g_q, g_op, g_sh, grad2d, {} if isinstance(timing, StageTimer) else tm.result()
+
+
+def _backward_args(fs, means, log_scales, quats, opacity_logits, sh):
+    """The parameters as the backward calls take them, the gradient tensors (that of the SH a pair
+    when sh is) and their addresses."""
+    n, dev = fs.n, means.device
     g_means = torch.empty(n, 3, dtype=torch.float32, device=dev)
     g_ls = torch.empty(n, 3, dtype=torch.float32, device=dev)
     g_q = torch.empty(n, 4, dtype=torch.float32, device=dev)
@@ -388,12 +460,27 @@ def backward_pass(fs: ForwardState, means, log_scales, quats, opacity_logits, sh
         g_a = torch.empty(n, 1, 3, dtype=torch.float32, device=dev)
         g_b = torch.empty(n, fs.sh_coeffs - 1, 3, dtype=torch.float32, device=dev)
         g_sh = (g_a, g_b)
-    call("gs_preprocess_bwd", ptr(means), ptr(log_scales), ptr(quats), ptr(opacity_logits), ptr(sh_a), ptr(sh_b),
-         n, fs.sh_coeffs, fs.sh_degree, fs.ccam if fs.ccam is not None else cam.c_struct(), ptr(fs.touched),
-         ptr(grad2d), ptr(conic64), ptr(g_means),
-         ptr(g_ls), ptr(g_q), ptr(g_op), ptr(g_a), ptr(g_b), st)
-    tm.mark("preprocess_bwd")
-    return g_means, g_ls, g_q, g_op, g_sh, grad2d, {} if isinstance(timing, StageTimer) else tm.result()
+    params = (ptr(means), ptr(log_scales), ptr(quats), ptr(opacity_logits), ptr(sh_a), ptr(sh_b), n, fs.sh_coeffs,
+              fs.sh_degree)
+    return params, (g_means, g_ls, g_q, g_op, g_sh), (ptr(g_means), ptr(g_ls), ptr(g_q), ptr(g_op), ptr(g_a), ptr(g_b))
+
+
+def _backward(view: _View, means, log_scales, quats, opacity_logits, sh, grad_image, grad_alpha, abs_grad: bool):
+    """backward_pass of an operator's view in one call."""
+    st = _lib.stream_handle(means.device)
+    grad_image = grad_image.contiguous().float()
+    if grad_alpha is not None:
+        grad_alpha = grad_alpha.contiguous().float()
+    # zeroed by the forward blend; a second backward of the same forward starts from zeros
+    grads, view._grads = view._grads, None
+    if grads is None:
+        grads = torch.zeros(view.n * (GRAD2D_FLOATS + 8), dtype=torch.float32, device=means.device)
+    grad2d, conic64 = _split_grads2d(grads, view.n)
+    params, gs, outs = _backward_args(view, means, log_scales, quats, opacity_logits, sh)
+    call("gs_view_backward", *params, view.m, view.ccam, view._state.data_ptr(), view._lists.data_ptr(), ptr(view.touched),
+         ptr(view.image), ptr(grad_image), ptr(grad_alpha), ptr(grad2d), ptr(conic64),
+         _lib.GS_ABS_GRAD if abs_grad else 0, *outs, st)
+    return *gs, grad2d
 
 
 def combined_grad2d(grad2d: torch.Tensor, conic64: torch.Tensor | None) -> torch.Tensor:
@@ -434,8 +521,12 @@ class _Rasterize3D(torch.autograd.Function):
     def forward(ctx, means, log_scales, quats, opacity_logits, sh, sh_rest, cam, sh_degree, bg, dinfo=None,
                 timer=None):
         shp = sh if sh_rest is None else (sh, sh_rest)
-        fs = forward_pass(means, log_scales, quats, opacity_logits, shp, cam, sh_degree, bg,
-                          timing=timer if timer is not None else False)
+        if timer is None:
+            fs = _forward(means, log_scales, quats, opacity_logits, shp, cam, sh_degree, bg)
+            n_buckets = fs.bucket_offsets()[-1]
+        else:  # stage by stage
+            fs = forward_pass(means, log_scales, quats, opacity_logits, shp, cam, sh_degree, bg, timing=timer)
+            n_buckets = fs.bucket_offsets[-1]
         # an output the loss does not use gets None, not a zero tensor: an alpha nobody
         # differentiates costs the backward nothing
         ctx.set_materialize_grads(False)
@@ -445,8 +536,6 @@ class _Rasterize3D(torch.autograd.Function):
         ctx.split = sh_rest is not None
         ctx.save_for_backward(means, log_scales, quats, opacity_logits, sh, sh_rest)
         alpha = fs.alpha.detach()  # 1 - final_T, written by the blend
-        n_buckets = fs.bucket_offsets[-1]
-        m = torch.tensor(fs.m, dtype=torch.int64)  # host tensor: the count is already on the host
         # The outputs are new tensor objects over the forward state's storage: were they the
         # state's own objects, output -> grad_fn -> ctx -> state -> output would be a reference
         # cycle, and each view's buffers (about 1 GB at 1M Gaussians) would wait for Python's
@@ -454,8 +543,8 @@ class _Rasterize3D(torch.autograd.Function):
         image, touched = fs.image.detach(), fs.touched.detach()
         if _Rasterize3D.track_visibility:
             _Rasterize3D.last_visibility = touched
-        ctx.mark_non_differentiable(touched, n_buckets, m)
-        return image, alpha, touched, n_buckets, m
+        ctx.mark_non_differentiable(touched, n_buckets)
+        return image, alpha, touched, n_buckets, fs.m  # (m: a host int)
 
     @staticmethod
     def backward(ctx, grad_image, grad_alpha, _grad_touched, _grad_nb, _grad_m):
@@ -466,11 +555,12 @@ class _Rasterize3D(torch.autograd.Function):
         shp = (sh, sh_rest) if ctx.split else sh
         # |dL/dmean2d| only when the caller's densification_info has its third row
         abs_grad = ctx.dinfo is not None and ctx.dinfo.shape[0] == 3
-        gm, gls, gq, gop, gsh, grad2d, _ = backward_pass(fs, means.contiguous(), log_scales.contiguous(),
-                                                         quats.contiguous(), opacity_logits.contiguous(),
-                                                         shp, grad_image, grad_alpha,
-                                                         timing=ctx.timer if ctx.timer is not None else False,
-                                                         abs_grad=abs_grad)
+        params = (means.contiguous(), log_scales.contiguous(), quats.contiguous(), opacity_logits.contiguous(), shp)
+        if ctx.timer is None:
+            gm, gls, gq, gop, gsh, grad2d = _backward(fs, *params, grad_image, grad_alpha, abs_grad)
+        else:
+            gm, gls, gq, gop, gsh, grad2d, _ = backward_pass(fs, *params, grad_image, grad_alpha, timing=ctx.timer,
+                                                             abs_grad=abs_grad)
         ctx.grad2d = grad2d
         if ctx.dinfo is not None:
             densification_stats(grad2d, fs.touched, fs.cam.width, fs.cam.height, ctx.dinfo)
@@ -523,7 +613,7 @@ def rasterize(means, scales, quats, opacities, sh, viewmat, K, W: int, H: int, b
     timer = StageTimer(True) if timing else None
     image, alpha, touched, n_buckets, m = _Rasterize3D.apply(means, scales, quats, opacities, sh_a, sh_b, cam,
                                                              sh_degree, bg, densification_info, timer)
-    aux = _Aux(tiles_touched=touched, visibility=touched, n_instances=int(m.item()), n_buckets=n_buckets)
+    aux = _Aux(tiles_touched=touched, visibility=touched, n_instances=m, n_buckets=n_buckets)
     if timer is not None:
         aux["timings"] = timer
     return image, alpha, aux
@@ -548,9 +638,9 @@ def rasterize_inference(means, scales, quats, opacities, sh, viewmat, K, W: int,
     means, scales, quats, opacities, sh = _prepare(means, scales, quats, opacities, sh, activated)
     cam = Camera.from_K(viewmat, K, W, H, near, far, proper_antialiasing, BINNING)
     bg = (0.0, 0.0, 0.0) if bg is None else tuple(float(x) for x in (bg.tolist() if torch.is_tensor(bg) else bg))
-    fs = forward_pass(means.detach(), scales.detach(), quats.detach(), opacities.detach(),
-                      tuple(t.detach() for t in sh) if isinstance(sh, tuple) else sh.detach(), cam,
-                      sh_degree=sh_degree, bg=bg, for_backward=False)
+    fs = _forward(means.detach(), scales.detach(), quats.detach(), opacities.detach(),
+                  tuple(t.detach() for t in sh) if isinstance(sh, tuple) else sh.detach(), cam, sh_degree, bg,
+                  for_backward=False)
     return fs.image, fs.alpha
 
 
@@ -570,7 +660,7 @@ def pruning_scores(means, scales, quats, opacities, sh, viewmat, K, W: int, H: i
     if tuple(scores.shape) != (n,) or scores.dtype != torch.float32 or not scores.is_contiguous() \
             or scores.device != means.device:
         raise ValueError(f"scores must be a contiguous float32 [{n}] tensor on {means.device}")
-    forward_pass(means.detach(), scales.detach(), quats.detach(), opacities.detach(),
-                 tuple(t.detach() for t in sh) if isinstance(sh, tuple) else sh.detach(), cam,
-                 sh_degree=sh_degree, _scores=scores)
+    _forward(means.detach(), scales.detach(), quats.detach(), opacities.detach(),
+             tuple(t.detach() for t in sh) if isinstance(sh, tuple) else sh.detach(), cam, sh_degree, (0.0, 0.0, 0.0),
+             scores=scores)
     return scores

@@ -56,7 +56,7 @@ def bin_gaussians(means: torch.Tensor, radii: torch.Tensor, depth: torch.Tensor,
     rect = torch.empty(n, 4, dtype=torch.int32, device=dev)
     counts = torch.empty(n, dtype=torch.int32, device=dev)
     call("gs2d_rects_toy", ptr(m32), ptr(r32), n, W, H, ptr(rect), ptr(counts), R2.stream(dev))
-    rb = R2.bin_rects(rect, counts, depth, W, H, want_order=True)
+    rb = R2.bin_rects(rect, counts, depth, W, H, want_order=True, want_tile_offsets=False)
     T = tiles_x * tiles_y
     return Bins(H, W, tiles_x, tiles_y, rect, rb.order.long(), rb.point_list, rb.ranges,
                 rb.bucket_offsets[:T], rb.bucket_to_tile, rb.num_buckets, rb.bucket_offsets)

@@ -115,8 +115,6 @@ def rasterize(means, conic, color, opacity, bins: Bins, bg=None, backend: str = 
     """Render a (3, H, W) image. backend: 'splat' (HIP, bucketed backward), 'pixel' (HIP,
     per-pixel backward) or 'ref' (render_reference: dense PyTorch ops on the tensors' device,
     autograd gradients; only when asked for by name)."""
-    if bg is None:
-        bg = torch.zeros(3, dtype=means.dtype, device=means.device)
     if backend == "ref":
         return render_reference(means, conic, color, opacity, bins, bg)
     if backend not in ("pixel", "splat"):

@@ -301,6 +301,51 @@ int gs_preprocess_bwd(const float* means, const float* log_scales, const float* 
                       float* grad_log_scales, float* grad_quats, float* grad_opacity_logits,
                       float* grad_sh, float* grad_sh_rest, void* stream);
 
+/* ---------------------------------------------------------------------------------------
+ * One view in three calls over two arenas: the entry points above run in order with the buffers
+ * between them carved from memory the caller allocates (torch: two tensors instead of a dozen).
+ * The results are those of the separate calls.
+ *   flags: GS_VIEW_BACKWARD (keep what the backward reads; without it the inference forward),
+ *   GS_VIEW_KEYS (room for the sorted 64-bit keys), GS_VIEW_NO_IMAGE (no image, hence no final_T).
+ * gs_view_plan: state_offsets[GS_VIEW_STATE_REGIONS] receives the byte offset of every region of
+ *   the state arena (GS_VIEW_REC ...), sizes[0] its size, sizes[1] the size of gs_view_begin's
+ *   scratch (its first 4 n bytes are the depth keys), sizes[2] the binning path (GS_BIN_PATH_*).
+ * gs_view_begin (n > 0): gs_preprocess_fwd, gs_count_begin (on the stream), gs_bin_prepare_3d. The
+ *   caller then takes the instance count m from gs_count_end.
+ * gs_view_plan_count: the same for the list arena: list_offsets[GS_VIEW_LIST_REGIONS], sizes[0] its
+ *   size, sizes[1] the fill's workspace, sizes[2] the bucket bound (m + 31 T) / 32.
+ * gs_view_finish: gs_bin_fill_3d and gs_blend_fwd_3d (flags 0 or GS_VIEW_BACKWARD).
+ * gs_view_backward: gs_blend_bwd_3d (flags: GS_ABS_GRAD; it adds to grad2d and grad_conic64, which
+ *   start from zeros) and gs_preprocess_bwd, after a forward with GS_VIEW_BACKWARD.
+ * Both arenas and the scratch are 256-byte aligned.
+ * ------------------------------------------------------------------------------------- */
+enum { GS_VIEW_BACKWARD = 1, GS_VIEW_KEYS = 2, GS_VIEW_NO_IMAGE = 4 };
+enum {
+  GS_VIEW_REC = 0, GS_VIEW_ORDER, GS_VIEW_OFFSETS, GS_VIEW_RANGES, GS_VIEW_BUCKET_OFFSETS, GS_VIEW_FINAL_T,
+  GS_VIEW_N_CONTRIB, GS_VIEW_TILE_MAX, GS_VIEW_STATE_REGIONS
+};
+enum {
+  GS_VIEW_POINT_LIST = 0, GS_VIEW_BUCKET_TO_TILE, GS_VIEW_BUCKET_LIST, GS_VIEW_CKPT, GS_VIEW_SORTED_KEYS,
+  GS_VIEW_LIST_REGIONS
+};
+int gs_view_plan(int64_t n, const gs_camera* cam, int flags, int64_t* state_offsets, int64_t* sizes);
+int gs_view_begin(const float* means, const float* log_scales, const float* quats, const float* opacity_logits,
+                  const float* sh, const float* sh_rest, int64_t n, int sh_coeffs, int sh_degree,
+                  const gs_camera* cam, int flags, void* state, uint32_t* tiles_touched, void* scratch,
+                  void* stream);
+int gs_view_plan_count(int64_t n, int64_t m, const gs_camera* cam, int flags, int64_t* list_offsets,
+                       int64_t* sizes);
+int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, void* lists,
+                   void* workspace, size_t workspace_bytes, const float* bg, float* image, float* alpha,
+                   float* clear, int64_t clear_floats, void* stream);
+int gs_view_backward(const float* means, const float* log_scales, const float* quats,
+                     const float* opacity_logits, const float* sh, const float* sh_rest, int64_t n,
+                     int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state, void* lists,
+                     const uint32_t* tiles_touched, const float* image, const float* grad_image,
+                     const float* grad_alpha, float* grad2d, double* grad_conic64, int flags, float* grad_means,
+                     float* grad_log_scales, float* grad_quats, float* grad_opacity_logits, float* grad_sh,
+                     float* grad_sh_rest, void* stream);
+
 /* Densification statistics of one backward, accumulated into info [rows, n] (rows 2 or 3) for
  * the visible Gaussians (tiles_touched > 0): info[0] += 1; info[1] += |(W/2 g_x, H/2 g_y)|, the
  * norm of the mean2d gradient in NDC units (grad2d[:, 0:2]); info[2] (rows == 3) += the same

@@ -306,3 +306,40 @@ def test_step_state_is_freed_without_the_cyclic_collector(surface):
     finally:
         gc.enable()
     assert grown <= 0, f"{grown} bytes still held after 4 steps"
+
+
+@gpu
+@pytest.mark.parametrize("binning", ["radix", "spans"])
+@pytest.mark.parametrize("n,W,H,split,behind", [
+    (0, 64, 48, False, False),     # no Gaussians
+    (100, 64, 48, True, True),     # none visible: no instances, an empty list arena
+    (1, 16, 16, False, False),     # one tile
+    (257, 33, 17, True, False),    # odd sizes: regions at their paddings
+    (20_001, 333, 250, False, False),
+])
+def test_one_call_view_equals_the_stages(n, W, H, split, behind, binning, monkeypatch):
+    """rasterize without stage marks (gs_view_begin, _finish, _backward over two arenas) against the
+    stage-by-stage calls that timing=True takes: the forward bit for bit, the gradients to the
+    atomics' order; a second backward of the same forward gives the first's gradients."""
+    monkeypatch.setattr(R, "BINNING", binning)
+    sc = scenes.small_scene(max(n, 1), W, H, seed=n)
+    cam = sc.cameras[0]
+    m, ls, q, op, sh = [t[:n].cuda().contiguous() for t in sc.params()]
+    if behind:
+        m = m * torch.tensor([1.0, 1.0, -1.0], device="cuda")
+    got = {}
+    gi = torch.randn(3, H, W, generator=torch.Generator().manual_seed(1)).cuda()
+    for timing in (False, True):
+        leaves = [t.clone().requires_grad_(True) for t in (m, ls, q, op, *((sh[:, :1], sh[:, 1:]) if split else (sh,)))]
+        img, alpha, aux = rasterize(*leaves[:4], tuple(leaves[4:]) if split else leaves[4], cam.viewmat, K_of(cam), W, H,
+                                    near=cam.near, far=cam.far, bg=(0.1, 0.2, 0.3), timing=timing)
+        g = torch.autograd.grad([img, alpha], leaves, [gi, gi[0]], retain_graph=True)
+        again = torch.autograd.grad([img, alpha], leaves, [gi, gi[0]])
+        got[timing] = (img, alpha, aux["tiles_touched"], aux["n_instances"], int(aux["n_buckets"]), g, again)
+    a, b = got[False], got[True]
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and torch.equal(a[2], b[2]) and a[3:5] == b[3:5]
+    assert (a[3] == 0) == (n == 0 or behind)
+    for x, y in [*zip(a[5], b[5]), *zip(a[5], a[6]), *zip(b[5], b[6])]:
+        assert x.shape == y.shape
+        # two orders of float32 sums of at most 256 * 16 terms per value and tile: 1e-5 of the norm
+        assert float((x - y).norm()) <= 1e-5 * float(y.norm())
