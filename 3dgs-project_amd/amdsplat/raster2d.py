@@ -86,7 +86,8 @@ def _host_sum(p: int, n: int, st) -> int:
 def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | None, width: int, height: int,
               want_order: bool = False, binning: str | None = None, want_tile_offsets: bool = True) -> RectBins:
     """Per-tile lists of the Gaussians whose tile rectangle covers the tile, in stable depth
-    order (depth given) or index order. Two host reads: the instance and bucket counts.
+    order (depth given) or index order. One host read, of the instance and bucket counts, before
+    the sort is enqueued (two, the second after it, on canvases beyond gs_rect_tiles_fit).
     binning: "auto", "spans" or "radix" (default: the module's BINNING); the lists are the same."""
     flags = _lib.BIN_FLAGS[binning or BINNING]
     dev = rects.device
@@ -94,11 +95,21 @@ def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | N
     tx, ty = tiles_of(width, height)
     T = tx * ty
     st = stream(dev)
-    m = _host_sum(ptr(counts), n, st) if n > 0 else 0
-    point_list = torch.empty(m, dtype=torch.int32, device=dev)
     ranges = torch.empty(T, 2, dtype=torch.int32, device=dev)
     tile_offsets = torch.empty(T + 1, dtype=torch.int32, device=dev) if want_tile_offsets else None
     boff = torch.empty(T + 1, dtype=torch.int32, device=dev)
+    m, nb = 0, None
+    if n > 0 and _lib.lib().gs_rect_tiles_fit(tx, ty):
+        ws = _u8(_lib.size_call("gs_rect_tiles_workspace_size", n, tx, ty), dev)
+        call("gs_rect_tiles_begin", ptr(rects), n, tx, ty, ranges.data_ptr(), ptr(tile_offsets), boff.data_ptr(),
+             ws.data_ptr(), ws.numel(), st)
+        mv, bv = C.c_uint64(), C.c_uint64()
+        call("gs_rect_tiles_end", C.byref(mv), C.byref(bv))
+        m, nb = int(mv.value), int(bv.value)
+        flags |= _lib.GS_BIN_TILES_KNOWN
+    elif n > 0:
+        m = _host_sum(ptr(counts), n, st)
+    point_list = torch.empty(m, dtype=torch.int32, device=dev)
     order = torch.empty(n, dtype=torch.int32, device=dev) if want_order else None
     d = None
     dcode = F32
@@ -110,11 +121,10 @@ def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | N
     ws = _u8(_lib.size_call("gs_bin_workspace_size", n, m, tx, ty, flags), dev)
     call("gs_bin_fill_rect", ptr(rects), ptr(d), dcode, ptr(counts), n, tx, ty, m, None, ptr(point_list), ptr(ranges),
          ptr(tile_offsets), ptr(boff), ptr(order), flags, ptr(ws), ws.numel(), st)
-    # the bucket table is filled to its bound (m + 31 T) / 32 while the host waits for the bucket count
-    bound = (m + (BUCKET - 1) * T) // BUCKET
-    b2t = torch.empty(max(bound, 1), dtype=torch.int32, device=dev)
-    call("gs_bucket_fill", ptr(boff), T, ptr(b2t), bound, st)
-    nb = _host_sum(boff.data_ptr() + 4 * T, 1, st) if m > 0 else 0
+    if nb is None:
+        nb = _host_sum(boff.data_ptr() + 4 * T, 1, st) if m > 0 else 0
+    b2t = torch.empty(max(nb, 1), dtype=torch.int32, device=dev)
+    call("gs_bucket_fill", ptr(boff), T, ptr(b2t), nb, st)
     return RectBins(point_list, ranges, tile_offsets, boff, b2t[:nb], order, nb)
 
 

@@ -27,11 +27,7 @@ __device__ __forceinline__ uint32_t block_inclusive_scan(uint32_t v, uint32_t* s
                                                          uint32_t& total) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t u = __shfl_up(v, off, 64);
-    if (lane >= off) v += u;
-  }
+  v = wave_incl_scan(v);
   if (lane == 63) s_wave[wave] = v;
   __syncthreads();
   uint32_t before = 0;
@@ -571,12 +567,8 @@ static void radix_sort(const K* k, const uint32_t* v, K* k_out, uint32_t* v_out,
 
 // Exclusive prefix sum over the wavefront; `total` receives the sum of all lanes.
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_t& total) {
-  uint32_t incl = v;
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t u = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += u;
-  }
-  total = __shfl(incl, kWave - 1, 64);
+  const uint32_t incl = wave_incl_scan(v);
+  total = wave_last(incl);
   return incl - v;
 }
 
@@ -873,97 +865,96 @@ __global__ __launch_bounds__(256) void tile_bounds_kernel(const uint32_t* __rest
   }
 }
 
-// One workgroup: bucket counts ceil(len / 32) per tile, their exclusive scan into
-// bucket_offsets [T + 1], and optionally the CSR tile offsets [T + 1]. With m == 0 it also
-// writes the (empty) ranges.
+// One workgroup of kBoThreads: the exclusive scans of the tiles' instance counts (count_of(t)) and of
+// their bucket counts ceil(len / 32); put(t, len, instances before, buckets before) for every tile.
+// A wavefront takes 512 consecutive tiles in rounds of 64, so that reads and writes are coalesced
+// (with eight consecutive tiles per thread the writes of 8160 tiles took 20 us of one CU).
 constexpr int kBoThreads = 1024;
 constexpr int kBoItems = 8;
 
-__global__ __launch_bounds__(kBoThreads) void bucket_offsets_kernel(uint32_t* __restrict__ ranges, int n_tiles,
-                                                                    int64_t m, uint32_t* __restrict__ boff,
-                                                                    uint32_t* __restrict__ tile_offsets,
-                                                                    uint32_t* __restrict__ list_header,
-                                                                    bool fix_empty) {
+template <typename F, typename P>
+__device__ __forceinline__ void tile_scan_block(F count_of, int n_tiles, P put, uint32_t* __restrict__ boff,
+                                                uint32_t* __restrict__ tile_offsets,
+                                                uint32_t* __restrict__ list_header) {
   __shared__ uint32_t s_wave[kBoThreads / kWave];
   __shared__ uint32_t s_wave_inst[kBoThreads / kWave];
   if (list_header && threadIdx.x < kListHeader) list_header[threadIdx.x] = 0u;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  // fix_empty: ranges come from the sort's atomic min / max, so a tile without instances still
-  // holds [~0, 0]; the instance counts are scanned beside the bucket counts and such a tile gets
-  // the empty range at its CSR position
   uint32_t run = 0, run_inst = 0;
   for (int c0 = 0; c0 < n_tiles; c0 += kBoThreads * kBoItems) {
-    uint32_t cnt[kBoItems], start[kBoItems], len[kBoItems], sum = 0, sum_inst = 0;
+    const int base = c0 + wave * (kWave * kBoItems) + lane;
+    uint32_t len[kBoItems], pos[kBoItems], pos_inst[kBoItems];
+#pragma unroll
+    for (int e = 0; e < kBoItems; ++e) len[e] = base + kWave * e < n_tiles ? count_of(base + kWave * e) : 0u;
 #pragma unroll
     for (int e = 0; e < kBoItems; ++e) {
-      const int t = c0 + static_cast<int>(threadIdx.x) * kBoItems + e;
-      cnt[e] = 0;
-      start[e] = 0;
-      len[e] = 0;
-      if (t < n_tiles) {
-        if (m > 0) {
-          start[e] = ranges[2 * t];
-          const uint32_t end = ranges[2 * t + 1];
-          len[e] = (fix_empty && start[e] == 0xffffffffu) ? 0u : end - start[e];
-          cnt[e] = (len[e] + kBucket - 1) / kBucket;
-        } else {
-          ranges[2 * t] = 0;
-          ranges[2 * t + 1] = 0;
-        }
-      }
-      sum += cnt[e];
-      sum_inst += len[e];
+      pos[e] = (len[e] + kBucket - 1) / kBucket;
+      pos_inst[e] = len[e];
     }
-    uint32_t incl = sum, incl_inst = sum_inst;
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t u = __shfl_up(incl, o, 64);
-      const uint32_t ui = __shfl_up(incl_inst, o, 64);
-      if (lane >= o) {
-        incl += u;
-        incl_inst += ui;
-      }
+    for (int e = 0; e < kBoItems; ++e) {
+      pos[e] = wave_incl_scan(pos[e]);
+      pos_inst[e] = wave_incl_scan(pos_inst[e]);
     }
-    if (lane == kWave - 1) {
-      s_wave[wave] = incl;
-      s_wave_inst[wave] = incl_inst;
+    uint32_t sum = 0, sum_inst = 0;  // the wavefront's earlier rounds
+#pragma unroll
+    for (int e = 0; e < kBoItems; ++e) {
+      const uint32_t t = wave_last(pos[e]), ti = wave_last(pos_inst[e]);
+      pos[e] += sum - (len[e] + kBucket - 1) / kBucket;
+      pos_inst[e] += sum_inst - len[e];
+      sum += t;
+      sum_inst += ti;
+    }
+    if (lane == 0) {
+      s_wave[wave] = sum;
+      s_wave_inst[wave] = sum_inst;
     }
     __syncthreads();
-    uint32_t before = 0, total = 0, before_inst = 0, total_inst = 0;
+    uint32_t before = run, total = 0, before_inst = run_inst, total_inst = 0;
+#pragma unroll
     for (int w = 0; w < kBoThreads / kWave; ++w) {
-      const uint32_t v = s_wave[w];
-      const uint32_t vi = s_wave_inst[w];
+      const uint32_t v = s_wave[w], vi = s_wave_inst[w];
       before += w < wave ? v : 0u;
       before_inst += w < wave ? vi : 0u;
       total += v;
       total_inst += vi;
     }
     __syncthreads();
-    uint32_t pos = run + before + incl - sum;
-    uint32_t pos_inst = run_inst + before_inst + incl_inst - sum_inst;
 #pragma unroll
     for (int e = 0; e < kBoItems; ++e) {
-      const int t = c0 + static_cast<int>(threadIdx.x) * kBoItems + e;
+      const int t = base + kWave * e;
       if (t < n_tiles) {
-        boff[t] = pos;
-        if (fix_empty && m > 0 && len[e] == 0) {
-          start[e] = pos_inst;
-          ranges[2 * t] = pos_inst;
-          ranges[2 * t + 1] = pos_inst;
-        }
-        if (tile_offsets) tile_offsets[t] = start[e];
+        boff[t] = before + pos[e];
+        if (tile_offsets) tile_offsets[t] = before_inst + pos_inst[e];
+        put(t, len[e], before_inst + pos_inst[e]);
       }
-      pos += cnt[e];
-      pos_inst += len[e];
     }
     run += total;
     run_inst += total_inst;
   }
   if (threadIdx.x == 0) {
     boff[n_tiles] = run;
-    if (tile_offsets) tile_offsets[n_tiles] = static_cast<uint32_t>(m);
+    if (tile_offsets) tile_offsets[n_tiles] = run_inst;
   }
+}
+
+// Bucket offsets (and CSR tile offsets) from the tiles' ranges. Ranges come from the sort's atomic
+// min / max, so a tile without instances still holds [~0, 0]: it gets the empty range at its CSR
+// position. With m == 0 every range is written empty.
+__global__ __launch_bounds__(kBoThreads) void bucket_offsets_kernel(uint32_t* ranges, int n_tiles, int64_t m,
+                                                                    uint32_t* __restrict__ boff,
+                                                                    uint32_t* __restrict__ tile_offsets,
+                                                                    uint32_t* __restrict__ list_header) {
+  const auto count_of = [=](int t) {
+    if (m <= 0) return 0u;
+    const uint32_t lo = ranges[2 * t], hi = ranges[2 * t + 1];
+    return lo == 0xffffffffu ? 0u : hi - lo;
+  };
+  const auto put = [=](int t, uint32_t len, uint32_t at) {
+    if (len == 0u) ranges[2 * t] = ranges[2 * t + 1] = at;
+  };
+  tile_scan_block(count_of, n_tiles, put, boff, tile_offsets, list_header);
 }
 
 // Full 64-bit keys of the sorted instances (tile << 32 | depth key), for callers that want them.
@@ -1055,12 +1046,7 @@ __device__ void span_row_bases(const uint32_t* __restrict__ rowtot, int tiles_y,
     v[e] = r < tiles_y ? span_pad(rowtot[r]) : 0u;
     sum += v[e];
   }
-  uint32_t incl = sum;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t u = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += u;
-  }
+  const uint32_t incl = wave_incl_scan(sum);
   if (lane == kWave - 1) s_wsum[wave] = incl;
   __syncthreads();
   uint32_t run = incl - sum;
@@ -1364,76 +1350,6 @@ __global__ __launch_bounds__(256) void span_place_kernel(const uint2* __restrict
   }
 }
 
-// Scan of the tile counts of a canvas (one workgroup of kBoThreads threads): ranges [start,
-// end), bucket offsets (32 entries per bucket), optionally CSR tile offsets, and the bucket
-// list header cleared.
-
-__device__ void tile_scan_block(const uint32_t* __restrict__ cnt, int n_tiles, uint32_t* __restrict__ ranges,
-                                uint32_t* __restrict__ boff, uint32_t* __restrict__ tile_offsets,
-                                uint32_t* __restrict__ list_header) {
-  __shared__ uint32_t s_wave[kBoThreads / kWave];
-  __shared__ uint32_t s_wave_inst[kBoThreads / kWave];
-  if (list_header && threadIdx.x < kListHeader) list_header[threadIdx.x] = 0u;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  uint32_t run = 0, run_inst = 0;
-  for (int c0 = 0; c0 < n_tiles; c0 += kBoThreads * kBoItems) {
-    uint32_t len[kBoItems], sum = 0, sum_inst = 0;
-#pragma unroll
-    for (int e = 0; e < kBoItems; ++e) {
-      const int t = c0 + static_cast<int>(threadIdx.x) * kBoItems + e;
-      len[e] = t < n_tiles ? cnt[t] : 0u;
-      sum += (len[e] + kBucket - 1) / kBucket;
-      sum_inst += len[e];
-    }
-    uint32_t incl = sum, incl_inst = sum_inst;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t u = __shfl_up(incl, o, 64);
-      const uint32_t ui = __shfl_up(incl_inst, o, 64);
-      if (lane >= o) {
-        incl += u;
-        incl_inst += ui;
-      }
-    }
-    if (lane == kWave - 1) {
-      s_wave[wave] = incl;
-      s_wave_inst[wave] = incl_inst;
-    }
-    __syncthreads();
-    uint32_t before = 0, total = 0, before_inst = 0, total_inst = 0;
-    for (int w = 0; w < kBoThreads / kWave; ++w) {
-      const uint32_t v = s_wave[w];
-      const uint32_t vi = s_wave_inst[w];
-      before += w < wave ? v : 0u;
-      before_inst += w < wave ? vi : 0u;
-      total += v;
-      total_inst += vi;
-    }
-    __syncthreads();
-    uint32_t pos = run + before + incl - sum;
-    uint32_t pos_inst = run_inst + before_inst + incl_inst - sum_inst;
-#pragma unroll
-    for (int e = 0; e < kBoItems; ++e) {
-      const int t = c0 + static_cast<int>(threadIdx.x) * kBoItems + e;
-      if (t < n_tiles) {
-        boff[t] = pos;
-        ranges[2 * t] = pos_inst;
-        ranges[2 * t + 1] = pos_inst + len[e];
-        if (tile_offsets) tile_offsets[t] = pos_inst;
-      }
-      pos += (len[e] + kBucket - 1) / kBucket;
-      pos_inst += len[e];
-    }
-    run += total;
-    run_inst += total_inst;
-  }
-  if (threadIdx.x == 0) {
-    boff[n_tiles] = run;
-    if (tile_offsets) tile_offsets[n_tiles] = run_inst;
-  }
-}
-
 // Chunks of the column pass: chunk k (a workgroup) holds span positions [k kSpanChunk,
 // (k + 1) kSpanChunk), all in one row (wavefront w takes the w-th kWaveSpans of them); row r's
 // chunks are [cb, cb + nc) (clamped to the capacity). Chunk counts are stored chunk-major:
@@ -1613,7 +1529,112 @@ __global__ __launch_bounds__(kBoThreads) void tile_scan_kernel(const uint32_t* _
                                                               uint32_t* __restrict__ boff,
                                                               uint32_t* __restrict__ tile_offsets,
                                                               uint32_t* __restrict__ list_header) {
-  tile_scan_block(tcnt, n_tiles, ranges, boff, tile_offsets, list_header);
+  const auto put = [=](int t, uint32_t len, uint32_t at) {
+    ranges[2 * t] = at;
+    ranges[2 * t + 1] = at + len;
+  };
+  tile_scan_block([=](int t) { return tcnt[t]; }, n_tiles,
+                  put, boff, tile_offsets,
+                  list_header);
+}
+
+// Tile counts of a rectangle binning from the rectangles alone: a rectangle adds +1 / -1 at its four
+// corners of a (tiles_x + 1) x (tiles_y + 1) array (clamped to the grid), whose two-dimensional
+// prefix sum is the count of every tile. With the counts the ranges, the bucket offsets and both
+// totals are known before the instances are sorted, so the host waits once, for these small
+// kernels, instead of twice, the second time for the whole sort (and the sort takes no ranges).
+// rect_diff_kernel: G workgroups each leave their rectangles' array in part[g]; rect_tiles_kernel
+// (one workgroup) sums them (G = 0: takes all rectangles itself), scans and stores the totals to
+// host memory.
+constexpr int kDiffThreads = 1024;
+constexpr int64_t kDiffMax = 16000;       // array entries (below 64 KB of LDS): canvases up to 2000 x 2000
+constexpr int64_t kDiffDirect = 8192;     // rectangles one workgroup takes alone
+constexpr int64_t kDiffPer = 16384;       // rectangles per workgroup beyond
+constexpr int kDiffGroups = 8;
+
+__device__ __forceinline__ void rect_diff_add(const int4* __restrict__ rects, int64_t lo, int64_t hi, int tiles_x,
+                                              int tiles_y, int* s_d) {
+  const int w = tiles_x + 1, n_d = w * (tiles_y + 1);
+  for (int q = threadIdx.x; q < n_d; q += kDiffThreads) s_d[q] = 0;
+  __syncthreads();
+  for (int64_t i = lo + threadIdx.x; i < hi; i += kDiffThreads) {
+    const int4 r = clamp_rect(rects[i], tiles_x, tiles_y);
+    if (r.z > r.x && r.w > r.y) {
+      atomicAdd(&s_d[r.y * w + r.x], 1);
+      atomicAdd(&s_d[r.y * w + r.z], -1);
+      atomicAdd(&s_d[r.w * w + r.x], -1);
+      atomicAdd(&s_d[r.w * w + r.z], 1);
+    }
+  }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(kDiffThreads) void rect_diff_kernel(const int4* __restrict__ rects, int64_t n, int tiles_x,
+                                                                 int tiles_y, int* __restrict__ part) {
+  extern __shared__ __align__(16) int s_diff[];
+  const int64_t per = (n + gridDim.x - 1) / gridDim.x, lo = per * blockIdx.x, hi = min(lo + per, n);
+  rect_diff_add(rects, lo, hi, tiles_x, tiles_y, s_diff);
+  const int n_d = (tiles_x + 1) * (tiles_y + 1);
+  for (int q = threadIdx.x; q < n_d; q += kDiffThreads) part[static_cast<int64_t>(blockIdx.x) * n_d + q] = s_diff[q];
+}
+
+__global__ __launch_bounds__(kDiffThreads) void rect_tiles_kernel(
+    const int4* __restrict__ rects, int64_t n, const int* __restrict__ part, int G, int tiles_x, int tiles_y,
+    uint32_t* __restrict__ ranges, uint32_t* __restrict__ boff,
+    uint32_t* __restrict__ tile_offsets, unsigned long long* __restrict__ host) {
+  extern __shared__ __align__(16) int s_diff[];
+  __shared__ unsigned long long s_m[kDiffThreads / kWave];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int w = tiles_x + 1, n_d = w * (tiles_y + 1);
+  if (G == 0) {
+    rect_diff_add(rects, 0, n, tiles_x, tiles_y, s_diff);
+  } else {
+    for (int q = tid; q < n_d; q += kDiffThreads) {
+      int v[kDiffGroups], sum = 0;  // (all loads in flight together)
+#pragma unroll
+      for (int g = 0; g < kDiffGroups; ++g) v[g] = g < G ? part[static_cast<int64_t>(g) * n_d + q] : 0;
+#pragma unroll
+      for (int g = 0; g < kDiffGroups; ++g) sum += v[g];
+      s_diff[q] = sum;
+    }
+    __syncthreads();
+  }
+  // along the rows, then down the columns: a wavefront per line
+  const auto scan_line = [&](int len, int first, int stride) {
+    unsigned long long sum = 0;
+    uint32_t carry = 0;
+    for (int c0 = 0; c0 < len; c0 += kWave) {
+      const int c = c0 + lane;
+      const uint32_t v = c < len ? static_cast<uint32_t>(s_diff[first + c * stride]) : 0u;
+      uint32_t total;
+      const uint32_t got = carry + wave_excl_scan(v, lane, total) + v;
+      if (c < len) {
+        s_diff[first + c * stride] = static_cast<int>(got);
+        sum += got;
+      }
+      carry += total;
+    }
+    return sum;
+  };
+  unsigned long long m = 0;
+  for (int y = wave; y < tiles_y; y += kDiffThreads / kWave) scan_line(tiles_x, y * w, 1);
+  __syncthreads();
+  for (int c = wave; c < tiles_x; c += kDiffThreads / kWave) m += scan_line(tiles_y, c, w);
+  for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off, 64);
+  if (lane == 0) s_m[wave] = m;
+  __syncthreads();
+  const auto put = [=](int t, uint32_t len, uint32_t at) {
+    ranges[2 * t] = at;
+    ranges[2 * t + 1] = at + len;
+  };
+  tile_scan_block([=](int t) { return static_cast<uint32_t>(s_diff[t / tiles_x * w + t % tiles_x]); }, tiles_x * tiles_y,
+                  put, boff, tile_offsets,
+                  nullptr);
+  if (tid == 0) {
+    for (int q = 1; q < kDiffThreads / kWave; ++q) m += s_m[q];
+    host[0] = m;
+    host[1] = boff[tiles_x * tiles_y];  // (written by this thread)
+  }
 }
 
 // Column pass, placement: workgroup per chunk, each wavefront places the instances of its
@@ -1728,12 +1749,7 @@ __global__ __launch_bounds__(256) void span_col_write_kernel(
 #pragma unroll
           for (int b = 0; b < 4; ++b) run = max(run, (w[q] >> (8 * b)) & 0xffu);
         // the largest marker of the lanes before this one (a wavefront max-scan), and the seed
-        uint32_t incl = run;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-          const uint32_t u = __shfl_up(incl, o, 64);
-          if (lane >= o) incl = max(incl, u);
-        }
+        const uint32_t incl = wave_scan(run, 0u, [](uint32_t x, uint32_t y) { return max(x, y); });
         uint32_t m = max(carry, __shfl_up(incl, 1, 64));
         if (lane == 0) m = carry;
 #pragma unroll
@@ -2017,7 +2033,7 @@ static void emit_and_sort(const SplatRec* rec, const int4* rects, const uint32_t
   }
   stage_mark("key_duplication", st);
   radix_sort(tkeys, tvals, tsorted, point_list, m, tile_bits, ws + L.sort, st, nullptr, nullptr, preset,
-             preset != nullptr && !sorted_keys);
+             tile_bits > 0 && !sorted_keys);
   stage_mark("tile_sort", st);
   if (sorted_keys)
     hipLaunchKernelGGL((full_keys_kernel<K>), dim3(grid_for(m, 256)), dim3(256), 0, st, tsorted, point_list, dkey_of,
@@ -2110,25 +2126,31 @@ static void bin_emit(const SplatRec* rec, const int4* rects, const uint32_t* dke
     // with at least one sort pass, the last pass takes the tile ranges (preset by the emission)
     // and the sorted keys are written only if the caller wants them; tile ids below 2^16 are
     // emitted and sorted as 16-bit keys
-    const bool sort_ranges = tile_bits > 0;
+    const bool known = (flags & GS_BIN_TILES_KNOWN) != 0;  // ranges and offsets are written already
+    const bool sort_ranges = tile_bits > 0 && !known;
     uint32_t* preset = sort_ranges ? ranges : nullptr;
-    const bool short_keys = sort_ranges && n_tiles <= 65536;
+    const bool short_keys = tile_bits > 0 && n_tiles <= 65536;
     if (short_keys)
       emit_and_sort<uint16_t>(rec, rects, dkey_of, dkey0, order, offsets, n, tiles_x, n_tiles, m, tile_bits,
                               sorted_keys, point_list, preset, L, ws, st);
     else
       emit_and_sort<uint32_t>(rec, rects, dkey_of, dkey0, order, offsets, n, tiles_x, n_tiles, m, tile_bits,
                               sorted_keys, point_list, preset, L, ws, st);
+    if (known) {
+      stage_mark("ranges_buckets", st);
+      return;
+    }
     if (!sort_ranges)
       hipLaunchKernelGGL(tile_bounds_kernel, dim3(grid_for((m + kBoundsPer - 1) / kBoundsPer, 256)), dim3(256), 0,
                          st, reinterpret_cast<const uint32_t*>(ws + L.tsorted), m, n_tiles, ranges);
     hipLaunchKernelGGL(bucket_offsets_kernel, dim3(1), dim3(kBoThreads), 0, st, ranges, n_tiles, m, bucket_offsets,
-                       tile_offsets, list_header, sort_ranges);
+                       tile_offsets, list_header);
     stage_mark("ranges_buckets", st);
     return;
   }
+  if (flags & GS_BIN_TILES_KNOWN) return;
   hipLaunchKernelGGL(bucket_offsets_kernel, dim3(1), dim3(kBoThreads), 0, st, ranges, n_tiles, m, bucket_offsets,
-                     tile_offsets, list_header, false);
+                     tile_offsets, list_header);
 }
 
 }  // namespace gs
@@ -2167,17 +2189,16 @@ namespace gs {
 struct CountSide {
   hipStream_t side = nullptr;
   hipEvent_t after = nullptr, done = nullptr;
-  unsigned long long* host_word = nullptr;  // pinned, coherent: the sum kernel stores to it directly
+  unsigned long long* host_word = nullptr;  // two words, pinned, coherent: the kernels store to them directly
   bool pending = false;
 };
 constexpr int kCountMaxDevices = 64;
 static thread_local CountSide g_count[kCountMaxDevices];
 }  // namespace gs
 
-extern "C" int gs_count_begin(const uint32_t* wave_counts, int64_t n_waves, int on_side_stream, void* stream) {
-  clear_error();
-  GS_REQUIRE(n_waves >= 0 && (n_waves == 0 || wave_counts), GS_ERR_ARG, "invalid count arguments");
-  GS_REQUIRE(aligned(wave_counts, 4), GS_ERR_ALIGN, "wave_counts must be 4-byte aligned");
+namespace gs {
+// This thread and device's resources, ready for a new count (*out), or an error.
+static int count_side(CountSide** out) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return check_launch("count_begin (device)");
   GS_REQUIRE(dev >= 0 && dev < kCountMaxDevices, GS_ERR_ARG, "device index %d out of range", dev);
@@ -2187,31 +2208,18 @@ extern "C" int gs_count_begin(const uint32_t* wave_counts, int64_t n_waves, int 
     if (hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&c.after, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c.done, hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&c.host_word), sizeof(unsigned long long), hipHostMallocCoherent) !=
+        hipHostMalloc(reinterpret_cast<void**>(&c.host_word), 2 * sizeof(unsigned long long), hipHostMallocCoherent) !=
             hipSuccess) {
       const int e = check_launch("count_begin (set-up)");
       c = CountSide{};  // (a partial set-up is retried on the next call; its pieces leak)
       return e ? e : GS_ERR_LAUNCH;
     }
   }
-  hipStream_t st = as_stream(stream);
-  hipStream_t run = st;
-  if (on_side_stream) {
-    if (hipEventRecord(c.after, st) != hipSuccess || hipStreamWaitEvent(c.side, c.after, 0) != hipSuccess)
-      return check_launch("count_begin (event)");
-    run = c.side;
-  }
-  // one thread stores the total straight into the pinned word: no copy to enqueue
-  hipLaunchKernelGGL(sum_u32_kernel, dim3(1), dim3(kSumThreads), 0, run, wave_counts, n_waves, c.host_word);
-  if (int e = check_launch("count_begin (sum)")) return e;
-  if (hipEventRecord(c.done, run) != hipSuccess) return check_launch("count_begin (event)");
-  c.pending = true;
+  *out = &c;
   return GS_OK;
 }
 
-extern "C" int gs_count_end(uint64_t* m) {
-  clear_error();
-  GS_REQUIRE(m, GS_ERR_ARG, "null pointer argument");
+static int count_wait(uint64_t* m, uint64_t* second) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return check_launch("count_end (device)");
   GS_REQUIRE(dev >= 0 && dev < kCountMaxDevices && g_count[dev].pending, GS_ERR_ARG,
@@ -2219,8 +2227,82 @@ extern "C" int gs_count_end(uint64_t* m) {
   CountSide& c = g_count[dev];
   c.pending = false;
   if (hipEventSynchronize(c.done) != hipSuccess) return check_launch("count_end");
-  *m = *c.host_word;
+  *m = c.host_word[0];
+  if (second) *second = c.host_word[1];
   return GS_OK;
+}
+}  // namespace gs
+
+extern "C" int gs_count_begin(const uint32_t* wave_counts, int64_t n_waves, int on_side_stream, void* stream) {
+  clear_error();
+  GS_REQUIRE(n_waves >= 0 && (n_waves == 0 || wave_counts), GS_ERR_ARG, "invalid count arguments");
+  GS_REQUIRE(aligned(wave_counts, 4), GS_ERR_ALIGN, "wave_counts must be 4-byte aligned");
+  CountSide* c = nullptr;
+  if (int e = count_side(&c)) return e;
+  hipStream_t st = as_stream(stream);
+  hipStream_t run = st;
+  if (on_side_stream) {
+    if (hipEventRecord(c->after, st) != hipSuccess || hipStreamWaitEvent(c->side, c->after, 0) != hipSuccess)
+      return check_launch("count_begin (event)");
+    run = c->side;
+  }
+  // one thread stores the total straight into the pinned word: no copy to enqueue
+  hipLaunchKernelGGL(sum_u32_kernel, dim3(1), dim3(kSumThreads), 0, run, wave_counts, n_waves, c->host_word);
+  if (int e = check_launch("count_begin (sum)")) return e;
+  if (hipEventRecord(c->done, run) != hipSuccess) return check_launch("count_begin (event)");
+  c->pending = true;
+  return GS_OK;
+}
+
+extern "C" int gs_count_end(uint64_t* m) {
+  clear_error();
+  GS_REQUIRE(m, GS_ERR_ARG, "null pointer argument");
+  return count_wait(m, nullptr);
+}
+
+extern "C" int gs_rect_tiles_fit(int tiles_x, int tiles_y) {
+  return tiles_x > 0 && tiles_y > 0 && (static_cast<int64_t>(tiles_x) + 1) * (tiles_y + 1) <= kDiffMax;
+}
+
+extern "C" size_t gs_rect_tiles_workspace_size(int64_t n, int tiles_x, int tiles_y) {
+  if (!gs_rect_tiles_fit(tiles_x, tiles_y)) return 0;
+  return n > kDiffDirect ? align_up(static_cast<size_t>(kDiffGroups) * (tiles_x + 1) * (tiles_y + 1) * 4) : 0;
+}
+
+extern "C" int gs_rect_tiles_begin(const int32_t* rects, int64_t n, int tiles_x, int tiles_y, uint32_t* ranges,
+                                   uint32_t* tile_offsets, uint32_t* bucket_offsets, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
+  clear_error();
+  GS_REQUIRE(n >= 0 && gs_rect_tiles_fit(tiles_x, tiles_y), GS_ERR_ARG, "invalid rect_tiles sizes (n=%lld, %d x %d)",
+             static_cast<long long>(n), tiles_x, tiles_y);
+  GS_REQUIRE((rects || n == 0) && ranges && bucket_offsets, GS_ERR_ARG, "null pointer argument");
+  GS_REQUIRE(aligned(rects, 16), GS_ERR_ALIGN, "rects must be 16-byte aligned");
+  const size_t need = gs_rect_tiles_workspace_size(n, tiles_x, tiles_y);
+  GS_REQUIRE(workspace_bytes >= need && (workspace || !need), GS_ERR_WORKSPACE, "rect_tiles workspace too small: need %zu bytes",
+             need);
+  CountSide* c = nullptr;
+  if (int e = count_side(&c)) return e;
+  hipStream_t st = as_stream(stream);
+  int* part = static_cast<int*>(workspace);
+  const int4* r4 = reinterpret_cast<const int4*>(rects);
+  const size_t lds = static_cast<size_t>(tiles_x + 1) * (tiles_y + 1) * 4;
+  int G = 0;
+  if (n > kDiffDirect) {
+    G = static_cast<int>(std::min<int64_t>((n + kDiffPer - 1) / kDiffPer, kDiffGroups));
+    hipLaunchKernelGGL(rect_diff_kernel, dim3(G), dim3(kDiffThreads), lds, st, r4, n, tiles_x, tiles_y, part);
+  }
+  hipLaunchKernelGGL(rect_tiles_kernel, dim3(1), dim3(kDiffThreads), lds, st, r4, n, part, G, tiles_x, tiles_y,
+                     ranges, bucket_offsets, tile_offsets, c->host_word);
+  if (int e = check_launch("rect_tiles_begin")) return e;
+  if (hipEventRecord(c->done, st) != hipSuccess) return check_launch("rect_tiles_begin (event)");
+  c->pending = true;
+  return GS_OK;
+}
+
+extern "C" int gs_rect_tiles_end(uint64_t* m, uint64_t* n_buckets) {
+  clear_error();
+  GS_REQUIRE(m && n_buckets, GS_ERR_ARG, "null pointer argument");
+  return count_wait(m, n_buckets);
 }
 
 extern "C" size_t gs_bin_prepare_workspace_size(int64_t n) { return prep_ws(n < 0 ? 0 : n); }

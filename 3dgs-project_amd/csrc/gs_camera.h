@@ -116,12 +116,8 @@ __device__ __forceinline__ uint32_t wave_count_rows(bool vis, const float4 a, co
     s_set[3 * lane + 2] = make_float4(__int_as_float(d.x), __int_as_float(d.y), __int_as_float(d.z),
                                       __int_as_float(d.w));
   }
-  uint32_t incl = rows;
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t u = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += u;
-  }
-  const uint32_t total = __shfl(incl, kWave - 1, 64);
+  const uint32_t incl = wave_incl_scan(rows);
+  const uint32_t total = wave_last(incl);
   s_rex[lane] = incl - rows;
   s_cnt[lane] = 0u;
   wave_sync();

@@ -74,6 +74,31 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Inclusive scan of f over the wavefront's lanes in lane order (every lane active; `id` is f's
+// identity): row shifts within the rows of 16, then the rows' last lanes broadcast to the rows after
+// them. Six DPP instructions on the VALU; the shuffles they replace go through the LDS unit
+// (ds_bpermute), whose throughput 16 wavefronts of a scanning workgroup share.
+template <typename F>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, uint32_t id, F f) {
+#define GS_DPP(CTRL, ROWS) \
+  v = f(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(id), static_cast<int>(v), CTRL, ROWS, 0xf, false)))
+  GS_DPP(0x111, 0xf);  // row_shr:1
+  GS_DPP(0x112, 0xf);  // row_shr:2
+  GS_DPP(0x114, 0xf);  // row_shr:4
+  GS_DPP(0x118, 0xf);  // row_shr:8
+  GS_DPP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  GS_DPP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef GS_DPP
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+  return wave_scan(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+// The last lane's value (of a scan: the total), in every lane.
+__device__ __forceinline__ uint32_t wave_last(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), kWave - 1));
+}
+
 // Logical index of workgroup b of n. Workgroups are dealt to the 8 XCDs round-robin
 // (b % 8); giving XCD x the contiguous logical range x * (n / 8) ... (a bijection for any n)
 // keeps neighbouring radix tiles -- whose runs of one digit are adjacent in the output, often

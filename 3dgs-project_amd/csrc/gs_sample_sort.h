@@ -265,8 +265,8 @@ __global__ __launch_bounds__(kSsThreads) void ss_scatter_kernel(
 
 // Fold of v over the workgroup of NT threads by f, to every thread.
 template <int NT, typename F>
-__device__ __forceinline__ uint32_t block_fold(uint32_t v, uint32_t* s_w, F f) {
-  for (int off = 32; off > 0; off >>= 1) v = f(v, static_cast<uint32_t>(__shfl_xor(v, off, 64)));
+__device__ __forceinline__ uint32_t block_fold(uint32_t v, uint32_t* s_w, F f) {  // (0 is f's identity)
+  v = wave_last(wave_scan(v, 0u, f));
   __syncthreads();
   if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -278,10 +278,8 @@ __device__ __forceinline__ uint32_t block_fold(uint32_t v, uint32_t* s_w, F f) {
 // Minimum of lo and maximum of hi over the workgroup, to every thread.
 template <int NT>
 __device__ __forceinline__ void block_min_max(uint32_t& lo, uint32_t& hi, uint32_t* s_w, uint32_t* s_w2) {
-  for (int off = 32; off > 0; off >>= 1) {
-    lo = min(lo, static_cast<uint32_t>(__shfl_xor(lo, off, 64)));
-    hi = max(hi, static_cast<uint32_t>(__shfl_xor(hi, off, 64)));
-  }
+  lo = wave_last(wave_scan(lo, ~0u, [](uint32_t x, uint32_t y) { return min(x, y); }));
+  hi = wave_last(wave_scan(hi, 0u, [](uint32_t x, uint32_t y) { return max(x, y); }));
   __syncthreads();
   if ((threadIdx.x & 63) == 0) {
     s_w[threadIdx.x >> 6] = lo;
@@ -298,12 +296,7 @@ __device__ __forceinline__ void block_min_max(uint32_t& lo, uint32_t& hi, uint32
 template <int NT>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_w, uint32_t& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t incl = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t u = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += u;
-  }
+  const uint32_t incl = wave_incl_scan(v);
   __syncthreads();
   if (lane == 63) s_w[wave] = incl;
   __syncthreads();

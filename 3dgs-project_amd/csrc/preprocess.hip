@@ -532,8 +532,7 @@ __global__ __launch_bounds__(256) void preprocess_fwd_kernel(
   }
   if (wave_counts) {
     // tiles touched by this wavefront's 64 Gaussians: the instance count m is their total
-    uint32_t s = (valid && g.vis) ? count : 0u;
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    const uint32_t s = wave_last(wave_incl_scan((valid && g.vis) ? count : 0u));
     if (lane == 0) wave_counts[wave_first / 64] = s;
   }
 }

@@ -68,6 +68,9 @@ typedef struct gs_camera {
  * the same lists, ranges and bucket offsets. */
 #define GS_BIN_SPANS 2
 #define GS_BIN_RADIX 4
+/* gs_bin_fill_rect only: gs_rect_tiles_begin wrote ranges, bucket_offsets (and tile_offsets) for
+ * these rectangles already; the fill leaves them as they are. */
+#define GS_BIN_TILES_KNOWN 8
 #define GS_BIN_SPAN_MIN_GAUSSIANS 2000000
 /* gs_bin_path values: the 3D fill's path for a camera and Gaussian count */
 enum { GS_BIN_PATH_RADIX = 0, GS_BIN_PATH_SPANS = 1 };
@@ -207,6 +210,19 @@ int gs_bin_fill_rect(const int32_t* rects, const void* depth, int depth_dtype, c
                      uint32_t* point_list, uint32_t* ranges, uint32_t* tile_offsets,
                      uint32_t* bucket_offsets, uint32_t* order, int flags, void* workspace,
                      size_t workspace_bytes, void* stream);
+
+/* The tile ranges, bucket offsets and (may be NULL) tile offsets of a rectangle binning from its
+ * rectangles alone, before any instance is emitted, and the totals read back to the host as
+ * gs_count_begin reads its count: gs_rect_tiles_begin enqueues the kernels, gs_rect_tiles_end (same
+ * thread and device) waits for them and returns the instance count and the bucket count. The fill
+ * then takes GS_BIN_TILES_KNOWN. For canvases with (tiles_x + 1)(tiles_y + 1) <= 16000
+ * (gs_rect_tiles_fit). Workspace from gs_rect_tiles_workspace_size. */
+int gs_rect_tiles_fit(int tiles_x, int tiles_y);
+size_t gs_rect_tiles_workspace_size(int64_t n, int tiles_x, int tiles_y);
+int gs_rect_tiles_begin(const int32_t* rects, int64_t n, int tiles_x, int tiles_y, uint32_t* ranges,
+                        uint32_t* tile_offsets, uint32_t* bucket_offsets, void* workspace,
+                        size_t workspace_bytes, void* stream);
+int gs_rect_tiles_end(uint64_t* m, uint64_t* n_buckets);
 
 /* bucket_to_tile[b] = tile of bucket b, for b < bucket_offsets[n_tiles] (read on device);
  * entries up to n_buckets_max are written, unused ones with 0xffffffff. */
