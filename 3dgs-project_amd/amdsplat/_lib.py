@@ -117,6 +117,7 @@ _SIGS = {
     "gs_densification_stats": (_i32, [_vp, _vp, _i64, _i32, _i32, _i32, _vp, _vp]),
     "gs_l1_ssim_workspace_size": (_sz, [_i32, _i32, _i32]),
     "gs_l1_ssim_fwd": (_i32, [_vp, _vp, _i32, _i32, _i32, C.c_float, _vp, _vp, _vp, _sz, _vp]),
+    "gs_l1_ssim_fwd_value": (_i32, [_vp, _vp, _i32, _i32, _i32, C.c_float, _vp, _vp, _vp, _vp, _sz, _vp]),
     "gs_l1_ssim_bwd": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, C.c_float, _vp, _vp, _vp]),
     "gs_l1_ssim_fwd_noalloc": (_i32, [_vp, _vp, _i32, _i32, _i32, C.c_float, _vp, _vp, _vp]),
     "gs_stage_marks": (_i32, [_i32]),

@@ -36,14 +36,15 @@ class _L1Ssim(torch.autograd.Function):
         dev = x.device
         dmap = torch.empty(C, 3, H, W, dtype=torch.float32, device=dev) if ctx.needs_input_grad[0] else None
         loss = torch.empty(3, dtype=torch.float32, device=dev)
+        value = torch.empty((), dtype=torch.float32, device=dev)
         ws = torch.empty(max(_lib.size_call("gs_l1_ssim_workspace_size", C, H, W), 1), dtype=torch.uint8, device=dev)
-        call("gs_l1_ssim_fwd", ptr(x), ptr(y), C, H, W, float(lambda_dssim), ptr(dmap), ptr(loss), ptr(ws),
-             ws.numel(), _lib.stream_handle(dev))
+        call("gs_l1_ssim_fwd_value", ptr(x), ptr(y), C, H, W, float(lambda_dssim), ptr(dmap), loss.data_ptr(),
+             value.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_handle(dev))
         ctx.save_for_backward(x, y, dmap)
         ctx.lam = float(lambda_dssim)
         ctx.in_shape = image.shape
         ctx.mark_non_differentiable(loss)
-        return loss[0].clone(), loss
+        return value, loss
 
     @staticmethod
     def backward(ctx, grad_out, _grad_parts):
@@ -52,7 +53,9 @@ class _L1Ssim(torch.autograd.Function):
             return None, None, None
         C, H, W = x.shape
         g = torch.empty_like(x)
-        go = grad_out.detach().to(torch.float32).contiguous().reshape(1)
+        go = grad_out.detach()
+        if go.dtype != torch.float32:
+            go = go.to(torch.float32)
         call("gs_l1_ssim_bwd", ptr(x), ptr(y), ptr(dmap), C, H, W, ctx.lam, ptr(go), ptr(g),
              _lib.stream_handle(x.device))
         return g.reshape(ctx.in_shape), None, None

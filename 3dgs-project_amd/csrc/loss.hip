@@ -7,7 +7,8 @@
 // fusedssim_backwardCUDA, results/phase1/README.md:46-47).
 //
 // One workgroup per 32x32 tile and channel. Forward: the tile plus a 5-pixel halo of both
-// images goes to LDS, the five moments (x, y, x^2, y^2, xy) are filtered separably (rows, then
+// images goes to LDS, the four moments that S depends on (x, y, x^2 + y^2, xy: the variances enter
+// only as their sum) are filtered separably (rows, then
 // columns; in each pass a thread computes four adjacent outputs from the 14 inputs they share,
 // so every input is read and squared once), and each pixel writes the three partial derivatives
 // of its SSIM value the backward needs (dS/dmu_x, dS/dE[x^2], dS/dE[xy]) plus per-workgroup
@@ -36,11 +37,13 @@ constexpr int kSsLimitTile = 16;                  // tile side of the allocation
 constexpr float kSsC1 = 0.01f * 0.01f;
 constexpr float kSsC2 = 0.03f * 0.03f;
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-// Forward LDS (floats): the five row-filtered planes, with the x and y patches placed after the
-// first three, so that only planes 3 and 4 share memory with the patches.
-constexpr int kSsFwdHold = 3;  // first plane held in registers over the row pass's barrier
+// Forward LDS (floats): the four row-filtered planes, with the x and y patches placed after the
+// first two, so that only planes 2 and 3 share memory with the patches. VALU and LDS bound: with
+// x^2 and y^2 as planes of their own (five) the 3 x 840 x 1297 frame took 34.5 us, so 27.9.
+constexpr int kSsMoments = 4;
+constexpr int kSsFwdHold = 2;  // first plane held in registers over the row pass's barrier
 constexpr int kSsFwdXy = kSsFwdHold * kSsIn * kSsHS;
-constexpr int kSsFwdLds = cmax(kSsFwdXy + 2 * kSsIn * kSsInS, 5 * kSsIn * kSsHS);
+constexpr int kSsFwdLds = cmax(kSsFwdXy + 2 * kSsIn * kSsInS, kSsMoments * kSsIn * kSsHS);
 // Backward: the three patches, then (same memory, every plane held) their row-filtered planes.
 constexpr int kSsBwdLds = cmax(3 * kSsIn * kSsInS, 3 * kSsIn * kSsHS);
 static_assert(kSsGroups * kSsTile == kSsThreads, "column pass: one thread per (column, row group)");
@@ -94,64 +97,67 @@ __device__ __forceinline__ void load_patches(const float* const (&src)[NP], int 
   }
 }
 
+// The kSsTaps-tap symmetric filter at out[q], q < kSsQ, from in[q .. q + kSsTaps - 1]: the two
+// inputs of a weight are added first and the small weights come first, so 1.4 roundings of the
+// result's size are made where a chain over the taps in order makes 2.3, for the same operations.
+__device__ __forceinline__ void filter4(const float (&in)[kSsSpan], const SsimWeights& G, float (&out)[kSsQ]) {
+#pragma unroll
+  for (int q = 0; q < kSsQ; ++q) {
+    float a = G.w[0] * (in[q] + in[q + kSsTaps - 1]);
+#pragma unroll
+    for (int t = 1; t < kSsHalo; ++t) a = fmaf(G.w[t], in[q + t] + in[q + kSsTaps - 1 - t], a);
+    out[q] = fmaf(G.w[kSsHalo], in[q + kSsHalo], a);
+  }
+}
+
 // Row pass of NP planes of a patch: item (r, g) filters patch row r (0 .. kSsIn-1) at the kSsQ
 // output columns kSsQ g .. kSsQ g + 3 from the kSsSpan inputs starting there (read as float4s).
-// Every input is read once; with kMoments (NP = 2: x and y) the five moments x, y, x^2, y^2, xy
-// are filtered and their products formed once per input. Output planes: [NO][kSsIn][kSsHS]. The
+// Every input is read once; with kMoments (NP = 2: x and y) the moments x, y, x^2 + y^2, xy are
+// filtered and their products formed once per input. Output planes: [NO][kSsIn][kSsHS]. The
 // planes from kHold on may share memory with the patch: they are kept in registers until the
 // workgroup has synchronised, then stored; planes below kHold are stored as each item ends. The
 // caller synchronises before reading any plane.
 template <int NP, bool kMoments, int kHold>
 __device__ __forceinline__ void row_pass(const float* s_in, float* s_h, const SsimWeights& G) {
-  constexpr int NO = kMoments ? 5 : NP;
+  constexpr int NO = kMoments ? kSsMoments : NP;
   constexpr int kItems = kSsIn * kSsGroups;
   constexpr int kRounds = (kItems + kSsThreads - 1) / kSsThreads;
-  float acc[kRounds][kSsQ][NO];
+  constexpr int kHeld = NO - kHold;
+  float held[kRounds][kHeld][kSsQ];
 #pragma unroll
   for (int rd = 0; rd < kRounds; ++rd) {
     const int it = static_cast<int>(threadIdx.x) + rd * kSsThreads;
     if (it >= kItems) continue;
     const int r = it / kSsGroups, g = it - r * kSsGroups;
+    float v[NP][4 * ((kSsSpan + 3) / 4)];
 #pragma unroll
-    for (int i4 = 0; i4 < (kSsSpan + 3) / 4; ++i4) {
-      float v[NP][4];
+    for (int p = 0; p < NP; ++p)
 #pragma unroll
-      for (int p = 0; p < NP; ++p) {
+      for (int i4 = 0; i4 < (kSsSpan + 3) / 4; ++i4) {
         const float4 f = *reinterpret_cast<const float4*>(s_in + (p * kSsIn + r) * kSsInS + kSsQ * g + 4 * i4);
-        v[p][0] = f.x;
-        v[p][1] = f.y;
-        v[p][2] = f.z;
-        v[p][3] = f.w;
+        v[p][4 * i4] = f.x;
+        v[p][4 * i4 + 1] = f.y;
+        v[p][4 * i4 + 2] = f.z;
+        v[p][4 * i4 + 3] = f.w;
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * i4 + e;  // input column kSsQ g + i
-        if (i >= kSsSpan) continue;
-        float m[NO];
-        if constexpr (kMoments) {
-          m[0] = v[0][e];
-          m[1] = v[1][e];
-          m[2] = v[0][e] * v[0][e];
-          m[3] = v[1][e] * v[1][e];
-          m[4] = v[0][e] * v[1][e];
-        } else {
+    for (int o = 0; o < NO; ++o) {
+      float in[kSsSpan], out[kSsQ];
 #pragma unroll
-          for (int p = 0; p < NP; ++p) m[p] = v[p][e];
-        }
+      for (int i = 0; i < kSsSpan; ++i) {
+        if (!kMoments || o < 2) in[i] = v[o < NP ? o : 0][i];
+        else if (o == 2) in[i] = v[0][i] * v[0][i] + v[1][i] * v[1][i];
+        else in[i] = v[0][i] * v[1][i];
+      }
+      filter4(in, G, out);
+      if (o < kHold) {
+        *reinterpret_cast<float4*>(s_h + (o * kSsIn + r) * kSsHS + kSsQ * g) =
+            make_float4(out[0], out[1], out[2], out[3]);
+      } else {
 #pragma unroll
-        for (int q = 0; q < kSsQ; ++q) {
-          const int t = i - q;  // tap of output column kSsQ g + q (taps in increasing order)
-          if (t < 0 || t >= kSsTaps) continue;
-#pragma unroll
-          for (int o = 0; o < NO; ++o)
-            acc[rd][q][o] = t == 0 ? G.w[0] * m[o] : fmaf(G.w[t], m[o], acc[rd][q][o]);
-        }
+        for (int q = 0; q < kSsQ; ++q) held[rd][o < kHold ? 0 : o - kHold][q] = out[q];
       }
     }
-#pragma unroll
-    for (int o = 0; o < kHold; ++o)
-      *reinterpret_cast<float4*>(s_h + (o * kSsIn + r) * kSsHS + kSsQ * g) =
-          make_float4(acc[rd][0][o], acc[rd][1][o], acc[rd][2][o], acc[rd][3][o]);
   }
   __syncthreads();  // the patch is read: its memory may now take the held planes
 #pragma unroll
@@ -162,7 +168,7 @@ __device__ __forceinline__ void row_pass(const float* s_in, float* s_h, const Ss
 #pragma unroll
     for (int o = kHold; o < NO; ++o)
       *reinterpret_cast<float4*>(s_h + (o * kSsIn + r) * kSsHS + kSsQ * g) =
-          make_float4(acc[rd][0][o], acc[rd][1][o], acc[rd][2][o], acc[rd][3][o]);
+          make_float4(held[rd][o - kHold][0], held[rd][o - kHold][1], held[rd][o - kHold][2], held[rd][o - kHold][3]);
   }
 }
 
@@ -172,17 +178,13 @@ template <int NO>
 __device__ __forceinline__ void col_pass(const float* __restrict__ s_h, int c, int g, const SsimWeights& G,
                                          float (&acc)[kSsQ][NO]) {
 #pragma unroll
-  for (int i = 0; i < kSsSpan; ++i) {
-    float h[NO];
+  for (int o = 0; o < NO; ++o) {
+    float in[kSsSpan], out[kSsQ];
 #pragma unroll
-    for (int o = 0; o < NO; ++o) h[o] = s_h[(o * kSsIn + kSsQ * g + i) * kSsHS + c];
+    for (int i = 0; i < kSsSpan; ++i) in[i] = s_h[(o * kSsIn + kSsQ * g + i) * kSsHS + c];
+    filter4(in, G, out);
 #pragma unroll
-    for (int q = 0; q < kSsQ; ++q) {
-      const int t = i - q;
-      if (t < 0 || t >= kSsTaps) continue;
-#pragma unroll
-      for (int o = 0; o < NO; ++o) acc[q][o] = t == 0 ? G.w[0] * h[o] : fmaf(G.w[t], h[o], acc[q][o]);
-    }
+    for (int q = 0; q < kSsQ; ++q) acc[q][o] = out[q];
   }
 }
 
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(kSsThreads) void ssim_fwd_kernel(const float* __res
                                                               const float* __restrict__ gt, int H, int W,
                                                               SsimWeights G, float* __restrict__ dmap,
                                                               float* __restrict__ partials) {
-  // row-filtered x, y, xx, yy, xy; the x and y patches from plane kSsFwdHold on
+  // row-filtered x, y, xx + yy, xy; the x and y patches from plane kSsFwdHold on
   __shared__ __align__(16) float s_buf[kSsFwdLds];
   __shared__ float s_red[2][4];
   const SsTile tl = ss_tile((W + kSsTile - 1) / kSsTile, (H + kSsTile - 1) / kSsTile);
@@ -231,8 +233,8 @@ __global__ __launch_bounds__(kSsThreads) void ssim_fwd_kernel(const float* __res
   row_pass<2, true, kSsFwdHold>(s_buf + kSsFwdXy, s_buf, G);
   __syncthreads();
   const int c = threadIdx.x & (kSsTile - 1), g = threadIdx.x / kSsTile;
-  float m[kSsQ][5];
-  col_pass<5>(s_buf, c, g, G, m);
+  float m[kSsQ][kSsMoments];
+  col_pass<kSsMoments>(s_buf, c, g, G, m);
   const int px = tx * kSsTile + c;
   float s_sum = 0.0f;
 #pragma unroll
@@ -242,8 +244,11 @@ __global__ __launch_bounds__(kSsThreads) void ssim_fwd_kernel(const float* __res
     if (py >= H || px >= W) continue;
     const float mu1 = m[q][0], mu2 = m[q][1];
     const float mu11 = mu1 * mu1, mu22 = mu2 * mu2, mu12 = mu1 * mu2;
-    const float A = 2.0f * mu12 + kSsC1, B = 2.0f * (m[q][4] - mu12) + kSsC2;
-    const float Cc = mu11 + mu22 + kSsC1, D = (m[q][2] - mu11) + (m[q][3] - mu22) + kSsC2;
+    // what the rounded products mu11, mu22, mu12 leave out, so that the variances do not lose it
+    const float e11 = fmaf(mu1, mu1, -mu11), e22 = fmaf(mu2, mu2, -mu22), e12 = fmaf(mu1, mu2, -mu12);
+    const float mu2s = mu11 + mu22;
+    const float A = 2.0f * mu12 + kSsC1, B = 2.0f * ((m[q][3] - mu12) - e12) + kSsC2;
+    const float Cc = mu2s + kSsC1, D = ((m[q][2] - mu2s) - (e11 + e22)) + kSsC2;
     // Cc >= C1 and D ~ C2 + variances are positive: one reciprocal each, no division
     const float rC = __builtin_amdgcn_rcpf(Cc), rD = __builtin_amdgcn_rcpf(D);
     const float rCD = rC * rD;
@@ -268,12 +273,13 @@ __global__ __launch_bounds__(kSsThreads) void ssim_fwd_kernel(const float* __res
 
 // One workgroup of kSsRedThreads: sums the per-tile partials in double (every load of a thread
 // issued before its first add), writes loss[0] = total, loss[1] = mean |x - y|, loss[2] = mean
-// SSIM.
+// SSIM, and the total again to *value (may be NULL).
 constexpr int kSsRedThreads = 1024;
 constexpr int kSsRedUnroll = 4;
 __global__ __launch_bounds__(kSsRedThreads) void ssim_reduce_kernel(const float* __restrict__ partials,
                                                                     int64_t n_blocks, double n_elems, float lambda,
-                                                                    float* __restrict__ loss) {
+                                                                    float* __restrict__ loss,
+                                                                    float* __restrict__ value) {
   __shared__ double s_sum[2][kSsRedThreads / 64];
   double a = 0.0, b = 0.0;
   for (int64_t k0 = threadIdx.x; k0 < n_blocks; k0 += kSsRedThreads * kSsRedUnroll) {
@@ -307,7 +313,9 @@ __global__ __launch_bounds__(kSsRedThreads) void ssim_reduce_kernel(const float*
       sb += s_sum[1][w];
     }
     const double ssim = sa / n_elems, l1 = sb / n_elems;
-    loss[0] = static_cast<float>((1.0 - lambda) * l1 + lambda * (1.0 - ssim));
+    const float total = static_cast<float>((1.0 - lambda) * l1 + lambda * (1.0 - ssim));
+    loss[0] = total;
+    if (value) *value = total;
     loss[1] = static_cast<float>(l1);
     loss[2] = static_cast<float>(ssim);
   }
@@ -388,13 +396,14 @@ extern "C" size_t gs_l1_ssim_workspace_size(int channels, int height, int width)
 // channel, every one written by ssim_fwd_kernel before ssim_reduce_kernel reads it, so nothing
 // has to start at zero).
 static int l1_ssim_fwd_launch(const float* image, const float* target, int channels, int height, int width,
-                              float lambda_dssim, float* dmap, float* loss, float* partials, hipStream_t st) {
+                              float lambda_dssim, float* dmap, float* loss, float* value, float* partials,
+                              hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(ssim_blocks(channels, height, width)));
   hipLaunchKernelGGL(ssim_fwd_kernel, grid, dim3(kSsThreads), 0, st, image, target, height, width, ssim_weights(),
                      dmap, partials);
   const double n = static_cast<double>(channels) * height * width;
   hipLaunchKernelGGL(ssim_reduce_kernel, dim3(1), dim3(kSsRedThreads), 0, st, partials,
-                     ssim_blocks(channels, height, width), n, lambda_dssim, loss);
+                     ssim_blocks(channels, height, width), n, lambda_dssim, loss, value);
   return check_launch("l1_ssim_fwd");
 }
 
@@ -407,16 +416,23 @@ static int l1_ssim_check_args(const float* image, const float* target, int chann
   return GS_OK;
 }
 
-extern "C" int gs_l1_ssim_fwd(const float* image, const float* target, int channels, int height, int width,
-                              float lambda_dssim, float* dmap, float* loss, void* workspace, size_t workspace_bytes,
-                              void* stream) {
+extern "C" int gs_l1_ssim_fwd_value(const float* image, const float* target, int channels, int height, int width,
+                                    float lambda_dssim, float* dmap, float* loss, float* value, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
   clear_error();
   const int rc = l1_ssim_check_args(image, target, channels, height, width, lambda_dssim, loss);
   if (rc != GS_OK) return rc;
   const size_t need = gs_l1_ssim_workspace_size(channels, height, width);
   GS_REQUIRE(workspace && workspace_bytes >= need, GS_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
-  return l1_ssim_fwd_launch(image, target, channels, height, width, lambda_dssim, dmap, loss,
+  return l1_ssim_fwd_launch(image, target, channels, height, width, lambda_dssim, dmap, loss, value,
                             static_cast<float*>(workspace), as_stream(stream));
+}
+
+extern "C" int gs_l1_ssim_fwd(const float* image, const float* target, int channels, int height, int width,
+                              float lambda_dssim, float* dmap, float* loss, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+  return gs_l1_ssim_fwd_value(image, target, channels, height, width, lambda_dssim, dmap, loss, nullptr, workspace,
+                              workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -472,8 +488,8 @@ extern "C" int gs_l1_ssim_fwd_noalloc(const float* image, const float* target, i
              channels, height, width, static_cast<long long>(tiles), GS_L1_SSIM_NOALLOC_MAX_TILES);
   float* partials = scratch_on_current_device();
   if (partials == nullptr) return GS_ERR_LAUNCH;
-  return l1_ssim_fwd_launch(image, target, channels, height, width, lambda_dssim, dmap, loss, partials,
-                            as_stream(stream));
+  return l1_ssim_fwd_launch(image, target, channels, height, width, lambda_dssim, dmap, loss, nullptr,
+                            partials, as_stream(stream));
 }
 
 extern "C" int gs_l1_ssim_bwd(const float* image, const float* target, const float* dmap, int channels, int height,

@@ -503,6 +503,10 @@ size_t gs_l1_ssim_workspace_size(int channels, int height, int width);
 int gs_l1_ssim_fwd(const float* image, const float* target, int channels, int height, int width,
                    float lambda_dssim, float* dmap, float* loss, void* workspace, size_t workspace_bytes,
                    void* stream);
+/* gs_l1_ssim_fwd that also writes the total to *value (may be NULL), apart from loss[3]. */
+int gs_l1_ssim_fwd_value(const float* image, const float* target, int channels, int height, int width,
+                         float lambda_dssim, float* dmap, float* loss, float* value, void* workspace,
+                         size_t workspace_bytes, void* stream);
 int gs_l1_ssim_bwd(const float* image, const float* target, const float* dmap, int channels, int height,
                    int width, float lambda_dssim, const float* grad_loss, float* grad_image, void* stream);
 
