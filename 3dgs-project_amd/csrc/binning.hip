@@ -1019,7 +1019,12 @@ __global__ void rect_counts_kernel(const int4* __restrict__ rects, int64_t n, in
 // emitted in depth order. No kernel waits on another workgroup.
 // ---------------------------------------------------------------------------------------
 constexpr int kSpanMaxDim = 512;   // tiles per side (the LDS of the placement kernels)
-constexpr int kRowChunk = 256;     // depth positions per wavefront in the row pass
+constexpr int kRowChunk = 256;     // depth positions per workgroup in the row pass
+// Consecutive chunks of the row pass that share an XCD, so that its L2 merges their writes.
+// One contiguous eighth of the chunks per XCD left most CUs idle for half the pass, the near eighth
+// holding most spans: 3M Gaussians, span_place 170 -> 101 us, span_gather 151 -> 142; bands of 4 and
+// 64 within 2 us.
+constexpr int kRowBand = 16;
 constexpr int kSpanChunk = 1024;   // spans per workgroup in the column pass
 constexpr int kSpanWaves = 4;      // wavefronts per workgroup (256 threads)
 constexpr int kColScanThreads = kBoThreads;  // the last workgroup runs tile_scan_block
@@ -1138,7 +1143,7 @@ __global__ __launch_bounds__(256) void span_gather_kernel(const SplatRec* __rest
   float4* s_set = reinterpret_cast<float4*>(s_wbase);
   uint32_t* s_rex = s_wbase + 64 * 12;
   uint32_t* s_gid = s_rex + 64;
-  const int c = xcd_tile(blockIdx.x, gridDim.x);  // the grid has n_chunks workgroups
+  const int c = xcd_band_tile(blockIdx.x, gridDim.x, kRowBand);  // the grid has n_chunks workgroups
   for (int q = threadIdx.x; q < ty4; q += 256) s_cnt[q] = 0u;
   const int64_t j = static_cast<int64_t>(c) * kRowChunk + wave * kWave + lane;
   uint32_t rows = 0, g = 0;
@@ -1295,7 +1300,7 @@ __global__ __launch_bounds__(256) void span_place_kernel(const uint2* __restrict
   uint32_t* s_pos = s_dyn + align4i(tiles_y + 1);  // [kSpanWaves][ty4]
   unsigned long long* s_cov =
       reinterpret_cast<unsigned long long*>(s_pos + kSpanWaves * ty4) + static_cast<int64_t>(wave) * ty4;
-  const int c = xcd_tile(blockIdx.x, gridDim.x);
+  const int c = xcd_band_tile(blockIdx.x, gridDim.x, kRowBand);
   const uint2 info = chunk_info[c];
   const uint32_t q0 = static_cast<uint32_t>((static_cast<uint64_t>(info.y) * wave) / kSpanWaves);
   const uint32_t q1 = static_cast<uint32_t>((static_cast<uint64_t>(info.y) * (wave + 1)) / kSpanWaves);
@@ -1637,42 +1642,52 @@ __global__ __launch_bounds__(kDiffThreads) void rect_tiles_kernel(
   }
 }
 
-// Column pass, placement: workgroup per chunk, each wavefront places the instances of its
-// kWaveSpans spans. Instance i of a wavefront's spans (numbered in (span, column) order) goes
-// to its tile's start + the chunk's offset in the tile + the earlier wavefronts' instances in
-// the column + its rank among the wavefront's earlier instances in the column. The instances
-// are taken in batches of R windows of 64: an owner table gives each instance its span; in a
-// window, each span (at most 64, all of distinct columns) ORs its bit (span - the window's first
-// span) into the window's column mask, so the rank inside the window is the number of lower
-// bits; a pass over the columns then turns the windows' counts into running positions.
-constexpr int kOwnerTable = 2048;  // instances per owner-table segment (one byte each)
+// Column pass, placement: workgroup per chunk, its instances sorted by column in LDS and written
+// out in that order, so a wavefront's store covers a few runs of a tile's list instead of 64 lists.
+// A chunk is taken in batches of consecutive spans, at most kG groups of 32 and at most kWriteCap
+// instances (a span has at most kSpanMaxDim):
+//   cover   each span toggles its bit in its group's word of its first column and of the column
+//           past its last; the exclusive-or of the words up to column t is then the set of the
+//           group's spans that cover t
+//   start   a scan of the words' bit counts, column by column and group by group, is the place of
+//           every word's first instance in the batch, and of every column in its tile's list
+//   stage   a thread per word puts its spans, in order, at that place (with the column)
+//   write   instance i of the batch goes to (its column's place in the list) - (the column's
+//           first i) + i
+// Bound by the lists' write and by LDS. Writing each instance straight to its list's next place,
+// 64 lists to a store, made one L2 request per instance and six times the lists' bytes of HBM
+// writes (3M Gaussians, 123 x 69 tiles: 442 us, 24.8M requests to HBM); so 258 us, 8.2M. Batches
+// of 5120 and 6144 instances: 270 and 260 us.
+constexpr uint32_t kWriteCap = 4096;  // instances of a batch
+// Groups of a batch and columns per thread: the words take 8 KB at 128 columns, 16 KB at 512.
+constexpr int write_groups(int tiles_x) { return tiles_x <= 256 ? 16 : 8; }
+constexpr size_t write_lds_words(int tx4, int ty4, int groups) {
+  return static_cast<size_t>(ty4) + 2 * tx4 + groups * tx4 + groups * 32 + kWriteCap + groups * tx4 / 2;
+}
+static_assert(kWriteCap >= kSpanMaxDim && kWriteCap <= 0xffff, "a batch takes a span; 16-bit places");
 
-template <bool kKeys, int R>
+template <bool kKeys, int kG>
 __global__ __launch_bounds__(256) void span_col_write_kernel(
     const uint2* __restrict__ spans, const uint32_t* __restrict__ rowtot, const uint32_t* __restrict__ colcnt,
     const uint32_t* __restrict__ ranges, int tiles_x, int tiles_y, int64_t span_cap, int64_t chunk_cap, int64_t m,
     uint32_t* __restrict__ point_list, uint64_t* __restrict__ keys, const uint32_t* __restrict__ dkey_of,
     uint32_t dkey0) {
+  constexpr int kPerThread = kG == 16 ? 1 : 2;  // columns
   extern __shared__ __align__(16) uint32_t s_dyn[];
   __shared__ uint32_t s_wsum[kSpanWaves];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  // LDS: row bases [tiles_y + 1]; column positions [kSpanWaves][tiles_x + 1]; per wavefront:
-  // the windows' column masks [R][tiles_x] (uint64) and offsets [R][tiles_x], the spans
-  // (uint2) and their instance prefix, the owner table (bytes)
+  __shared__ uint32_t s_end;
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
   const int tx4 = align4i(tiles_x + 1);
-  const int wave_words = R * 3 * tx4 + 2 * kWaveSpans + (kWaveSpans + 4) + kOwnerTable / 4;
-  uint32_t* s_rbase = s_dyn;
-  uint32_t* s_cpos = s_dyn + align4i(tiles_y + 1);  // [kSpanWaves][tx4]
-  uint32_t* s_w = s_cpos + kSpanWaves * tx4 + wave * wave_words;
-  unsigned long long* s_cov = reinterpret_cast<unsigned long long*>(s_w);  // [R][tx4]
-  uint32_t* s_off = s_w + 2 * R * tx4;                                       // [R][tx4]
-  uint2* s_span = reinterpret_cast<uint2*>(s_off + R * tx4);                 // [kWaveSpans]
-  uint32_t* s_pre = s_off + R * tx4 + 2 * kWaveSpans;                        // [kWaveSpans + 1]
-  uint8_t* s_tbl = reinterpret_cast<uint8_t*>(s_pre + kWaveSpans + 4);       // [kOwnerTable]
-  uint32_t* s_pos = s_cpos + wave * tx4;
+  uint32_t* s_rbase = s_dyn;                                       // [tiles_y + 1]
+  uint32_t* s_pos = s_dyn + align4i(tiles_y + 1);                  // [tx4] next place in the column's list
+  uint32_t* s_to = s_pos + tx4;                                    // [tx4] that, less the column's first i
+  uint32_t* s_cov = s_to + tx4;                                    // [kG][tx4]
+  uint32_t* s_id = s_cov + kG * tx4;                               // [kG * 32] the batch's Gaussians
+  uint32_t* s_stage = s_id + kG * 32;                              // [kWriteCap] column << 16 | span
+  uint16_t* s_at = reinterpret_cast<uint16_t*>(s_stage + kWriteCap);  // [kG][tx4]
+  for (int q = tid; q < kG * tx4; q += 256) s_cov[q] = 0u;
+  if (tid == 0) s_end = ~0u;
   span_row_bases<256>(rowtot, tiles_y, s_rbase, s_wsum);
-  for (int q = lane; q < R * tx4; q += kWave) s_cov[q] = 0ull;
   const int64_t n_chunks = min<int64_t>(s_rbase[tiles_y] / kSpanChunk, chunk_cap);
   const XcdRange xr = xcd_range(n_chunks);
   for (int64_t k = xr.lo + xr.wid; k < xr.hi; k += xr.nw) {
@@ -1680,145 +1695,133 @@ __global__ __launch_bounds__(256) void span_col_write_kernel(
     const int64_t lim = min<int64_t>(static_cast<int64_t>(s_rbase[sc.row]) + rowtot[sc.row], span_cap);
     const int64_t t_row = static_cast<int64_t>(sc.row) * tiles_x;
     uint2 sp[kPerLane];
-    load_wave_spans(spans, k, wave, lane, lim, tiles_x, sp);
-    wave_column_counts(sp, tiles_x, lane, s_pos);
+    load_wave_spans(spans, k, wave, lane, lim, tiles_x, sp);  // spans kPerLane * tid ...
+    for (int t = tid; t < tiles_x; t += 256) s_pos[t] = ranges[2 * (t_row + t)] + colcnt[k * tiles_x + t];
+    uint32_t sum = 0;
+#pragma unroll
+    for (int e = 0; e < kPerLane; ++e) sum += sp[e].y >> 16;
+    uint32_t first = wave_incl_scan(sum);
+    if (lane == kWave - 1) s_wsum[wave] = first;
+    first -= sum;
     __syncthreads();
-    // each wavefront's first position in every column: the tile's start, the chunk's offset in
-    // the tile, then the earlier wavefronts' instances
-    for (int t = threadIdx.x; t < tiles_x; t += 256) {
-      uint32_t run = ranges[2 * (t_row + t)] + colcnt[k * tiles_x + t];
+    uint32_t all = 0;
 #pragma unroll
-      for (int q = 0; q < kSpanWaves; ++q) {
-        const uint32_t c = s_cpos[q * tx4 + t];
-        s_cpos[q * tx4 + t] = run;
-        run += c;
+    for (int q = 0; q < kSpanWaves; ++q) {
+      if (q < wave) first += s_wsum[q];
+      all += s_wsum[q];
+    }
+    // the batch: spans a .. b - 1, of which `done` instances lie before
+    uint32_t a = 0, done = 0;
+    while (done < all) {
+      uint32_t b = a + kG * 32;
+      if (all - done > kWriteCap) {  // up to the first span that ends beyond the batch's instances
+        uint32_t run = first;
+#pragma unroll
+        for (int e = 0; e < kPerLane; ++e) {
+          const uint32_t i = static_cast<uint32_t>(kPerLane * tid + e);
+          run += sp[e].y >> 16;
+          if (i < b && run > done + kWriteCap) {
+            atomicMin(&s_end, i);
+            break;
+          }
+        }
+        __syncthreads();
+        b = min(b, s_end);
       }
-    }
-    __syncthreads();
-    // the wavefront's non-empty spans, compacted in order: span index c of s_span / s_pre is the
-    // c-th non-empty one, so the 64 consecutive instances of a window always lie in at most 64
-    // consecutive span indices (the rank bits below), whatever spans were empty
-    uint32_t sum = 0, nz = 0;
-#pragma unroll
-    for (int e = 0; e < kPerLane; ++e) {
-      sum += sp[e].y >> 16;
-      nz += (sp[e].y >> 16) != 0u ? 1u : 0u;
-    }
-    uint32_t total, n_nz;
-    uint32_t run = wave_excl_scan(sum, lane, total);
-    uint32_t ci = wave_excl_scan(nz, lane, n_nz);
-    uint32_t cidx[kPerLane];
-#pragma unroll
-    for (int e = 0; e < kPerLane; ++e) {
-      cidx[e] = ci;
-      if ((sp[e].y >> 16) != 0u) {
-        s_pre[ci] = run;
-        s_span[ci] = sp[e];
-        ++ci;
-      }
-      run += sp[e].y >> 16;
-    }
-    uint32_t carry = 0u;  // the span holding the last instance of the previous segment
-    for (uint32_t t0 = 0; t0 < total; t0 += kOwnerTable) {
-      const uint32_t t1 = min<uint32_t>(t0 + kOwnerTable, total);
-      wave_sync();  // the previous segment is done with the table
-      // owner table: every instance of the segment gets its span's index. The spans' instances
-      // are consecutive in span order, so the owner of instance i is the largest span index
-      // whose first instance is at or before i: each non-empty span starting in the segment
-      // marks its first entry, and a prefix maximum over the entries (seeded with the span
-      // holding the segment's first instance) fills the rest, in the same few instructions
-      // whatever the spans' widths.
-      uint32_t* s_tw = reinterpret_cast<uint32_t*>(s_tbl);
-      for (int q = lane; q < kOwnerTable / 4; q += kWave) s_tw[q] = 0u;
-      wave_sync();
 #pragma unroll
       for (int e = 0; e < kPerLane; ++e) {
-        if ((sp[e].y >> 16) == 0u) continue;
-        const uint32_t st = s_pre[cidx[e]];
-        if (st >= t0 && st < t1) s_tbl[st - t0] = static_cast<uint8_t>(cidx[e]);
+        const uint32_t i = static_cast<uint32_t>(kPerLane * tid + e), at = i - a;
+        const uint32_t tx0 = sp[e].y & 0xffffu, nt = sp[e].y >> 16;
+        if (i >= a && i < b && nt) {
+          s_id[at] = sp[e].x;
+          uint32_t* w = s_cov + (at >> 5) * tx4 + tx0;
+          atomicXor(w, 1u << (at & 31u));
+          atomicXor(w + nt, 1u << (at & 31u));
+        }
       }
-      wave_sync();
+      __syncthreads();
       {
-        constexpr int kBytes = kOwnerTable / kWave;  // 32 consecutive entries per lane
-        uint32_t w[kBytes / 4];
+        constexpr int kMine = kG / kSpanWaves;  // groups of this wavefront, scanned side by side
+        uint32_t carry[kMine];
 #pragma unroll
-        for (int q = 0; q < kBytes / 4; ++q) w[q] = s_tw[lane * (kBytes / 4) + q];
-        uint32_t run = 0u;
+        for (int j = 0; j < kMine; ++j) carry[j] = 0u;
+        for (int c0 = 0; c0 < tiles_x; c0 += kWave) {
+          const int t = c0 + lane;
+          uint32_t* w = s_cov + wave * kMine * tx4 + t;
+          uint32_t v[kMine];
 #pragma unroll
-        for (int q = 0; q < kBytes / 4; ++q)
+          for (int j = 0; j < kMine; ++j) v[j] = t < tiles_x ? w[j * tx4] : 0u;
 #pragma unroll
-          for (int b = 0; b < 4; ++b) run = max(run, (w[q] >> (8 * b)) & 0xffu);
-        // the largest marker of the lanes before this one (a wavefront max-scan), and the seed
-        const uint32_t incl = wave_scan(run, 0u, [](uint32_t x, uint32_t y) { return max(x, y); });
-        uint32_t m = max(carry, __shfl_up(incl, 1, 64));
-        if (lane == 0) m = carry;
-#pragma unroll
-        for (int q = 0; q < kBytes / 4; ++q) {
-          uint32_t out = 0u;
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            m = max(m, (w[q] >> (8 * b)) & 0xffu);
-            out |= m << (8 * b);
+          for (int j = 0; j < kMine; ++j) {
+            v[j] = carry[j] ^ wave_scan(v[j], 0u, [](uint32_t x, uint32_t y) { return x ^ y; });
+            carry[j] = wave_last(v[j]);
+            if (t < tiles_x) w[j * tx4] = v[j];
           }
-          s_tw[lane * (kBytes / 4) + q] = out;
         }
       }
-      wave_sync();
-      carry = s_tbl[t1 - 1 - t0];
-      for (uint32_t b0 = t0; b0 < t1; b0 += R * kWave) {
-        uint32_t col[R], g[R], bit[R], low[R];
-        bool live[R];
+      __syncthreads();
+      uint32_t cnt[kPerThread][kG], col[kPerThread], mine = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const uint32_t w0 = b0 + r * kWave;
-          const uint32_t i = w0 + static_cast<uint32_t>(lane);
-          live[r] = i < t1;
-          col[r] = g[r] = bit[r] = 0u;
-          if (live[r]) {
-            const uint32_t own = s_tbl[i - t0];
-            const uint32_t first = s_tbl[w0 - t0];  // the window's first span
-            const uint2 e = s_span[own];
-            col[r] = (e.y & 0xffffu) + (i - s_pre[own]);
-            g[r] = e.x;
-            bit[r] = own - first;  // < 64: 64 instances lie in at most 64 compacted spans
-          }
+      for (int j = 0; j < kPerThread; ++j) {
+        const int t = kPerThread * tid + j;
+        col[j] = 0;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+          cnt[j][g] = t < tiles_x ? static_cast<uint32_t>(__popc(s_cov[g * tx4 + t])) : 0u;
+          col[j] += cnt[j][g];
         }
+        mine += col[j];
+      }
+      uint32_t at = wave_incl_scan(mine);
+      if (lane == kWave - 1) s_wsum[wave] = at;
+      at -= mine;
+      __syncthreads();
+      uint32_t total = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-          if (live[r]) atomicOr(&s_cov[r * tx4 + col[r]], 1ull << bit[r]);
-        wave_sync();
+      for (int q = 0; q < kSpanWaves; ++q) {
+        if (q < wave) at += s_wsum[q];
+        total += s_wsum[q];
+      }
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-          low[r] = live[r] ? static_cast<uint32_t>(__popcll(s_cov[r * tx4 + col[r]] & ((1ull << bit[r]) - 1ull))) : 0u;
-        wave_sync();
-        // the windows' counts per column -> running positions (and the masks cleared)
+      for (int j = 0; j < kPerThread; ++j) {
+        const int t = kPerThread * tid + j;
+        if (t >= tiles_x) continue;
+        const uint32_t pos = s_pos[t];
+        s_to[t] = pos - at;
+        s_pos[t] = pos + col[j];
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+          s_at[g * tx4 + t] = static_cast<uint16_t>(at);
+          at += cnt[j][g];
+        }
+      }
+      __syncthreads();
+      for (int g = wave; g < kG; g += kSpanWaves)
         for (int t = lane; t < tiles_x; t += kWave) {
-          uint32_t p = s_pos[t];
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            s_off[r * tx4 + t] = p;
-            p += static_cast<uint32_t>(__popcll(s_cov[r * tx4 + t]));
-            s_cov[r * tx4 + t] = 0ull;
-          }
-          s_pos[t] = p;
-        }
-        wave_sync();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          if (live[r]) {
-            const uint32_t pos = s_off[r * tx4 + col[r]] + low[r];
-            if (pos < m) {
-              point_list[pos] = g[r];
-              if constexpr (kKeys)
-                keys[pos] = (static_cast<uint64_t>(t_row + col[r]) << 32) |
-                            static_cast<uint32_t>(dkey_of[g[r]] + dkey0);
-            }
+          uint32_t cov = s_cov[g * tx4 + t], p = s_at[g * tx4 + t];
+          const uint32_t tag = static_cast<uint32_t>(t) << 16 | static_cast<uint32_t>(g * 32);
+          while (cov) {
+            s_stage[p++] = tag + static_cast<uint32_t>(__builtin_ctz(cov));
+            cov &= cov - 1u;
           }
         }
-        wave_sync();  // the offsets are rewritten by the next batch
+      __syncthreads();
+#pragma unroll 4
+      for (uint32_t i = static_cast<uint32_t>(tid); i < total; i += 256) {
+        const uint32_t v = s_stage[i], t = v >> 16, g = s_id[v & 0xffffu], pos = s_to[t] + i;
+        if (pos < m) {
+          point_list[pos] = g;
+          if constexpr (kKeys)
+            keys[pos] = (static_cast<uint64_t>(t_row + t) << 32) | static_cast<uint32_t>(dkey_of[g] + dkey0);
+        }
       }
+      for (int q = tid; q < kG * tx4; q += 256) s_cov[q] = 0u;
+      if (tid == 0) s_end = ~0u;
+      a = b;
+      done += total;
+      __syncthreads();  // the stage and the Gaussians are rewritten
     }
-    __syncthreads();  // the column positions are rewritten for the next chunk
+    if (all == 0) __syncthreads();  // s_wsum and s_pos are rewritten by the next chunk
   }
 }
 
@@ -2062,13 +2065,8 @@ static void bin_spans(const SplatRec* rec, const int4* rects, const uint32_t* dk
   const size_t lds_place = static_cast<size_t>(a4(tiles_y + 1) + kSpanWaves * a4(tiles_y) * 3) * 4;
   const int tx4 = a4(tiles_x + 1);
   const size_t lds_ccount = (static_cast<size_t>(a4(tiles_y + 1)) + kSpanWaves * tx4) * 4;
-  // placement windows per batch: fewer windows cost more wavefront syncs per window, more cost LDS
-  // and so occupancy; up to 128 tile columns the LDS stays near 36 KB (4 workgroups per CU)
-  // (3M SH3, 123 columns: 351 us with 2 windows, 363 with 4, 379 with 1)
-  const int R = tiles_x <= 64 ? 4 : tiles_x <= 256 ? 2 : 1;
-  const size_t lds_cwrite =
-      (static_cast<size_t>(a4(tiles_y + 1)) + kSpanWaves * tx4 +
-       kSpanWaves * (R * 3 * tx4 + 2 * kWaveSpans + (kWaveSpans + 4) + kOwnerTable / 4)) * 4;
+  const int groups = write_groups(tiles_x);
+  const size_t lds_cwrite = write_lds_words(tx4, a4(tiles_y + 1), groups) * 4;
   const unsigned g_rows = static_cast<unsigned>(L.n_chunks);  // a workgroup per chunk
   // the column kernels deal their chunks to the 8 XCDs in contiguous ranges: a multiple of 8
   // workgroups
@@ -2087,14 +2085,14 @@ static void bin_spans(const SplatRec* rec, const int4* rects, const uint32_t* dk
   hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(kBoThreads), 0, st, tcnt, tiles_x * tiles_y, ranges,
                      bucket_offsets, tile_offsets, list_header);
   stage_mark("span_columns", st);
-#define GS_SPAN_WRITE(KEYS, RR)                                                                                     \
-  hipLaunchKernelGGL((span_col_write_kernel<KEYS, RR>), dim3(g_cols), dim3(256), lds_cwrite, st, spans, rowtot,     \
+#define GS_SPAN_WRITE(KEYS, GROUPS)                                                                                 \
+  hipLaunchKernelGGL((span_col_write_kernel<KEYS, GROUPS>), dim3(g_cols), dim3(256), lds_cwrite, st, spans, rowtot, \
                      colhist, ranges, tiles_x, tiles_y, L.span_cap, L.chunk_cap, m, point_list, sorted_keys, dkey_of, \
                      dkey0)
   if (sorted_keys) {
-    if (R == 4) GS_SPAN_WRITE(true, 4); else if (R == 2) GS_SPAN_WRITE(true, 2); else GS_SPAN_WRITE(true, 1);
+    if (groups == 16) GS_SPAN_WRITE(true, 16); else GS_SPAN_WRITE(true, 8);
   } else {
-    if (R == 4) GS_SPAN_WRITE(false, 4); else if (R == 2) GS_SPAN_WRITE(false, 2); else GS_SPAN_WRITE(false, 1);
+    if (groups == 16) GS_SPAN_WRITE(false, 16); else GS_SPAN_WRITE(false, 8);
   }
 #undef GS_SPAN_WRITE
   stage_mark("span_write", st);

@@ -107,5 +107,14 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
   const int q = n / 8, r = n % 8, x = b % 8, k = b / 8;
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + k;
 }
+// The same in bands: XCD x takes the bands x, x + 8, ... of `band` consecutive indexes (and the last
+// n % (8 band) as above). For work whose cost runs with the index -- depth-ordered chunks: near
+// Gaussians have many spans, culled ones none -- where one contiguous eighth would be one XCD's.
+__device__ __forceinline__ int xcd_band_tile(int b, int n, int band) {
+  const int full = n / (8 * band) * (8 * band);
+  if (b >= full) return full + xcd_tile(b - full, n - full);
+  const int x = b % 8, k = b / 8;
+  return (k / band * 8 + x) * band + k % band;
+}
 
 }  // namespace gs

@@ -8,11 +8,10 @@
 //
 // One workgroup per 32x32 tile and channel. Forward: the tile plus a 5-pixel halo of both
 // images goes to LDS, the four moments that S depends on (x, y, x^2 + y^2, xy: the variances enter
-// only as their sum) are filtered separably (rows, then
-// columns; in each pass a thread computes four adjacent outputs from the 14 inputs they share,
-// so every input is read and squared once), and each pixel writes the three partial derivatives
-// of its SSIM value the backward needs (dS/dmu_x, dS/dE[x^2], dS/dE[xy]) plus per-workgroup
-// partial sums for the loss value.
+// only as their sum) are filtered separably (rows, then columns; in each pass a thread computes
+// four adjacent outputs from the 14 inputs they share, so every input is read and squared once),
+// and each pixel writes the three partial derivatives of its SSIM value the backward needs
+// (dS/dmu_x, dS/dE[x^2], dS/dE[xy]) plus per-workgroup partial sums for the loss value.
 // Backward: the same separable filter on the three partial maps (the Gaussian is symmetric, so
 // the transpose of the zero-padded filter is itself), then
 //   dL/dx = (1 - lambda) sign(x - y) / N - lambda / N (G*a + 2 x G*b + y G*c).

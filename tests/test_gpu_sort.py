@@ -181,6 +181,19 @@ def test_rect_binning_matches_the_stable_sort(W, H, n, rmax, binning):
     assert np.array_equal(rb.bucket_offsets.cpu().numpy().astype(np.int64), boff)
 
 
+@pytest.mark.parametrize("W,H,n,rmax", [
+    (4096, 24, 9_000, 257),    # 256 columns, a thread each; batches end at 4096 instances
+    (4112, 24, 9_000, 258),    # 257 columns, two a thread
+    (8192, 16, 1_100, 2_000),  # spans of up to 512 columns, one row, two chunks
+    (1024, 16, 5_000, 2),      # half of the spans empty, batches of 512 spans
+    (1040, 16, 513, 2),        # 65 columns: a second wavefront's worth of one
+])
+def test_span_write_batches(W, H, n, rmax):
+    """The column placement where its batches end: at 4096 instances, at 512 spans (256 beyond 256
+    columns), and where a thread's columns or a wavefront's columns begin."""
+    test_rect_binning_matches_the_stable_sort(W, H, n, rmax, "spans")
+
+
 @pytest.mark.parametrize("n,offset", [(0, 0), (1, 0), (3, 1), (4097, 0), (1_000_003, 1), (15_625, 0)])
 def test_sum_u32(n, offset):
     """gs_sum_u32 (the instance count of the 3D forward) against numpy's uint64 sum, over values up to
