@@ -139,6 +139,7 @@ class _View:
         self.touched = self.image = self.alpha = None
         self.timings: dict = {}
         self._state = self._lists = self._grads = None
+        self.last_conic64 = None  # the float64 conic sums of the last backward
         self._soff, self._loff = _lib.ViewStateOffsets(), _lib.ViewListOffsets()
 
     def _view(self, arena, off, count, dtype, *shape):
@@ -476,6 +477,7 @@ def _backward(view: _View, means, log_scales, quats, opacity_logits, sh, grad_im
     if grads is None:
         grads = torch.zeros(view.n * (GRAD2D_FLOATS + 8), dtype=torch.float32, device=means.device)
     grad2d, conic64 = _split_grads2d(grads, view.n)
+    view.last_conic64 = conic64
     params, gs, outs = _backward_args(view, means, log_scales, quats, opacity_logits, sh)
     call("gs_view_backward", *params, view.m, view.ccam, view._state.data_ptr(), view._lists.data_ptr(), ptr(view.touched),
          ptr(view.image), ptr(grad_image), ptr(grad_alpha), ptr(grad2d), ptr(conic64),
