@@ -1656,8 +1656,8 @@ __global__ __launch_bounds__(kDiffThreads) void rect_tiles_kernel(
 //           first i) + i
 // Bound by the lists' write and by LDS. Writing each instance straight to its list's next place,
 // 64 lists to a store, made one L2 request per instance and six times the lists' bytes of HBM
-// writes (3M Gaussians, 123 x 69 tiles: 442 us, 24.8M requests to HBM); so 258 us, 8.2M. Batches
-// of 5120 and 6144 instances: 270 and 260 us.
+// writes (3M Gaussians, 123 x 69 tiles: 442 us, 24.8M requests to HBM); so 231 us, 8.2M.
+// (Batches of 5120 and 6144 instances: 5 % and 1 % slower.)
 constexpr uint32_t kWriteCap = 4096;  // instances of a batch
 // Groups of a batch and columns per thread: the words take 8 KB at 128 columns, 16 KB at 512.
 constexpr int write_groups(int tiles_x) { return tiles_x <= 256 ? 16 : 8; }
@@ -2085,8 +2085,11 @@ static void bin_spans(const SplatRec* rec, const int4* rects, const uint32_t* dk
   hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(kBoThreads), 0, st, tcnt, tiles_x * tiles_y, ranges,
                      bucket_offsets, tile_offsets, list_header);
   stage_mark("span_columns", st);
+  // a workgroup for one or two chunks, so that the hardware evens out what the chunks differ in
+  // (3M SH3, 10.7k chunks: 2048 workgroups 258 us, 4096 243, 7168 231, 10752 236)
+  const unsigned g_write = std::min<unsigned>((static_cast<unsigned>(L.chunk_cap) + 7u) & ~7u, 8192u);
 #define GS_SPAN_WRITE(KEYS, GROUPS)                                                                                 \
-  hipLaunchKernelGGL((span_col_write_kernel<KEYS, GROUPS>), dim3(g_cols), dim3(256), lds_cwrite, st, spans, rowtot, \
+  hipLaunchKernelGGL((span_col_write_kernel<KEYS, GROUPS>), dim3(g_write), dim3(256), lds_cwrite, st, spans, rowtot, \
                      colhist, ranges, tiles_x, tiles_y, L.span_cap, L.chunk_cap, m, point_list, sorted_keys, dkey_of, \
                      dkey0)
   if (sorted_keys) {
