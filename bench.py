@@ -158,12 +158,17 @@ def stage_bytes(fs, n_visible, active_buckets, splat_steps, used_pairs, staged, 
     T = fs.cam.n_tiles
     P = fs.cam.width * fs.cam.height
     B = int(fs.bucket_offsets[-1].item())
-    # the depth sort: 3 radix passes over N (histogram read 4 B, key+value read and write 16 B),
-    # the last one also gathering the counts into depth order (read + write 8 B)
-    sub = {"depth_sort": 3 * 20 * n + (8 * n if spans is None else 0)}
+    if spans is None and n <= 1 << 20:
+        # the depth order with the offsets: keys read by the bucket count and the scatter (8 B),
+        # key+value written and read (16 B), tile counts read, order and offsets written (12 B)
+        sub = {"depth_sort": 36 * n}
+    else:
+        # 3 radix passes over N (histogram read 4 B, key+value read and write 16 B), the last one
+        # also gathering the counts into depth order (read + write 8 B)
+        sub = {"depth_sort": 3 * 20 * n + (8 * n if spans is None else 0)}
     if spans is None:
-        # the scan of the counts in depth order (read, offsets written)
-        sub["instance_offsets"] = 8 * n
+        if n > 1 << 20:  # the scan of the counts in depth order (read, offsets written)
+            sub["instance_offsets"] = 8 * n
         # tile keys of 16 bits below 65536 tiles, else 32
         kb = 2 if T <= 65536 else 4
         # emission: order and offset per Gaussian, 48 B of the record of the visible, key + value
@@ -172,7 +177,7 @@ def stage_bytes(fs, n_visible, active_buckets, splat_steps, used_pairs, staged, 
         sub["key_duplication"] = 8 * n + 48 * n_visible + (kb + 4) * m
         sub["tile_sort"] = (kb + 2 * (kb + 4)) * m + (kb + (kb + 4) + 4) * m
         sub["ranges_buckets"] = 20 * T + 4 * B
-        depth = sub["depth_sort"] + sub["instance_offsets"]
+        depth = sub["depth_sort"] + sub.get("instance_offsets", 0)
     else:
         # rows: order 4 B and 48 B of the record of the visible per Gaussian, each span gathered
         # (8 B written, read) and placed by row (8 B written); columns: each span read by the
