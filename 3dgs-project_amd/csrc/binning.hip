@@ -1013,8 +1013,8 @@ __global__ void rect_counts_kernel(const int4* __restrict__ rects, int64_t n, in
 //            ranges and bucket offsets (span_col_scan_kernel); each chunk expands its spans into
 //            instances and writes the Gaussian of each at its tile's start + the chunk's offset
 //            + its rank among the chunk's instances in that column (span_col_write_kernel).
-// Ranks inside a wavefront come from ballots over the row or column bits in item order, and
-// chunks keep their order through the scans, so both passes are stable and a tile's list
+// Ranks inside a chunk come from coverage masks (of a row, of a column) whose bits are in item
+// order, and chunks keep their order through the scans, so both passes are stable and a tile's list
 // holds its Gaussians in depth order: the order of a stable sort by tile of the instances
 // emitted in depth order. No kernel waits on another workgroup.
 // ---------------------------------------------------------------------------------------

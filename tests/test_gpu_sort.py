@@ -194,6 +194,19 @@ def test_span_write_batches(W, H, n, rmax):
     test_rect_binning_matches_the_stable_sort(W, H, n, rmax, "spans")
 
 
+@pytest.mark.parametrize("tiles_x,tiles_y", [
+    (124, 127),  # 125 * 128 = 16000 corner sums: the largest canvas that fits one workgroup
+    (125, 127),  # one column more: tile counts after the emission instead
+    (1, 1),
+])
+@pytest.mark.parametrize("n", [1, 8192, 8193])
+def test_rect_tiles_edges(tiles_x, tiles_y, n):
+    """Tile counts from the rectangles' corners at the largest canvas they fit and one past it, and at
+    the rectangle counts where a second workgroup's difference array is added."""
+    assert bool(_lib.lib().gs_rect_tiles_fit(tiles_x, tiles_y)) == ((tiles_x + 1) * (tiles_y + 1) <= 16000)
+    test_rect_binning_matches_the_stable_sort(16 * tiles_x, 16 * tiles_y, n, 6, "radix")
+
+
 @pytest.mark.parametrize("n,offset", [(0, 0), (1, 0), (3, 1), (4097, 0), (1_000_003, 1), (15_625, 0)])
 def test_sum_u32(n, offset):
     """gs_sum_u32 (the instance count of the 3D forward) against numpy's uint64 sum, over values up to
