@@ -263,7 +263,9 @@ __global__ __launch_bounds__(kSsThreads) void ss_scatter_kernel(
   }
 }
 
-// Fold of v over the workgroup of NT threads by f, to every thread.
+// Fold of v over the workgroup of NT threads by f, to every thread. As in the two functions below, the
+// words s_w are still being read by other wavefronts when it returns: nothing may be stored there
+// before the next barrier (each of the three begins its own stores with one).
 template <int NT, typename F>
 __device__ __forceinline__ uint32_t block_fold(uint32_t v, uint32_t* s_w, F f) {  // (0 is f's identity)
   v = wave_last(wave_scan(v, 0u, f));
@@ -412,6 +414,7 @@ __global__ __launch_bounds__(NT) void ss_local_kernel(SsLocalArgs a) {
   __shared__ uint32_t s_bin[(NB > kWaves * 256 ? NB : kWaves * 256) + 1];
   __shared__ uint32_t s_start[256];
   __shared__ uint32_t s_w[kWaves];
+  __shared__ uint32_t s_top;  // number of keys equal to the largest
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const auto hi = [](uint32_t x, uint32_t y) { return max(x, y); };
   const uint32_t b0 = a.starts ? a.starts[blockIdx.x] : 0u;
@@ -478,10 +481,10 @@ __global__ __launch_bounds__(NT) void ss_local_kernel(SsLocalArgs a) {
       if (k0 + lane < used * kWaves) s_start[k0 + lane] = run + ex;
       run += total;
     }
-    if (lane == 0) s_w[0] = run;
+    if (lane == 0) s_top = run;  // (not to s_w: block_fold's readers may still be at it)
   }
   __syncthreads();
-  const uint32_t n_top = s_w[0], n_low = len - n_top;
+  const uint32_t n_top = s_top, n_low = len - n_top;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (r >= used) break;  // (uniform)
