@@ -814,16 +814,22 @@ __device__ __forceinline__ double swap16_add(double a, double b) {
   return f64_of(l[0], h[0]) + f64_of(l[1], h[1]);
 }
 
-// Lane 16's value in every lane.
-__device__ __forceinline__ float read_lane16(float v) {
-  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 16));
-}
-__device__ __forceinline__ double read_lane16(double v) {
-  return f64_of(__builtin_amdgcn_readlane(lo32(v), 16), __builtin_amdgcn_readlane(hi32(v), 16));
+// The totals of the lane's group of 8 from its pair of values.
+template <typename S>
+__device__ __forceinline__ void group_totals(S& u0, S& u1) {
+  u0 += dpp<0x141>(u0);  // row_half_mirror
+  u1 += dpp<0x141>(u1);
+  u0 += dpp<0xB1>(u0);  // quad_perm [1,0,3,2]
+  u1 += dpp<0xB1>(u1);
+  u0 += dpp<0x4E>(u0);  // quad_perm [2,3,0,1]
+  u1 += dpp<0x4E>(u1);
+  // (the totals are formed here, with every lane active, so that the DPP moves fold into the
+  // adds rather than the adds sinking into the owners' branch)
+  asm volatile("" : "+v"(u0), "+v"(u1));
 }
 
-// Reduction of one bucket-splat step (the 3D backward without the |dL/dmean2d| sums, and the 2D
-// rule sets). In: the
+// Reduction of one bucket-splat step (the 3D backward without the |dL/dmean2d| sums, and the toy2d
+// rules). In: the
 // lane's sums over its 4 pixels (one column) of h, h dy, h dy^2 and the three colour sums, and
 // the column's dx. The 4 lanes of a column (lane ^ 16, ^ 32) are summed first, transposing: xor
 // 32 with v_permlane32_swap over the pairs (h, red), (h dy, green), (h dy^2, blue), leaving the
@@ -848,15 +854,26 @@ __device__ __forceinline__ void wave_reduce_cols(S sh, S shy, S shyy, S cr, S cg
   const bool b3 = (lane & 8) != 0;
   u0 = (b3 ? v1 : v0) + dpp<0x128>(b3 ? v0 : v1);  // row_ror:8 = partner lane ^ 8
   u1 = (b3 ? v3 : t1) + dpp<0x128>(b3 ? t1 : v3);
-  u0 += dpp<0x141>(u0);  // row_half_mirror
-  u1 += dpp<0x141>(u1);
-  u0 += dpp<0xB1>(u0);  // quad_perm [1,0,3,2]
-  u1 += dpp<0xB1>(u1);
-  u0 += dpp<0x4E>(u0);  // quad_perm [2,3,0,1]
-  u1 += dpp<0x4E>(u1);
-  // (the totals are formed here, with every lane active, so that the DPP moves fold into the
-  // adds rather than the adds sinking into the owners' branch)
-  asm volatile("" : "+v"(u0), "+v"(u1));
+  group_totals(u0, u1);
+}
+
+// The same of the phase0 rules, whose shape and mean gradients are sums of h a and h b (a = l0 dx +
+// l1 dy, b = l2 dy, formed at each pixel): xor 32 over the pairs (h a, red), (h a dy, green),
+// (h b, blue), (h b dy, h), xor 16 over the pairs of those, the dx factor on the columns' h a. On return
+//   g 0: (sum h a, sum h b)            g 1: (sum h a dx, sum h b)
+//   g 2: (sum h a dy, sum h b dy)      g 4: (red, blue)        g 6: (green, sum h)
+// (g 3, 5, 7 hold repeats).
+template <typename S>
+__device__ __forceinline__ void wave_reduce_cols_chol(S sha, S shay, S shb, S shby, S sh, S cr, S cg, S cb, S dx,
+                                                      bool row0, S& u0, S& u1) {
+  const int lane = threadIdx.x & 63;
+  const S s0 = swap32_add(sha, cr), s1 = swap32_add(shay, cg), s2 = swap32_add(shb, cb), s3 = swap32_add(shby, sh);
+  const S t0 = swap16_add(s0, s1), t1 = swap16_add(s2, s3);
+  const S v1 = t0 * (row0 ? dx : S(1));
+  const bool b3 = (lane & 8) != 0;
+  u0 = (b3 ? v1 : t0) + dpp<0x128>(b3 ? t0 : v1);
+  u1 = t1 + dpp<0x128>(t1);
+  group_totals(u0, u1);
 }
 
 __device__ __forceinline__ void wave_reduce12(const double* v, double& u0, double& u1) {
@@ -1214,12 +1231,12 @@ __global__ __launch_bounds__(bwd_waves<kRules3D>() * kWave) void blend_bwd_bucke
 }
 
 // A staged splat of the 2D rule sets with the coefficient pairs of its final gradients: the owner
-// lanes' gradients are -(c0 u0 + c1 u1) of wave_reduce_cols's totals, pair i in co[2 i], co[2 i + 1].
+// lanes' gradients are -(c0 u0 + c1 u1) of the reduction's totals, pair i in co[2 i], co[2 i + 1].
 template <typename S>
 struct alignas(16) Staged2D {
   S mx, my, s0, s1, s2, o, cr, cg, cb;
   S cut;     // alpha < 1/255 wherever the exponent is not above this
-  S co[16];  // pairs of lanes 0, 1 (mean), 8, 9, 17 (shape), 16 (opacity), red or green, blue
+  S co[16];  // (owner2d says whose pair each is)
 };
 
 template <int R, typename S>
@@ -1230,16 +1247,18 @@ __device__ __forceinline__ Staged2D<S> stage2d(const Staged<S>& r, S cut) {
   s.cut = cut;
   S* c = s.co;
   if constexpr (R == kRulesPhase0) {
-    // power = -(a^2 + b^2) / 2, a = l0 dx + l1 dy, b = l2 dy, d = pixel - mean: with Q = L L^T the mean's
-    // gradient is Q (sum h dx, sum h dy), that of l0 -(l0 sum h dx^2 + l1 sum h dx dy), of l1
-    // -(l0 sum h dx dy + l1 sum h dy^2) (its second part is added apart: another group's total), of
-    // l2 -l2 sum h dy^2; the opacity logit's dL/do o (1 - o) = (1 - o) sum h
-    const S A = r.s0 * r.s0, B = r.s0 * r.s1, C = r.s1 * r.s1 + r.s2 * r.s2;
-    c[0] = -A; c[1] = -B; c[2] = -B; c[3] = -C;
-    c[4] = r.s0; c[5] = r.s1;
-    c[6] = S(0); c[7] = r.s0;
-    c[8] = -(S(1) - r.o); c[9] = S(0);
-    c[10] = S(0); c[11] = r.s2;
+    // power = -(a^2 + b^2) / 2, a = l0 dx + l1 dy, b = l2 dy, d = pixel - mean: the mean's gradient is
+    // (l0 sum h a, l1 sum h a + l2 sum h b), that of l0 -sum h a dx, of l1 -sum h a dy, of l2
+    // -sum h b dy; the opacity logit's dL/do o (1 - o) = (1 - o) sum h. (Along an elongated rotated
+    // splat l0 dx and l1 dy cancel: sums of h dx and h dy combined with Q = L L^T afterwards lose what
+    // their sizes differ from the gradients'. Error of the mean's gradient against float64 at standard
+    // deviations 2:10 / 0.6:60 px: 1.0e-5 / 2.2e-4 with them, so
+    // 2.3e-6 / 7.9e-6.)
+    c[0] = -r.s0; c[1] = S(0); c[2] = -r.s1; c[3] = -r.s2;
+    c[4] = S(1); c[5] = S(0);
+    c[6] = S(0); c[7] = S(1);
+    c[8] = S(0); c[9] = -(S(1) - r.o);
+    c[10] = S(-1); c[11] = S(0);
   } else {
     // power = -1/2 (A dx^2 + 2 B dx dy + C dy^2), d = mean - pixel; dL/do = (sum h) / o, since
     // h = alpha dL/dalpha and alpha = o G wherever it is not clamped (there h is 0)
@@ -1251,6 +1270,38 @@ __device__ __forceinline__ Staged2D<S> stage2d(const Staged<S>& r, S cut) {
   }
   c[12] = S(-1); c[13] = S(0); c[14] = S(0); c[15] = S(-1);
   return s;
+}
+
+// Which value of the gradient record a lane adds (slot; -1: none), and its coefficient pair.
+struct Owner2D {
+  int slot, pair;
+};
+
+template <int R>
+__device__ __forceinline__ Owner2D owner2d(int lane) {
+  switch (lane) {
+    case 0: return {0, 0};   // the mean
+    case 1: return {1, 1};
+    case 8: return {2, 2};   // conic A | l0
+    case 17: return {4, R == kRulesPhase0 ? 3 : 5};  // conic C | l2
+    case 32: return {6, 6};  // red
+  }
+  if constexpr (R == kRulesPhase0) {
+    switch (lane) {
+      case 16: return {3, 2};  // l1
+      case 33: return {8, 7};  // blue
+      case 48: return {7, 5};  // green
+      case 49: return {5, 4};  // opacity
+    }
+  } else {
+    switch (lane) {
+      case 9: return {3, 3};   // conic B
+      case 16: return {5, 4};  // opacity
+      case 33: return {7, 7};  // green
+      case 49: return {8, 7};  // blue
+    }
+  }
+  return {-1, 7};
 }
 
 // a / b rounded as the division instruction sequence rounds it for b in [0.01, 1] (one Newton step
@@ -1269,7 +1320,7 @@ __device__ __forceinline__ double div_unit(double a, double b) { return a / b; }
 // a row whose lanes' exponents are all at or below the splat's cut skips the exponential.
 // VALU bound. Against a loop that evaluated every row of every entry and reduced twelve sums per
 // splat with wave_reduce12: toy2d 1024^2, 200k splats 192 -> 104 us; phase0 1080p, 50k splats
-// 247 -> 140 us without the counts, 572 -> 146 + 6.5 us with them.
+// 247 -> 149 us without the counts, 572 -> 150 + 6.5 us with them.
 // kCount: the bucket's reduced steps and its splat-pixel evaluations (a pixel evaluates every list
 // entry up to its stop) are added, as integers, to slots 9 and 10 of its first splat's gradient
 // record, which fold_counts_kernel sums and clears: one counter that every wavefront adds to costs
@@ -1360,26 +1411,9 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
   }
   wave_sync();
 
-  const int slot = lane == 0    ? 0
-                   : lane == 1  ? 1
-                   : lane == 8  ? 2
-                   : lane == 9  ? 3
-                   : lane == 16 ? 5
-                   : lane == 17 ? 4
-                   : lane == 32 ? 6
-                   : lane == 33 ? 7
-                   : lane == 49 ? 8
-                                : -1;
+  const Owner2D own = owner2d<R>(lane);
+  const int slot = own.slot, pair = own.pair;
   const bool owner = slot >= 0;
-  // the lane's coefficient pair within a staged splat
-  const int pair = lane == 0    ? 0
-                   : lane == 1  ? 1
-                   : lane == 8  ? 2
-                   : lane == 9  ? 3
-                   : lane == 16 ? 4
-                   : lane == 17 ? 5
-                   : lane == 32 ? 6
-                                : 7;
   const bool row0 = lane < 16;
   uint32_t steps = 0;  // reduced splats (scalar)
   for (int j = 0; j < jmax; ++j) {
@@ -1398,14 +1432,16 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
       k1 = s1 * dx;
     }
     S sh = S(0), shy = S(0), shyy = S(0), cr = S(0), cg = S(0), cb = S(0);
+    S sha = S(0), shay = S(0);  // (phase0; there shy and shyy sum h b and h b dy)
     uint64_t used = 0;
 #pragma unroll
     for (int r = 0; r < kPixPerLane; ++r) {
       if (((plane[r] >> j) & 1u) == 0u || j >= lim_row[r]) continue;  // wave-uniform
-      S dy, power;
+      S dy, power, pa, pb;
       if constexpr (R == kRulesPhase0) {
         dy = pyf[r] - my;
-        const S pa = k0 + s1 * dy, pb = s2 * dy;
+        pa = k0 + s1 * dy;
+        pb = s2 * dy;
         power = S(-0.5) * (pa * pa + pb * pb);
       } else {
         dy = my - pyf[r];
@@ -1429,7 +1465,15 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
         const S oma = S(1) - alpha;
         const S dLda = T[r] * dot - div_unit(rho[r], oma);
         const S h = clamped ? S(0) : alpha * dLda;  // dL/dpower
-        const S hy = h * dy;
+        S hy;
+        if constexpr (R == kRulesPhase0) {
+          const S ha = h * pa;
+          sha += ha;
+          shay = fma(ha, dy, shay);
+          hy = h * pb;
+        } else {
+          hy = h * dy;
+        }
         sh += h;
         shy += hy;
         shyy = fma(hy, dy, shyy);
@@ -1441,12 +1485,11 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
     if (used == 0) continue;  // wave-uniform
     ++steps;
     S u0, u1;
-    wave_reduce_cols(sh, shy, shyy, cr, cg, cb, dx, row0, u0, u1);
-    S g = fma(-sp.co[2 * pair], u0, -(sp.co[2 * pair + 1] * u1));
-    if constexpr (R == kRulesPhase0) {
-      const S uyy = read_lane16(u1);  // sum h dy^2
-      if (lane == 9) g = fma(-s1, uyy, g);
-    }
+    if constexpr (R == kRulesPhase0)
+      wave_reduce_cols_chol(sha, shay, shy, shyy, sh, cr, cg, cb, dx, row0, u0, u1);
+    else
+      wave_reduce_cols(sh, shy, shyy, cr, cg, cb, dx, row0, u0, u1);
+    const S g = fma(-sp.co[2 * pair], u0, -(sp.co[2 * pair + 1] * u1));
     if (owner) atomic_add_grad(a.grad_rec + static_cast<int64_t>(s_id[j]) * kGrad2D + slot, g);
   }
   if constexpr (kCount) {

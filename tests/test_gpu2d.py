@@ -548,3 +548,57 @@ def test_blend2d_edge_splats_against_oracle(rules, dtype):
                                 counters=ctr)
         assert rel(g[:, :9], g_ref[:, :9]) < (1e-4 if dtype == np.float32 else 1e-9)
         assert int(ctr[0]) == atomics and int(ctr[2]) == ref["evals"]
+
+
+def phase0_single(p, W, H, gi, mask, dtype):
+    """Gradients of one phase0 splat of opacity 1/2 on its own (mean, shape), pixel by pixel in dtype:
+    h = alpha dL/dalpha, a = l0 dx + l1 dy and b = l2 dy formed at each pixel, then sums of h a, h b,
+    h a dx, h a dy, h b dy."""
+    mx, my, l0, l1, l2, *color = [dtype(x) for x in p]
+    y, x = np.nonzero(mask)
+    dx, dy = x.astype(dtype) + dtype(0.5) - mx, y.astype(dtype) + dtype(0.5) - my
+    a, b = l0 * dx + l1 * dy, l2 * dy
+    alpha = dtype(0.5) * np.exp(dtype(-0.5) * (a * a + b * b))
+    h = alpha * (gi[y, x].astype(dtype) * np.array(color, dtype)).sum(1)
+    ha, hb = h * a, h * b
+    u = ha.sum()
+    return (np.array([l0 * u, l1 * u + l2 * hb.sum()]),
+            -np.array([(ha * dx).sum(), (ha * dy).sum(), (hb * dy).sum()]))
+
+
+@pytest.mark.parametrize("dtype,exact", [(np.float32, np.float64), (np.float64, np.longdouble)])
+@pytest.mark.parametrize("s1,s2", [(2, 10), (1, 30), (0.6, 60), (1, 100)])
+def test_phase0_backward_of_rotated_splats(s1, s2, dtype, exact):
+    """Rotated elongated splats, each alone in its image: along such a splat l0 dx and l1 dy cancel in
+    a, so sums over the pixels of anything without a as a factor are far larger than the gradients.
+    The error per splat, root mean square over 24 of them, is that of the plain sums in the same
+    type (phase0_single), which are as many additions in another order, and of two roundings of a
+    pixel's dL/dalpha that those lack: the kernel's own exponential (within an ulp of its result) and
+    the term of the colours behind the splat (zero here but for its rounding; alpha <= 1/2). Three
+    errors of the plain sums' size at most, and two roundings for the final products."""
+    W = H = 208
+    rng = np.random.default_rng(int(10 * s1 + s2))
+    T = (W // 16) * (H // 16)
+    err = []
+    for k in range(24):
+        th = np.deg2rad(rng.uniform(15, 75)) * (1 if k % 2 else -1)
+        c, s, ia, ib = np.cos(th), np.sin(th), 1 / s1 ** 2, 1 / s2 ** 2
+        A, B, C = c * c * ia + s * s * ib, c * s * (ia - ib), s * s * ia + c * c * ib
+        l0 = np.sqrt(A)
+        p = np.array([*rng.uniform(90, 118, 2), l0, B / l0, np.sqrt(C - B * B / A), *rng.uniform(0.2, 1, 3)], dtype)
+        gi = rng.uniform(0, 1, (H, W, 3)).astype(dtype)
+        t = [cuda(x) for x in (p[None, :2], p[None, 2:5], p[None, 5:], np.zeros(1, dtype))]
+        rec = R2.pack(R2.PHASE0, *t)
+        toff, ids = torch.arange(T + 1, dtype=torch.int32, device="cuda"), torch.zeros(T, dtype=torch.int32, device="cuda")
+        image, _, nc, last, tmax, ckpt = R2.blend_fwd(R2.PHASE0, rec, toff, 1, ids, toff, T, W, H)
+        g = R2.blend_bwd_bucket(R2.PHASE0, rec, toff, 1, ids, toff, toff[:T].contiguous(), T, W, H, image, cuda(gi), last,
+                                tmax, ckpt)
+        mask = nc.cpu().numpy() > 0
+        got = [x.cpu().numpy()[0] for x in R2.split_grads(g)[:2]]
+        ref, plain = phase0_single(p, W, H, gi, mask, exact), phase0_single(p, W, H, gi, mask, dtype)
+        err.append([[float(np.linalg.norm((x - r).astype(exact).astype(float)) / np.linalg.norm(r.astype(float)))
+                     for x, r in zip(q, ref)] for q in (got, plain)])
+    e, e_plain = np.sqrt(np.mean(np.square(err), 0))
+    print(f"phase0 {s1}:{s2} {dtype.__name__}: mean {e[0]:.2e} (plain {e_plain[0]:.2e}), shape {e[1]:.2e} "
+          f"(plain {e_plain[1]:.2e})")
+    assert (e <= 3 * e_plain + 2 * np.finfo(dtype).eps).all()
