@@ -40,6 +40,7 @@ GS_FLOAT32, GS_FLOAT64, GS_BFLOAT16 = 0, 1, 2
 GS_CAM_PROPER_ANTIALIASING = 1  # gs_camera.flags bit
 GS_BIN_SPANS, GS_BIN_RADIX = 2, 4  # binning path forced (gs_camera.flags, rect flags)
 GS_BIN_TILES_KNOWN = 8  # gs_bin_fill_rect after gs_rect_tiles_begin
+RECT_TILES_OTHER = (1 << 64) - 1  # gs_rect_tiles_end's bucket count: the counts are not the rectangles' own
 BIN_FLAGS = {"auto": 0, "spans": GS_BIN_SPANS, "radix": GS_BIN_RADIX}
 GS_BIN_PATH_RADIX, GS_BIN_PATH_SPANS = 0, 1  # gs_bin_path
 GS_VIEW_BACKWARD, GS_VIEW_KEYS, GS_VIEW_NO_IMAGE = 1, 2, 4  # gs_view_* flags
@@ -95,7 +96,7 @@ _SIGS = {
                                 _sz, _vp]),
     "gs_rect_tiles_fit": (_i32, [_i32, _i32]),
     "gs_rect_tiles_workspace_size": (_sz, [_i64, _i32, _i32]),
-    "gs_rect_tiles_begin": (_i32, [_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "gs_rect_tiles_begin": (_i32, [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _sz, _vp]),
     "gs_rect_tiles_end": (_i32, [C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
     "gs_bucket_fill": (_i32, [_vp, _i32, _vp, _i64, _vp]),
     "gs_blend_fwd_3d": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, C.POINTER(C.c_float), _vp, _vp, _vp, _vp, _vp, _vp, _vp,

@@ -86,8 +86,10 @@ def _host_sum(p: int, n: int, st) -> int:
 def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | None, width: int, height: int,
               want_order: bool = False, binning: str | None = None, want_tile_offsets: bool = True) -> RectBins:
     """Per-tile lists of the Gaussians whose tile rectangle covers the tile, in stable depth
-    order (depth given) or index order. One host read, of the instance and bucket counts, before
-    the sort is enqueued (two, the second after it, on canvases beyond gs_rect_tiles_fit).
+    order (depth given) or index order. counts: the tiles that each rectangle covers (int32 [n]), or
+    0 to leave a Gaussian out. One host read, of the instance and bucket counts, before the sort is
+    enqueued (two, the second after it, on canvases beyond gs_rect_tiles_fit or where the counts
+    leave Gaussians out).
     binning: "auto", "spans" or "radix" (default: the module's BINNING); the lists are the same."""
     flags = _lib.BIN_FLAGS[binning or BINNING]
     dev = rects.device
@@ -101,13 +103,14 @@ def bin_rects(rects: torch.Tensor, counts: torch.Tensor, depth: torch.Tensor | N
     m, nb = 0, None
     if n > 0 and _lib.lib().gs_rect_tiles_fit(tx, ty):
         ws = _u8(_lib.size_call("gs_rect_tiles_workspace_size", n, tx, ty), dev)
-        call("gs_rect_tiles_begin", ptr(rects), n, tx, ty, ranges.data_ptr(), ptr(tile_offsets), boff.data_ptr(),
-             ws.data_ptr(), ws.numel(), st)
+        call("gs_rect_tiles_begin", ptr(rects), ptr(counts), n, tx, ty, ranges.data_ptr(), ptr(tile_offsets),
+             boff.data_ptr(), ws.data_ptr(), ws.numel(), st)
         mv, bv = C.c_uint64(), C.c_uint64()
         call("gs_rect_tiles_end", C.byref(mv), C.byref(bv))
-        m, nb = int(mv.value), int(bv.value)
-        flags |= _lib.GS_BIN_TILES_KNOWN
-    elif n > 0:
+        if bv.value != _lib.RECT_TILES_OTHER:
+            m, nb = int(mv.value), int(bv.value)
+            flags |= _lib.GS_BIN_TILES_KNOWN
+    if n > 0 and nb is None:
         m = _host_sum(ptr(counts), n, st)
     point_list = torch.empty(m, dtype=torch.int32, device=dev)
     order = torch.empty(n, dtype=torch.int32, device=dev) if want_order else None

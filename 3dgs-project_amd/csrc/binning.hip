@@ -1548,43 +1548,55 @@ __global__ __launch_bounds__(kBoThreads) void tile_scan_kernel(const uint32_t* _
 // prefix sum is the count of every tile. With the counts the ranges, the bucket offsets and both
 // totals are known before the instances are sorted, so the host waits once, for these small
 // kernels, instead of twice, the second time for the whole sort (and the sort takes no ranges).
-// rect_diff_kernel: G workgroups each leave their rectangles' array in part[g]; rect_tiles_kernel
-// (one workgroup) sums them (G = 0: takes all rectangles itself), scans and stores the totals to
-// host memory.
+// rect_diff_kernel: G workgroups each leave their rectangles' array in part[g]; its last word, after
+// the corners, is not 0 where one of a caller's counts (may be NULL) is not its rectangle's own --
+// Gaussians left out by a count of 0, say: the emission goes by the counts, so these ranges would not
+// be those of its instances. rect_tiles_kernel (one workgroup) sums the arrays (G = 0: takes all
+// rectangles itself), scans and stores the totals to host memory, or kDiffOther in place of the bucket
+// count where that word is set.
 constexpr int kDiffThreads = 1024;
 constexpr int64_t kDiffMax = 16000;       // array entries (below 64 KB of LDS): canvases up to 2000 x 2000
 constexpr int64_t kDiffDirect = 8192;     // rectangles one workgroup takes alone
 constexpr int64_t kDiffPer = 16384;       // rectangles per workgroup beyond
 constexpr int kDiffGroups = 8;
+constexpr unsigned long long kDiffOther = ~0ull;
 
-__device__ __forceinline__ void rect_diff_add(const int4* __restrict__ rects, int64_t lo, int64_t hi, int tiles_x,
-                                              int tiles_y, int* s_d) {
+__device__ __forceinline__ void rect_diff_add(const int4* __restrict__ rects, const uint32_t* __restrict__ counts,
+                                             int64_t lo, int64_t hi, int tiles_x, int tiles_y, int* s_d) {
   const int w = tiles_x + 1, n_d = w * (tiles_y + 1);
-  for (int q = threadIdx.x; q < n_d; q += kDiffThreads) s_d[q] = 0;
+  for (int q = threadIdx.x; q <= n_d; q += kDiffThreads) s_d[q] = 0;
   __syncthreads();
+  uint32_t other = 0;
   for (int64_t i = lo + threadIdx.x; i < hi; i += kDiffThreads) {
+    const uint32_t given = counts ? counts[i] : 0u;  // (loaded beside the rectangle, not after it)
     const int4 r = clamp_rect(rects[i], tiles_x, tiles_y);
-    if (r.z > r.x && r.w > r.y) {
+    const uint32_t own = r.z > r.x && r.w > r.y ? static_cast<uint32_t>((r.z - r.x) * (r.w - r.y)) : 0u;
+    other |= given ^ own;
+    if (own) {
       atomicAdd(&s_d[r.y * w + r.x], 1);
       atomicAdd(&s_d[r.y * w + r.z], -1);
       atomicAdd(&s_d[r.w * w + r.x], -1);
       atomicAdd(&s_d[r.w * w + r.z], 1);
     }
   }
+  if (counts && other) s_d[n_d] = 1;
   __syncthreads();
 }
 
-__global__ __launch_bounds__(kDiffThreads) void rect_diff_kernel(const int4* __restrict__ rects, int64_t n, int tiles_x,
-                                                                 int tiles_y, int* __restrict__ part) {
+__global__ __launch_bounds__(kDiffThreads) void rect_diff_kernel(const int4* __restrict__ rects,
+                                                                 const uint32_t* __restrict__ counts, int64_t n,
+                                                                 int tiles_x, int tiles_y, int* __restrict__ part) {
   extern __shared__ __align__(16) int s_diff[];
   const int64_t per = (n + gridDim.x - 1) / gridDim.x, lo = per * blockIdx.x, hi = min(lo + per, n);
-  rect_diff_add(rects, lo, hi, tiles_x, tiles_y, s_diff);
+  rect_diff_add(rects, counts, lo, hi, tiles_x, tiles_y, s_diff);
   const int n_d = (tiles_x + 1) * (tiles_y + 1);
-  for (int q = threadIdx.x; q < n_d; q += kDiffThreads) part[static_cast<int64_t>(blockIdx.x) * n_d + q] = s_diff[q];
+  part += static_cast<int64_t>(blockIdx.x) * (n_d + 1);
+  for (int q = threadIdx.x; q <= n_d; q += kDiffThreads) part[q] = s_diff[q];
 }
 
 __global__ __launch_bounds__(kDiffThreads) void rect_tiles_kernel(
-    const int4* __restrict__ rects, int64_t n, const int* __restrict__ part, int G, int tiles_x, int tiles_y,
+    const int4* __restrict__ rects, const uint32_t* __restrict__ counts, int64_t n, const int* __restrict__ part, int G,
+    int tiles_x, int tiles_y,
     uint32_t* __restrict__ ranges, uint32_t* __restrict__ boff,
     uint32_t* __restrict__ tile_offsets, unsigned long long* __restrict__ host) {
   extern __shared__ __align__(16) int s_diff[];
@@ -1592,12 +1604,12 @@ __global__ __launch_bounds__(kDiffThreads) void rect_tiles_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int w = tiles_x + 1, n_d = w * (tiles_y + 1);
   if (G == 0) {
-    rect_diff_add(rects, 0, n, tiles_x, tiles_y, s_diff);
+    rect_diff_add(rects, counts, 0, n, tiles_x, tiles_y, s_diff);
   } else {
-    for (int q = tid; q < n_d; q += kDiffThreads) {
+    for (int q = tid; q <= n_d; q += kDiffThreads) {
       int v[kDiffGroups], sum = 0;  // (all loads in flight together)
 #pragma unroll
-      for (int g = 0; g < kDiffGroups; ++g) v[g] = g < G ? part[static_cast<int64_t>(g) * n_d + q] : 0;
+      for (int g = 0; g < kDiffGroups; ++g) v[g] = g < G ? part[static_cast<int64_t>(g) * (n_d + 1) + q] : 0;
 #pragma unroll
       for (int g = 0; g < kDiffGroups; ++g) sum += v[g];
       s_diff[q] = sum;
@@ -1638,7 +1650,7 @@ __global__ __launch_bounds__(kDiffThreads) void rect_tiles_kernel(
   if (tid == 0) {
     for (int q = 1; q < kDiffThreads / kWave; ++q) m += s_m[q];
     host[0] = m;
-    host[1] = boff[tiles_x * tiles_y];  // (written by this thread)
+    host[1] = s_diff[n_d] ? kDiffOther : boff[tiles_x * tiles_y];  // (the last written by this thread)
   }
 }
 
@@ -2267,12 +2279,13 @@ extern "C" int gs_rect_tiles_fit(int tiles_x, int tiles_y) {
 
 extern "C" size_t gs_rect_tiles_workspace_size(int64_t n, int tiles_x, int tiles_y) {
   if (!gs_rect_tiles_fit(tiles_x, tiles_y)) return 0;
-  return n > kDiffDirect ? align_up(static_cast<size_t>(kDiffGroups) * (tiles_x + 1) * (tiles_y + 1) * 4) : 0;
+  const size_t words = static_cast<size_t>(tiles_x + 1) * (tiles_y + 1) + 1;
+  return n > kDiffDirect ? align_up(kDiffGroups * words * 4) : 0;
 }
 
-extern "C" int gs_rect_tiles_begin(const int32_t* rects, int64_t n, int tiles_x, int tiles_y, uint32_t* ranges,
-                                   uint32_t* tile_offsets, uint32_t* bucket_offsets, void* workspace,
-                                   size_t workspace_bytes, void* stream) {
+extern "C" int gs_rect_tiles_begin(const int32_t* rects, const uint32_t* counts, int64_t n, int tiles_x, int tiles_y,
+                                   uint32_t* ranges, uint32_t* tile_offsets, uint32_t* bucket_offsets,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   GS_REQUIRE(n >= 0 && gs_rect_tiles_fit(tiles_x, tiles_y), GS_ERR_ARG, "invalid rect_tiles sizes (n=%lld, %d x %d)",
              static_cast<long long>(n), tiles_x, tiles_y);
@@ -2286,14 +2299,15 @@ extern "C" int gs_rect_tiles_begin(const int32_t* rects, int64_t n, int tiles_x,
   hipStream_t st = as_stream(stream);
   int* part = static_cast<int*>(workspace);
   const int4* r4 = reinterpret_cast<const int4*>(rects);
-  const size_t lds = static_cast<size_t>(tiles_x + 1) * (tiles_y + 1) * 4;
+  const size_t lds = (static_cast<size_t>(tiles_x + 1) * (tiles_y + 1) + 1) * 4;
   int G = 0;
   if (n > kDiffDirect) {
     G = static_cast<int>(std::min<int64_t>((n + kDiffPer - 1) / kDiffPer, kDiffGroups));
-    hipLaunchKernelGGL(rect_diff_kernel, dim3(G), dim3(kDiffThreads), lds, st, r4, n, tiles_x, tiles_y, part);
+    hipLaunchKernelGGL(rect_diff_kernel, dim3(G), dim3(kDiffThreads), lds, st, r4, counts, n, tiles_x, tiles_y,
+                       part);
   }
-  hipLaunchKernelGGL(rect_tiles_kernel, dim3(1), dim3(kDiffThreads), lds, st, r4, n, part, G, tiles_x, tiles_y,
-                     ranges, bucket_offsets, tile_offsets, c->host_word);
+  hipLaunchKernelGGL(rect_tiles_kernel, dim3(1), dim3(kDiffThreads), lds, st, r4, counts, n, part, G, tiles_x,
+                     tiles_y, ranges, bucket_offsets, tile_offsets, c->host_word);
   if (int e = check_launch("rect_tiles_begin")) return e;
   if (hipEventRecord(c->done, st) != hipSuccess) return check_launch("rect_tiles_begin (event)");
   c->pending = true;

@@ -215,12 +215,14 @@ int gs_bin_fill_rect(const int32_t* rects, const void* depth, int depth_dtype, c
  * rectangles alone, before any instance is emitted, and the totals read back to the host as
  * gs_count_begin reads its count: gs_rect_tiles_begin enqueues the kernels, gs_rect_tiles_end (same
  * thread and device) waits for them and returns the instance count and the bucket count. The fill
- * then takes GS_BIN_TILES_KNOWN. For canvases with (tiles_x + 1)(tiles_y + 1) <= 16000
+ * then takes GS_BIN_TILES_KNOWN. counts (may be NULL): the counts that the fill is to be given; where
+ * one of them is not its rectangle's own (gs_rect_counts), the bucket count is UINT64_MAX, and the
+ * fill is called without GS_BIN_TILES_KNOWN and with m the sum of the counts. For canvases with (tiles_x + 1)(tiles_y + 1) <= 16000
  * (gs_rect_tiles_fit). Workspace from gs_rect_tiles_workspace_size. */
 int gs_rect_tiles_fit(int tiles_x, int tiles_y);
 size_t gs_rect_tiles_workspace_size(int64_t n, int tiles_x, int tiles_y);
-int gs_rect_tiles_begin(const int32_t* rects, int64_t n, int tiles_x, int tiles_y, uint32_t* ranges,
-                        uint32_t* tile_offsets, uint32_t* bucket_offsets, void* workspace,
+int gs_rect_tiles_begin(const int32_t* rects, const uint32_t* counts, int64_t n, int tiles_x, int tiles_y,
+                        uint32_t* ranges, uint32_t* tile_offsets, uint32_t* bucket_offsets, void* workspace,
                         size_t workspace_bytes, void* stream);
 int gs_rect_tiles_end(uint64_t* m, uint64_t* n_buckets);
 

@@ -207,6 +207,33 @@ def test_rect_tiles_edges(tiles_x, tiles_y, n):
     test_rect_binning_matches_the_stable_sort(16 * tiles_x, 16 * tiles_y, n, 6, "radix")
 
 
+@pytest.mark.parametrize("W,H,n", [
+    (333, 250, 5_000),    # one workgroup takes the rectangles
+    (640, 480, 40_000),   # three of them
+    (2064, 2064, 5_000),  # tile counts after the emission
+])
+def test_rect_binning_leaves_out_what_has_a_count_of_zero(W, H, n):
+    """A Gaussian with a count of 0 is in no list, whatever its rectangle covers."""
+    rng = np.random.default_rng(n)
+    tiles_x, tiles_y = (W + 15) // 16, (H + 15) // 16
+    x0, y0 = rng.integers(0, tiles_x, n), rng.integers(0, tiles_y, n)
+    rects = np.stack([x0, y0, np.minimum(x0 + 3, tiles_x), np.minimum(y0 + 2, tiles_y)], 1).astype(np.int32)
+    depth = rng.random(n).astype(np.float32)
+    out = rng.random(n) < 0.3
+    dev = torch.device("cuda")
+    rd = torch.from_numpy(rects).to(dev)
+    counts = torch.empty(n, dtype=torch.int32, device=dev)
+    call("gs_rect_counts", ptr(rd), n, tiles_x, tiles_y, ptr(counts), _lib.stream_handle(dev))
+    counts[torch.from_numpy(out).to(dev)] = 0
+    rb = R2.bin_rects(rd, counts, torch.from_numpy(depth).to(dev), W, H, binning="radix")
+    rects[out] = 0
+    pl, ranges, boff = numpy_rect_binning(rects, depth, tiles_x, tiles_x * tiles_y)
+    assert np.array_equal(rb.point_list.cpu().numpy(), pl)
+    assert np.array_equal(rb.ranges.cpu().numpy().astype(np.int64), ranges)
+    assert np.array_equal(rb.tile_offsets.cpu().numpy().astype(np.int64), np.append(ranges[:, 0], len(pl)))
+    assert np.array_equal(rb.bucket_offsets.cpu().numpy().astype(np.int64), boff) and rb.num_buckets == boff[-1]
+
+
 @pytest.mark.parametrize("n,offset", [(0, 0), (1, 0), (3, 1), (4097, 0), (1_000_003, 1), (15_625, 0)])
 def test_sum_u32(n, offset):
     """gs_sum_u32 (the instance count of the 3D forward) against numpy's uint64 sum, over values up to
