@@ -2385,9 +2385,11 @@ extern "C" int gs_bin_fill_3d(const float* splat_rec, const uint32_t* depth_keys
   GS_REQUIRE(m == 0 || offsets || path == GS_BIN_PATH_SPANS, GS_ERR_ARG, "this fill emits instances: it needs the offsets");
   GS_REQUIRE(!(sorted_keys && m > 0 && !depth_keys), GS_ERR_ARG, "sorted_keys need depth_keys");
   GS_REQUIRE(aligned(splat_rec, 16), GS_ERR_ALIGN, "splat_rec must be 16-byte aligned");
+  // (a camera's flags say nothing about ranges: GS_BIN_TILES_KNOWN is the rectangle fill's)
   bin_emit(reinterpret_cast<const SplatRec*>(splat_rec), nullptr, depth_keys, k.dkey0, order,
            offsets, n, k.tiles_x,
-           k.tiles_y, m, sorted_keys, point_list, ranges, nullptr, bucket_offsets, bucket_list, cam->flags,
+           k.tiles_y, m, sorted_keys, point_list, ranges, nullptr, bucket_offsets, bucket_list,
+           cam->flags & ~GS_BIN_TILES_KNOWN,
            static_cast<char*>(workspace), as_stream(stream));
   return check_launch("bin_fill_3d");
 }

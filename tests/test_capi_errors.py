@@ -175,6 +175,33 @@ def test_fill_workspace_short_then_a_good_call():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m_zero", [False, True])
+def test_a_cameras_other_flag_bits_do_not_change_the_fill(m_zero):
+    """gs_bin_fill_3d writes ranges, bucket offsets and the bucket list's header whatever bits beyond the
+    GS_CAM_* and path ones gs_camera.flags holds (GS_BIN_TILES_KNOWN belongs to gs_bin_fill_rect)."""
+    from amdsplat import raster3d as R
+    from amdsplat import scenes
+
+    sc = scenes.small_scene(3000, 160, 120, seed=3, sh_coeffs=16)
+    fs = R.forward_pass(*[t.cuda().contiguous() for t in sc.params()], sc.cameras[0], sh_degree=3)
+    L = _lib.lib()
+    cc = type(fs.ccam).from_buffer_copy(fs.ccam)
+    cc.flags |= _lib.GS_BIN_TILES_KNOWN
+    n, m, T = fs.n, 0 if m_zero else fs.m, fs.cam.n_tiles
+    ws = torch.empty(L.gs_bin_fill_3d_workspace_size(n, m, cc), dtype=torch.uint8, device="cuda")
+    pl, ranges, boff, header = (torch.full((k,), -3, dtype=torch.int32, device="cuda") for k in (fs.m, 2 * T, T + 1, 4))
+    assert L.gs_bin_fill_3d(ptr(fs.rec), None, ptr(fs.order), ptr(fs.offsets), n, cc, m, None, ptr(pl), ptr(ranges),
+                            ptr(boff), ptr(header), ptr(ws), ws.numel(), None) == 0
+    torch.cuda.synchronize()
+    assert not bool(header.any())
+    if m_zero:
+        assert not bool(ranges.any()) and not bool(boff.any())
+    else:
+        assert torch.equal(pl, fs.point_list) and torch.equal(ranges.view(T, 2), fs.ranges)
+        assert torch.equal(boff, fs.bucket_offsets)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("side", [0, 1])
 def test_count_readback_pairs_and_sums(side):
     """gs_count_begin / gs_count_end: the sum of the counts on either stream; an end without a
