@@ -139,6 +139,9 @@ class _View:
         self.touched = self.image = self.alpha = None
         self.timings: dict = {}
         self._state = self._lists = self._grads = None
+        # the tiles' first buckets (for the backward), a tensor of their own: rasterize returns their last
+        # word, and a caller who keeps that keeps this table, not an arena
+        self.boff = None
         self.last_conic64 = None  # the float64 conic sums of the last backward
         self._soff, self._loff = _lib.ViewStateOffsets(), _lib.ViewListOffsets()
 
@@ -164,7 +167,7 @@ class _View:
 
     def bucket_offsets(self) -> torch.Tensor:
         T = self.cam.n_tiles
-        return self._s(_lib.VIEW_BUCKET_OFFSETS, T + 1, torch.int32, T + 1)
+        return self.boff if self.boff is not None else self._s(_lib.VIEW_BUCKET_OFFSETS, T + 1, torch.int32, T + 1)
 
     def state(self) -> "ForwardState":
         n, m, nb, T = self.n, self.m, self.n_buckets_max, self.cam.n_tiles
@@ -356,6 +359,7 @@ def _forward_rest(fs: _View, dev, st, tm, scratch, timing, keep_keys, scores):
         # the backward's screen gradients [n, 12] float32 and the elongated splats' float64 conic
         # sums [n, 4], one buffer that the forward blend's workgroups zero
         grads = fs._grads = torch.empty(n * (GRAD2D_FLOATS + 8), dtype=torch.float32, device=dev)
+        fs.boff = torch.empty(cam.n_tiles + 1, dtype=torch.int32, device=dev)
     if scores is None:
         fs.image = torch.empty(3, H, W, dtype=torch.float32, device=dev)
         fs.alpha = torch.empty(H, W, dtype=torch.float32, device=dev)
@@ -374,13 +378,14 @@ def _forward_rest(fs: _View, dev, st, tm, scratch, timing, keep_keys, scores):
     lists = fs._lists = _u8(sizes[0], dev)
     clear, n_clear = (ptr(grads), grads.numel()) if grads is not None else (None, 0)
     if scores is None and not keep_keys and not tm.enabled:
-        call("gs_view_finish", n, m, ccam, flags, fs._state.data_ptr(), lists.data_ptr(), ws.data_ptr(), ws.numel(), bg3,
-             fs.image.data_ptr(), fs.alpha.data_ptr(), clear, n_clear, st)
+        call("gs_view_finish", n, m, ccam, flags, fs._state.data_ptr(), lists.data_ptr(), ptr(fs.boff), ws.data_ptr(),
+             ws.numel(), bg3, fs.image.data_ptr(), fs.alpha.data_ptr(), clear, n_clear, st)
         return fs
     back = fs.for_backward
     rec = fs.state_ptr(_lib.VIEW_REC) if n else None
     point_list = fs.list_ptr(_lib.VIEW_POINT_LIST) if m else None
-    ranges, boff = fs.state_ptr(_lib.VIEW_RANGES), fs.state_ptr(_lib.VIEW_BUCKET_OFFSETS)
+    ranges = fs.state_ptr(_lib.VIEW_RANGES)
+    boff = fs.boff.data_ptr() if back else fs.state_ptr(_lib.VIEW_BUCKET_OFFSETS)
     blist = fs.list_ptr(_lib.VIEW_BUCKET_LIST) if back else None
     # the fill also clears the bucket list's header for the forward blend
     call("gs_bin_fill_3d", rec, scratch.data_ptr() if n else None, fs.state_ptr(_lib.VIEW_ORDER) if n else None,
@@ -479,8 +484,8 @@ def _backward(view: _View, means, log_scales, quats, opacity_logits, sh, grad_im
     grad2d, conic64 = _split_grads2d(grads, view.n)
     view.last_conic64 = conic64
     params, gs, outs = _backward_args(view, means, log_scales, quats, opacity_logits, sh)
-    call("gs_view_backward", *params, view.m, view.ccam, view._state.data_ptr(), view._lists.data_ptr(), ptr(view.touched),
-         ptr(view.image), ptr(grad_image), ptr(grad_alpha), ptr(grad2d), ptr(conic64),
+    call("gs_view_backward", *params, view.m, view.ccam, view._state.data_ptr(), view._lists.data_ptr(), ptr(view.boff),
+         ptr(view.touched), ptr(view.image), ptr(grad_image), ptr(grad_alpha), ptr(grad2d), ptr(conic64),
          _lib.GS_ABS_GRAD if abs_grad else 0, *outs, st)
     return *gs, grad2d
 

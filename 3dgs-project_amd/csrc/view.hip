@@ -8,7 +8,7 @@ namespace gs {
 
 static int64_t up256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
-// The regions of the state arena, in order (gs_view_state).
+// The regions of the state arena, in order (GS_VIEW_REC ...), and its size.
 static int64_t state_layout(int64_t n, const CamK& k, int flags, int64_t* off) {
   const int64_t T = static_cast<int64_t>(k.tiles_x) * k.tiles_y, P = static_cast<int64_t>(k.width) * k.height;
   const bool bwd = (flags & GS_VIEW_BACKWARD) != 0, image = !(flags & GS_VIEW_NO_IMAGE);
@@ -110,8 +110,8 @@ extern "C" int gs_view_begin(const float* means, const float* log_scales, const 
 }
 
 extern "C" int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, void* lists,
-                              void* workspace, size_t workspace_bytes, const float* bg, float* image, float* alpha,
-                              float* clear, int64_t clear_floats, void* stream) {
+                              uint32_t* bucket_offsets, void* workspace, size_t workspace_bytes, const float* bg,
+                              float* image, float* alpha, float* clear, int64_t clear_floats, void* stream) {
   clear_error();
   if (int e = check_cam(cam)) return e;
   GS_REQUIRE(state && lists && !(flags & (GS_VIEW_NO_IMAGE | GS_VIEW_KEYS)), GS_ERR_ARG, "invalid view_finish arguments");
@@ -127,7 +127,7 @@ extern "C" int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int fl
   uint32_t* offsets = gs_bin_path(n, cam) == GS_BIN_PATH_SPANS ? nullptr : u32(st + so[GS_VIEW_OFFSETS]);
   uint32_t* point_list = m ? u32(li + lo[GS_VIEW_POINT_LIST]) : nullptr;
   uint32_t* ranges = u32(st + so[GS_VIEW_RANGES]);
-  uint32_t* boff = u32(st + so[GS_VIEW_BUCKET_OFFSETS]);
+  uint32_t* boff = bucket_offsets ? bucket_offsets : u32(st + so[GS_VIEW_BUCKET_OFFSETS]);
   uint32_t* blist = bwd ? u32(li + lo[GS_VIEW_BUCKET_LIST]) : nullptr;
   if (int e = gs_bin_fill_3d(rec, nullptr, u32(st + so[GS_VIEW_ORDER]), offsets, n, cam, m, nullptr, point_list, ranges,
                              boff, blist, workspace, workspace_bytes, stream))
@@ -144,8 +144,9 @@ extern "C" int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int fl
 extern "C" int gs_view_backward(const float* means, const float* log_scales, const float* quats,
                                 const float* opacity_logits, const float* sh, const float* sh_rest, int64_t n,
                                 int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state, void* lists,
-                                const uint32_t* tiles_touched, const float* image, const float* grad_image,
-                                const float* grad_alpha, float* grad2d, double* grad_conic64, int flags,
+                                const uint32_t* bucket_offsets, const uint32_t* tiles_touched, const float* image,
+                                const float* grad_image, const float* grad_alpha, float* grad2d, double* grad_conic64,
+                                int flags,
                                 float* grad_means, float* grad_log_scales, float* grad_quats,
                                 float* grad_opacity_logits, float* grad_sh, float* grad_sh_rest, void* stream) {
   clear_error();
@@ -159,7 +160,8 @@ extern "C" int gs_view_backward(const float* means, const float* log_scales, con
   char* li = static_cast<char*>(lists);
   const auto u32 = [](char* p) { return reinterpret_cast<uint32_t*>(p); };
   if (int e = gs_blend_bwd_3d(n ? reinterpret_cast<float*>(st + so[GS_VIEW_REC]) : nullptr, u32(st + so[GS_VIEW_RANGES]),
-                              m ? u32(li + lo[GS_VIEW_POINT_LIST]) : nullptr, u32(st + so[GS_VIEW_BUCKET_OFFSETS]),
+                              m ? u32(li + lo[GS_VIEW_POINT_LIST]) : nullptr,
+                              bucket_offsets ? bucket_offsets : u32(st + so[GS_VIEW_BUCKET_OFFSETS]),
                               sizes[2] ? u32(li + lo[GS_VIEW_BUCKET_TO_TILE]) : nullptr, sizes[2], n, k.width, k.height,
                               image, grad_image, reinterpret_cast<float*>(st + so[GS_VIEW_FINAL_T]), grad_alpha,
                               reinterpret_cast<int32_t*>(st + so[GS_VIEW_N_CONTRIB]), u32(st + so[GS_VIEW_TILE_MAX]),

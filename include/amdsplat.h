@@ -335,6 +335,9 @@ int gs_preprocess_bwd(const float* means, const float* log_scales, const float* 
  * gs_view_finish: gs_bin_fill_3d and gs_blend_fwd_3d (flags 0 or GS_VIEW_BACKWARD).
  * gs_view_backward: gs_blend_bwd_3d (flags: GS_ABS_GRAD; it adds to grad2d and grad_conic64, which
  *   start from zeros) and gs_preprocess_bwd, after a forward with GS_VIEW_BACKWARD.
+ * bucket_offsets (may be NULL: GS_VIEW_BUCKET_OFFSETS of the state arena) [T+1]: memory of the caller's
+ *   for the tiles' first buckets, for one that keeps the bucket count longer than the arenas; the
+ *   backward is given the forward's.
  * Both arenas and the scratch are 256-byte aligned.
  * ------------------------------------------------------------------------------------- */
 enum { GS_VIEW_BACKWARD = 1, GS_VIEW_KEYS = 2, GS_VIEW_NO_IMAGE = 4 };
@@ -354,14 +357,14 @@ int gs_view_begin(const float* means, const float* log_scales, const float* quat
 int gs_view_plan_count(int64_t n, int64_t m, const gs_camera* cam, int flags, int64_t* list_offsets,
                        int64_t* sizes);
 int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, void* lists,
-                   void* workspace, size_t workspace_bytes, const float* bg, float* image, float* alpha,
-                   float* clear, int64_t clear_floats, void* stream);
+                   uint32_t* bucket_offsets, void* workspace, size_t workspace_bytes, const float* bg,
+                   float* image, float* alpha, float* clear, int64_t clear_floats, void* stream);
 int gs_view_backward(const float* means, const float* log_scales, const float* quats,
                      const float* opacity_logits, const float* sh, const float* sh_rest, int64_t n,
                      int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state, void* lists,
-                     const uint32_t* tiles_touched, const float* image, const float* grad_image,
-                     const float* grad_alpha, float* grad2d, double* grad_conic64, int flags, float* grad_means,
-                     float* grad_log_scales, float* grad_quats, float* grad_opacity_logits, float* grad_sh,
+                     const uint32_t* bucket_offsets, const uint32_t* tiles_touched, const float* image,
+                     const float* grad_image, const float* grad_alpha, float* grad2d, double* grad_conic64, int flags,
+                     float* grad_means, float* grad_log_scales, float* grad_quats, float* grad_opacity_logits, float* grad_sh,
                      float* grad_sh_rest, void* stream);
 
 /* Densification statistics of one backward, accumulated into info [rows, n] (rows 2 or 3) for

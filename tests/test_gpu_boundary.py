@@ -309,6 +309,36 @@ def test_step_state_is_freed_without_the_cyclic_collector(surface):
 
 
 @gpu
+@pytest.mark.parametrize("timing", [False, True])
+def test_a_kept_aux_does_not_keep_the_forward_state(timing):
+    """What a caller may keep of aux beyond the backward, its bucket count, holds no more than the table
+    of the tiles' first buckets that it is a word of (not the records, orders and pixel states)."""
+    sc = scenes.small_scene(20_000, 333, 250, seed=5, sh_coeffs=16)
+    cam = sc.cameras[0]
+    leaves = [t.cuda().contiguous().requires_grad_(True) for t in faster_gs_params(sc)]
+    kept = []
+
+    def step():
+        m, ls, q, op, sh0, shr = leaves
+        img, _, aux = rasterize(m, ls, q, op, (sh0, shr), cam.viewmat, K_of(cam), cam.width, cam.height, near=cam.near,
+                                far=cam.far, timing=timing)
+        img.sum().backward()
+        kept.append(aux["n_buckets"])
+        for t in leaves:
+            t.grad = None
+
+    step()  # first call: workspace and allocator warm-up
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    for _ in range(4):
+        step()
+    torch.cuda.synchronize()
+    table = (4 * (((333 + 15) // 16) * ((250 + 15) // 16) + 1) + 511) // 512 * 512  # (the allocator's granularity)
+    assert torch.cuda.memory_allocated() - base <= 4 * table
+    assert len({int(b) for b in kept}) == 1 and int(kept[0]) > 0
+
+
+@gpu
 @pytest.mark.parametrize("binning", ["radix", "spans"])
 @pytest.mark.parametrize("n,W,H,split,behind", [
     (0, 64, 48, False, False),     # no Gaussians
