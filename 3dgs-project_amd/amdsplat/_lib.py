@@ -105,13 +105,13 @@ _SIGS = {
     "gs_blend_bwd_3d": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                _vp, _vp, _vp, _i32, _vp, _vp]),
     "gs_view_plan": (_i32, [_i64, C.POINTER(GsCamera), _i32, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
-    "gs_view_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, C.POINTER(GsCamera), _i32, _vp, _vp, _vp,
-                             _vp]),
+    "gs_view_begin": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, C.POINTER(GsCamera), _i32, _vp, _sz, _vp,
+                             _vp, _sz, _vp]),
     "gs_view_plan_count": (_i32, [_i64, _i64, C.POINTER(GsCamera), _i32, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
-    "gs_view_finish": (_i32, [_i64, _i64, C.POINTER(GsCamera), _i32, _vp, _vp, _vp, _vp, _sz, C.POINTER(C.c_float), _vp,
-                              _vp, _vp, _i64, _vp]),
-    "gs_view_backward": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i64, C.POINTER(GsCamera), _vp, _vp, _vp,
-                                _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "gs_view_finish": (_i32, [_i64, _i64, C.POINTER(GsCamera), _i32, _vp, _sz, _vp, _sz, _vp, _vp, _sz,
+                              C.POINTER(C.c_float), _vp, _vp, _vp, _i64, _vp]),
+    "gs_view_backward": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i64, C.POINTER(GsCamera), _vp, _sz,
+                                _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gs_preprocess_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, C.POINTER(GsCamera), _vp, _vp,
                                  _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gs_adam_step": (_i32, [C.POINTER(GsAdamGroup), _i32, _i64, _vp, _vp]),

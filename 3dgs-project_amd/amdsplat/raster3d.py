@@ -310,7 +310,8 @@ def _forward(means, log_scales, quats, opacity_logits, sh, cam: Camera, sh_degre
     # the count-dependent buffers without the stream draining first.
     one_call = n > 0 and not tm.enabled and not COUNT_ON_SIDE_STREAM
     if one_call:
-        call("gs_view_begin", *params, ccam, flags, state.data_ptr(), touched.data_ptr(), scratch.data_ptr(), st)
+        call("gs_view_begin", *params, ccam, flags, state.data_ptr(), state.numel(), touched.data_ptr(),
+             scratch.data_ptr(), scratch.numel(), st)
     else:
         held = _begin_stages(fs, params, scratch, tm, st)  # noqa: F841 (read until the count has ended)
     try:
@@ -378,8 +379,9 @@ def _forward_rest(fs: _View, dev, st, tm, scratch, timing, keep_keys, scores):
     lists = fs._lists = _u8(sizes[0], dev)
     clear, n_clear = (ptr(grads), grads.numel()) if grads is not None else (None, 0)
     if scores is None and not keep_keys and not tm.enabled:
-        call("gs_view_finish", n, m, ccam, flags, fs._state.data_ptr(), lists.data_ptr(), ptr(fs.boff), ws.data_ptr(),
-             ws.numel(), bg3, fs.image.data_ptr(), fs.alpha.data_ptr(), clear, n_clear, st)
+        call("gs_view_finish", n, m, ccam, flags, fs._state.data_ptr(), fs._state.numel(), lists.data_ptr(),
+             lists.numel(), ptr(fs.boff), ws.data_ptr(), ws.numel(), bg3, fs.image.data_ptr(), fs.alpha.data_ptr(),
+             clear, n_clear, st)
         return fs
     back = fs.for_backward
     rec = fs.state_ptr(_lib.VIEW_REC) if n else None
@@ -484,9 +486,9 @@ def _backward(view: _View, means, log_scales, quats, opacity_logits, sh, grad_im
     grad2d, conic64 = _split_grads2d(grads, view.n)
     view.last_conic64 = conic64
     params, gs, outs = _backward_args(view, means, log_scales, quats, opacity_logits, sh)
-    call("gs_view_backward", *params, view.m, view.ccam, view._state.data_ptr(), view._lists.data_ptr(), ptr(view.boff),
-         ptr(view.touched), ptr(view.image), ptr(grad_image), ptr(grad_alpha), ptr(grad2d), ptr(conic64),
-         _lib.GS_ABS_GRAD if abs_grad else 0, *outs, st)
+    call("gs_view_backward", *params, view.m, view.ccam, view._state.data_ptr(), view._state.numel(),
+         view._lists.data_ptr(), view._lists.numel(), ptr(view.boff), ptr(view.touched), ptr(view.image),
+         ptr(grad_image), ptr(grad_alpha), ptr(grad2d), ptr(conic64), _lib.GS_ABS_GRAD if abs_grad else 0, *outs, st)
     return *gs, grad2d
 
 

@@ -2232,6 +2232,11 @@ static int count_side(CountSide** out) {
   return GS_OK;
 }
 
+int check_count() {
+  CountSide* c = nullptr;
+  return count_side(&c);
+}
+
 static int count_wait(uint64_t* m, uint64_t* second) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return check_launch("count_end (device)");

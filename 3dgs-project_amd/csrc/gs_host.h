@@ -25,6 +25,11 @@ void stage_mark(const char* name, hipStream_t st);
 // captured in a HIP graph).
 void fill_zero_f32(float* p, int64_t n, hipStream_t st);
 
+// Checks that calls of several stages make before they enqueue the first: the SH layout; whether this
+// thread and device can begin a count.
+int check_sh(int sh_coeffs, int sh_degree);
+int check_count();
+
 #define GS_REQUIRE(cond, code, ...) \
   do {                              \
     if (!(cond)) {                  \

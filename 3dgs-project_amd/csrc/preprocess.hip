@@ -814,13 +814,15 @@ static void launch_pre_bwd(int64_t blocks, hipStream_t st, const float* means, c
                      reinterpret_cast<float4*>(gq), gop, gsh);
 }
 
-static int check_sh(int sh_coeffs, int sh_degree) {
+namespace gs {
+int check_sh(int sh_coeffs, int sh_degree) {
   GS_REQUIRE(sh_coeffs == 1 || sh_coeffs == 4 || sh_coeffs == 9 || sh_coeffs == 16, GS_ERR_ARG,
              "sh_coeffs must be 1, 4, 9 or 16 (got %d)", sh_coeffs);
   GS_REQUIRE(sh_degree >= 0 && (sh_degree + 1) * (sh_degree + 1) <= sh_coeffs, GS_ERR_ARG,
              "sh_degree %d needs more than %d coefficients", sh_degree, sh_coeffs);
   return GS_OK;
 }
+}  // namespace gs
 
 extern "C" int gs_preprocess_fwd(const float* means, const float* log_scales, const float* quats,
                                  const float* opacity_logits, const float* sh, const float* sh_rest,

@@ -1,7 +1,8 @@
 // One 3D view in three calls: the stages' entry points (preprocess, count, depth order | fill,
 // forward blend | blend backward, preprocess backward) run in order over buffers that a caller
 // allocates as two arenas, so that a host program pays for two allocations and three calls per
-// view instead of about twenty of each. The stages and their checks are those of the entry points.
+// view instead of about twenty of each. The stages and their checks are those of the entry points;
+// what a later stage would refuse is refused before the first is enqueued.
 #include "gs_host.h"
 
 namespace gs {
@@ -40,6 +41,14 @@ static BeginScratch begin_scratch(int64_t n) {
   s.prep = s.waves + up256(4 * ((n + 63) / 64));
   s.end = s.prep + up256(static_cast<int64_t>(gs_bin_prepare_workspace_size(n)));
   return s;
+}
+
+static int check_arena(const void* p, size_t have, int64_t need, const char* name) {
+  GS_REQUIRE(p, GS_ERR_ARG, "null pointer argument (%s)", name);
+  GS_REQUIRE(aligned(p, 256), GS_ERR_ALIGN, "the %s must be 256-byte aligned", name);
+  GS_REQUIRE(have >= static_cast<size_t>(need), GS_ERR_WORKSPACE, "%s too small: need %lld bytes", name,
+             static_cast<long long>(need));
+  return GS_OK;
 }
 
 }  // namespace gs
@@ -82,14 +91,17 @@ extern "C" int gs_view_plan_count(int64_t n, int64_t m, const gs_camera* cam, in
 extern "C" int gs_view_begin(const float* means, const float* log_scales, const float* quats,
                              const float* opacity_logits, const float* sh, const float* sh_rest, int64_t n,
                              int sh_coeffs, int sh_degree, const gs_camera* cam, int flags, void* state,
-                             uint32_t* tiles_touched, void* scratch, void* stream) {
+                             size_t state_bytes, uint32_t* tiles_touched, void* scratch, size_t scratch_bytes,
+                             void* stream) {
   clear_error();
   if (int e = check_cam(cam)) return e;
-  GS_REQUIRE(n > 0 && n < (int64_t(1) << 32) && state && scratch, GS_ERR_ARG, "invalid view_begin arguments");
-  GS_REQUIRE(aligned(state, 256) && aligned(scratch, 256), GS_ERR_ALIGN, "state and scratch must be 256-byte aligned");
+  GS_REQUIRE(n > 0 && n < (int64_t(1) << 32), GS_ERR_ARG, "invalid view_begin arguments");
   int64_t off[GS_VIEW_STATE_REGIONS];
-  state_layout(n, make_cam(*cam), flags, off);
+  const int64_t need = state_layout(n, make_cam(*cam), flags, off);
   const BeginScratch s = begin_scratch(n);
+  if (int e = check_arena(state, state_bytes, need, "state arena")) return e;
+  if (int e = check_arena(scratch, scratch_bytes, s.end, "scratch")) return e;
+  if (int e = check_count()) return e;
   char* st = static_cast<char*>(state);
   char* sc = static_cast<char*>(scratch);
   const auto u32 = [](char* p) { return reinterpret_cast<uint32_t*>(p); };
@@ -109,16 +121,23 @@ extern "C" int gs_view_begin(const float* means, const float* log_scales, const 
   return GS_OK;
 }
 
-extern "C" int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, void* lists,
-                              uint32_t* bucket_offsets, void* workspace, size_t workspace_bytes, const float* bg,
-                              float* image, float* alpha, float* clear, int64_t clear_floats, void* stream) {
+extern "C" int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, size_t state_bytes,
+                              void* lists, size_t lists_bytes, uint32_t* bucket_offsets, void* workspace,
+                              size_t workspace_bytes, const float* bg, float* image, float* alpha, float* clear,
+                              int64_t clear_floats, void* stream) {
   clear_error();
   if (int e = check_cam(cam)) return e;
-  GS_REQUIRE(state && lists && !(flags & (GS_VIEW_NO_IMAGE | GS_VIEW_KEYS)), GS_ERR_ARG, "invalid view_finish arguments");
+  GS_REQUIRE(!(flags & (GS_VIEW_NO_IMAGE | GS_VIEW_KEYS)), GS_ERR_ARG, "invalid view_finish arguments");
   int64_t so[GS_VIEW_STATE_REGIONS], lo[GS_VIEW_LIST_REGIONS], sizes[3];
   const CamK k = make_cam(*cam);
-  state_layout(n, k, flags, so);
   if (int e = gs_view_plan_count(n, m, cam, flags, lo, sizes)) return e;
+  if (int e = check_arena(state, state_bytes, state_layout(n, k, flags, so), "state arena")) return e;
+  if (int e = check_arena(lists, lists_bytes, sizes[0], "list arena")) return e;
+  // (the blend's own checks, made before the fill is enqueued)
+  GS_REQUIRE(image, GS_ERR_ARG, "null pointer argument");
+  GS_REQUIRE(clear_floats >= 0 && clear_floats % 4 == 0 && (clear || clear_floats == 0), GS_ERR_ARG,
+             "clear must hold a multiple of 4 floats");
+  GS_REQUIRE(aligned(clear, 16), GS_ERR_ALIGN, "clear must be 16-byte aligned");
   char* st = static_cast<char*>(state);
   char* li = static_cast<char*>(lists);
   const auto u32 = [](char* p) { return reinterpret_cast<uint32_t*>(p); };
@@ -143,19 +162,28 @@ extern "C" int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int fl
 
 extern "C" int gs_view_backward(const float* means, const float* log_scales, const float* quats,
                                 const float* opacity_logits, const float* sh, const float* sh_rest, int64_t n,
-                                int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state, void* lists,
-                                const uint32_t* bucket_offsets, const uint32_t* tiles_touched, const float* image,
-                                const float* grad_image, const float* grad_alpha, float* grad2d, double* grad_conic64,
-                                int flags,
+                                int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state,
+                                size_t state_bytes, void* lists, size_t lists_bytes, const uint32_t* bucket_offsets,
+                                const uint32_t* tiles_touched, const float* image, const float* grad_image,
+                                const float* grad_alpha, float* grad2d, double* grad_conic64, int flags,
                                 float* grad_means, float* grad_log_scales, float* grad_quats,
                                 float* grad_opacity_logits, float* grad_sh, float* grad_sh_rest, void* stream) {
   clear_error();
   if (int e = check_cam(cam)) return e;
-  GS_REQUIRE(state && lists, GS_ERR_ARG, "invalid view_backward arguments");
+  if (int e = check_sh(sh_coeffs, sh_degree)) return e;
   int64_t so[GS_VIEW_STATE_REGIONS], lo[GS_VIEW_LIST_REGIONS], sizes[3];
   const CamK k = make_cam(*cam);
-  state_layout(n, k, GS_VIEW_BACKWARD, so);
   if (int e = gs_view_plan_count(n, m, cam, GS_VIEW_BACKWARD, lo, sizes)) return e;
+  if (int e = check_arena(state, state_bytes, state_layout(n, k, GS_VIEW_BACKWARD, so), "state arena")) return e;
+  if (int e = check_arena(lists, lists_bytes, sizes[0], "list arena")) return e;
+  // (the preprocess backward's own checks, made before the blend's is enqueued)
+  GS_REQUIRE(n == 0 || (means && log_scales && quats && opacity_logits && sh && tiles_touched && grad2d && grad_means &&
+                        grad_log_scales && grad_quats && grad_opacity_logits && grad_sh),
+             GS_ERR_ARG, "null pointer argument");
+  GS_REQUIRE(n == 0 || !sh_rest == !grad_sh_rest, GS_ERR_ARG, "sh_rest and grad_sh_rest go together");
+  GS_REQUIRE(n == 0 || !(sh_rest && sh_coeffs == 1), GS_ERR_ARG, "sh_rest given for a DC-only model");
+  GS_REQUIRE(n == 0 || (aligned(quats, 16) && aligned(grad_quats, 16)), GS_ERR_ALIGN,
+             "quats and grad_quats must be 16-byte aligned");
   char* st = static_cast<char*>(state);
   char* li = static_cast<char*>(lists);
   const auto u32 = [](char* p) { return reinterpret_cast<uint32_t*>(p); };

@@ -338,7 +338,8 @@ int gs_preprocess_bwd(const float* means, const float* log_scales, const float* 
  * bucket_offsets (may be NULL: GS_VIEW_BUCKET_OFFSETS of the state arena) [T+1]: memory of the caller's
  *   for the tiles' first buckets, for one that keeps the bucket count longer than the arenas; the
  *   backward is given the forward's.
- * Both arenas and the scratch are 256-byte aligned.
+ * Both arenas and the scratch are 256-byte aligned and given with their sizes (GS_ERR_WORKSPACE if one
+ * is smaller than the plan's).
  * ------------------------------------------------------------------------------------- */
 enum { GS_VIEW_BACKWARD = 1, GS_VIEW_KEYS = 2, GS_VIEW_NO_IMAGE = 4 };
 enum {
@@ -352,18 +353,20 @@ enum {
 int gs_view_plan(int64_t n, const gs_camera* cam, int flags, int64_t* state_offsets, int64_t* sizes);
 int gs_view_begin(const float* means, const float* log_scales, const float* quats, const float* opacity_logits,
                   const float* sh, const float* sh_rest, int64_t n, int sh_coeffs, int sh_degree,
-                  const gs_camera* cam, int flags, void* state, uint32_t* tiles_touched, void* scratch,
-                  void* stream);
+                  const gs_camera* cam, int flags, void* state, size_t state_bytes, uint32_t* tiles_touched,
+                  void* scratch, size_t scratch_bytes, void* stream);
 int gs_view_plan_count(int64_t n, int64_t m, const gs_camera* cam, int flags, int64_t* list_offsets,
                        int64_t* sizes);
-int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, void* lists,
-                   uint32_t* bucket_offsets, void* workspace, size_t workspace_bytes, const float* bg,
-                   float* image, float* alpha, float* clear, int64_t clear_floats, void* stream);
+int gs_view_finish(int64_t n, int64_t m, const gs_camera* cam, int flags, void* state, size_t state_bytes,
+                   void* lists, size_t lists_bytes, uint32_t* bucket_offsets, void* workspace,
+                   size_t workspace_bytes, const float* bg, float* image, float* alpha, float* clear,
+                   int64_t clear_floats, void* stream);
 int gs_view_backward(const float* means, const float* log_scales, const float* quats,
                      const float* opacity_logits, const float* sh, const float* sh_rest, int64_t n,
-                     int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state, void* lists,
-                     const uint32_t* bucket_offsets, const uint32_t* tiles_touched, const float* image,
-                     const float* grad_image, const float* grad_alpha, float* grad2d, double* grad_conic64, int flags,
+                     int sh_coeffs, int sh_degree, int64_t m, const gs_camera* cam, void* state,
+                     size_t state_bytes, void* lists, size_t lists_bytes, const uint32_t* bucket_offsets,
+                     const uint32_t* tiles_touched, const float* image, const float* grad_image,
+                     const float* grad_alpha, float* grad2d, double* grad_conic64, int flags,
                      float* grad_means, float* grad_log_scales, float* grad_quats, float* grad_opacity_logits, float* grad_sh,
                      float* grad_sh_rest, void* stream);
 

@@ -8,7 +8,8 @@ message (gs_last_error) and enqueues nothing; the Python surfaces raise.
 
   - Without a GPU (argument checks that come before anything touches the device): NULL
     pointers, negative or out-of-range sizes, unknown enums, invalid cameras, missing
-    workspaces. Only NULL pointers are passed, so nothing could be dereferenced.
+    workspaces. Only NULL pointers, or made-up addresses where a call is refused for an alignment or
+    a size, are passed, so nothing could be dereferenced.
   - With a GPU (marked `gpu`): a workspace one byte short and a misaligned pointer, each with
     real device buffers of the full size, checking that the outputs were not touched and that
     the next, valid call succeeds and is right; bad tensors at the Python surfaces.
@@ -114,6 +115,72 @@ def test_missing_workspace_is_refused():
     assert L.gs_bin_fill_3d_workspace_size(n, 5 * n, c) <= L.gs_bin_workspace_size(n, 5 * n, 40, 30, 0)
 
 
+BIG, ARENA, ODD = 1 << 40, 256, 256 + 16  # a size no plan reaches; an aligned and a misaligned address
+
+
+def view_calls(L, n=10, m=20, state=ARENA, state_bytes=BIG, lists=ARENA, lists_bytes=BIG, c=None, flags=1, image=None,
+               clear=(None, 0), coeffs=16, degree=3):
+    """gs_view_begin, _finish and _backward with made-up arenas and NULL everywhere else."""
+    c = cam() if c is None else c
+    return (lambda: L.gs_view_begin(None, None, None, None, None, None, n, coeffs, degree, c, flags, state, state_bytes,
+                                    None, lists, lists_bytes, None),
+            lambda: L.gs_view_finish(n, m, c, flags, state, state_bytes, lists, lists_bytes, None, None, 0, None, image,
+                                     None, *clear, None),
+            lambda: L.gs_view_backward(None, None, None, None, None, None, n, coeffs, degree, m, c, state, state_bytes,
+                                       lists, lists_bytes, None, None, None, None, None, None, None, 0, None, None, None,
+                                       None, None, None, None))
+
+
+def test_view_plans_refuse_bad_sizes():
+    L = _lib.lib()
+    off, loff, sizes = _lib.ViewStateOffsets(), _lib.ViewListOffsets(), _lib.ViewSizes()
+    for n in (-1, 1 << 32):
+        expect(L.gs_view_plan(n, cam(), 1, off, sizes), GS_ERR_ARG, "invalid view_plan arguments")
+    expect(L.gs_view_plan(5, cam(), 1, None, sizes), GS_ERR_ARG, "invalid view_plan arguments")
+    expect(L.gs_view_plan(5, cam(), 1, off, None), GS_ERR_ARG, "invalid view_plan arguments")
+    expect(L.gs_view_plan(5, cam(W=0), 1, off, sizes), GS_ERR_ARG, "image size")
+    for n, m in ((-1, 0), (0, -1), (5, 1 << 32)):
+        expect(L.gs_view_plan_count(n, m, cam(), 1, loff, sizes), GS_ERR_ARG, "invalid view_plan_count arguments")
+    expect(L.gs_view_plan_count(5, 5, cam(), 1, None, sizes), GS_ERR_ARG, "invalid view_plan_count arguments")
+    expect(L.gs_view_plan_count(5, 5, None, 1, loff, sizes), GS_ERR_ARG, "camera is NULL")
+
+
+def test_view_calls_refuse_bad_arenas():
+    """Sizes, alignments and NULLs of the arenas, one byte short of the plan's, and what the second stage
+    of a call would refuse."""
+    L = _lib.lib()
+    off, loff, sizes, lsizes = _lib.ViewStateOffsets(), _lib.ViewListOffsets(), _lib.ViewSizes(), _lib.ViewSizes()
+    assert L.gs_view_plan(10, cam(), 1, off, sizes) == 0 and L.gs_view_plan_count(10, 20, cam(), 1, loff, lsizes) == 0
+    for k, call in enumerate(view_calls(L, c=cam(near=0.0))):
+        expect(call(), GS_ERR_ARG, "near")
+    for call in view_calls(L, n=-1):
+        expect(call(), GS_ERR_ARG, "invalid view_")
+    for call in view_calls(L, m=1 << 32)[1:]:
+        expect(call(), GS_ERR_ARG, "invalid view_plan_count")
+    second = "scratch", "list arena", "list arena"  # (the helper's lists are gs_view_begin's scratch)
+    for name, call in zip(second, view_calls(L, lists=None)):
+        expect(call(), GS_ERR_ARG, f"null pointer argument ({name})")
+    for name, call in zip(second, view_calls(L, lists=ODD)):
+        expect(call(), GS_ERR_ALIGN, f"the {name} must be 256-byte aligned")
+    for name, need, call in zip(second, (sizes[1], lsizes[0], lsizes[0]),
+                                [view_calls(L, lists_bytes=b - 1)[k] for k, b in
+                                 enumerate((sizes[1], lsizes[0], lsizes[0]))]):
+        expect(call(), GS_ERR_WORKSPACE, f"{name} too small: need {need} bytes")
+    for call in view_calls(L, state=None):
+        expect(call(), GS_ERR_ARG, "null pointer argument (state arena)")
+    for call in view_calls(L, state=ODD):
+        expect(call(), GS_ERR_ALIGN, "the state arena must be 256-byte aligned")
+    for call in view_calls(L, state_bytes=sizes[0] - 1):
+        expect(call(), GS_ERR_WORKSPACE, f"state arena too small: need {sizes[0]} bytes")
+    for flags in (_lib.GS_VIEW_NO_IMAGE, _lib.GS_VIEW_KEYS | 1):
+        expect(view_calls(L, flags=flags)[1](), GS_ERR_ARG, "invalid view_finish arguments")
+    expect(view_calls(L)[1](), GS_ERR_ARG, "null pointer argument")  # the image
+    expect(view_calls(L, image=ARENA, clear=(ARENA, 6))[1](), GS_ERR_ARG, "a multiple of 4 floats")
+    expect(view_calls(L, image=ARENA, clear=(ARENA + 4, 8))[1](), GS_ERR_ALIGN, "clear must be 16-byte aligned")
+    expect(view_calls(L)[2](), GS_ERR_ARG, "null pointer argument")  # the parameters and gradients
+    expect(view_calls(L, coeffs=5)[2](), GS_ERR_ARG, "sh_coeffs must be 1, 4, 9 or 16")
+
+
 # ---------------------------------------------------------------------------------------
 # Device-side failures (real buffers of the full size; nothing may be written)
 # ---------------------------------------------------------------------------------------
@@ -172,6 +239,74 @@ def test_fill_workspace_short_then_a_good_call():
                             ptr(boff), None, ptr(ws), need, None) == 0
     torch.cuda.synchronize()
     assert torch.equal(pl, fs.point_list) and torch.equal(ranges, fs.ranges) and torch.equal(boff, fs.bucket_offsets)
+
+
+@pytest.mark.gpu
+def test_view_arenas_short_then_good_calls():
+    """gs_view_begin, _finish and _backward with an arena one byte short and without an output: refused,
+    nothing written, no count left pending; then the good calls give rasterize's image and gradients."""
+    from amdsplat import raster3d as R
+    from amdsplat import scenes
+
+    sc = scenes.small_scene(3000, 160, 120, seed=3, sh_coeffs=16)
+    c = sc.cameras[0]
+    p = [t.cuda().contiguous() for t in sc.params()]
+    W, H, n = c.width, c.height, p[0].shape[0]
+    L, cc = _lib.lib(), c.c_struct()
+    off, loff, sizes, lsizes = _lib.ViewStateOffsets(), _lib.ViewListOffsets(), _lib.ViewSizes(), _lib.ViewSizes()
+    byte = lambda k: torch.full((k,), 77, dtype=torch.uint8, device="cuda")
+    f32 = lambda *shape: torch.full(shape, -9.0, device="cuda")
+    untouched = lambda *ts: all(bool((t == t.flatten()[0]).all()) for t in ts)
+    assert L.gs_view_plan(n, cc, 1, off, sizes) == 0
+    state, scratch = byte(sizes[0]), byte(sizes[1])
+    touched = torch.full((n,), -9, dtype=torch.int32, device="cuda")
+    par = [ptr(t) for t in p] + [None]
+    begin = lambda a=0, b=0: L.gs_view_begin(*par, n, 16, 3, cc, 1, ptr(state), state.numel() - a, ptr(touched),
+                                             ptr(scratch), scratch.numel() - b, None)
+    expect(begin(a=1), GS_ERR_WORKSPACE, "state arena too small")
+    expect(begin(b=1), GS_ERR_WORKSPACE, "scratch too small")
+    torch.cuda.synchronize()
+    assert untouched(state, scratch, touched)
+    waves = torch.ones(4, dtype=torch.int32, device="cuda")
+    m = ctypes.c_uint64()
+    assert L.gs_count_begin(ptr(waves), 4, 0, None) == 0
+    expect(begin(), GS_ERR_ARG, "was not ended")  # another count is pending: nothing enqueued
+    assert L.gs_count_end(ctypes.byref(m)) == 0 and m.value == 4
+    torch.cuda.synchronize()
+    assert untouched(state, scratch, touched)
+    assert begin() == 0 and L.gs_count_end(ctypes.byref(m)) == 0
+    m = m.value
+    assert L.gs_view_plan_count(n, m, cc, 1, loff, lsizes) == 0
+    lists, ws = byte(lsizes[0]), byte(lsizes[1])
+    boff = torch.full((c.n_tiles + 1,), -9, dtype=torch.int32, device="cuda")
+    image, alpha, g2 = f32(3, H, W), f32(H, W), f32(n * 20)
+    finish = lambda a=0, b=0, im=image: L.gs_view_finish(
+        n, m, cc, 1, ptr(state), state.numel() - a, ptr(lists), lists.numel() - b, ptr(boff), ptr(ws), ws.numel(),
+        _lib.float3((0.1, 0.2, 0.3)), ptr(im), ptr(alpha), ptr(g2), g2.numel(), None)
+    expect(finish(a=1), GS_ERR_WORKSPACE, "state arena too small")
+    expect(finish(b=1), GS_ERR_WORKSPACE, "list arena too small")
+    expect(finish(im=None), GS_ERR_ARG, "null pointer")
+    torch.cuda.synchronize()
+    assert untouched(lists, ws, boff, image, alpha, g2)
+    assert finish() == 0
+    outs = [f32(n, 3), f32(n, 3), f32(n, 4), f32(n), f32(n, 16, 3)]
+    gi = torch.randn(3, H, W, generator=torch.Generator().manual_seed(1)).cuda()
+    backward = lambda a=0, b=0, last=outs[4]: L.gs_view_backward(
+        *par, n, 16, 3, m, cc, ptr(state), state.numel() - a, ptr(lists), lists.numel() - b, ptr(boff), ptr(touched),
+        ptr(image), ptr(gi), None, ptr(g2), ptr(g2) + 48 * n, 0, *[ptr(t) for t in outs[:4]], ptr(last), None, None)
+    expect(backward(a=1), GS_ERR_WORKSPACE, "state arena too small")
+    expect(backward(b=1), GS_ERR_WORKSPACE, "list arena too small")
+    expect(backward(last=None), GS_ERR_ARG, "null pointer")
+    torch.cuda.synchronize()
+    assert untouched(*outs) and not bool(g2.any())  # (the forward's zeros)
+    assert backward() == 0
+    leaves = [t.clone().requires_grad_(True) for t in p]
+    K = torch.tensor([[c.fx, 0.0, c.cx], [0.0, c.fy, c.cy], [0.0, 0.0, 1.0]])
+    ref, ref_alpha, aux = R.rasterize(*leaves, c.viewmat, K, W, H, near=c.near, far=c.far, bg=(0.1, 0.2, 0.3))
+    ref.backward(gi)
+    assert aux["n_instances"] == m and torch.equal(ref, image) and torch.equal(ref_alpha, alpha)
+    for t, x in zip(leaves, outs):  # two orders of float32 sums of at most 256 * 16 terms per value and tile
+        assert float((t.grad - x).norm()) <= 1e-5 * float(t.grad.norm())
 
 
 @pytest.mark.gpu
