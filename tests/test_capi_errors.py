@@ -181,6 +181,37 @@ def test_view_calls_refuse_bad_arenas():
     expect(view_calls(L, coeffs=5)[2](), GS_ERR_ARG, "sh_coeffs must be 1, 4, 9 or 16")
 
 
+def test_rect_tiles_refuse_bad_arguments():
+    L = _lib.lib()
+    m, b = ctypes.c_uint64(), ctypes.c_uint64()
+    assert not L.gs_rect_tiles_fit(0, 4) and not L.gs_rect_tiles_fit(126, 126) and L.gs_rect_tiles_fit(124, 127)
+    n = 100_000  # (several workgroups: a workspace)
+    need = L.gs_rect_tiles_workspace_size(n, 40, 30)
+    assert need > 0 and L.gs_rect_tiles_workspace_size(n, 126, 126) == 0
+    begin = lambda n=n, tx=40, ty=30, rects=ARENA, ranges=ARENA, boff=ARENA, ws=ARENA, size=need: L.gs_rect_tiles_begin(
+        rects, None, n, tx, ty, ranges, None, boff, ws, size, None)
+    for kw in (dict(n=-1), dict(tx=0), dict(tx=126, ty=126)):
+        expect(begin(**kw), GS_ERR_ARG, "invalid rect_tiles sizes")
+    for kw in (dict(rects=None), dict(ranges=None), dict(boff=None)):
+        expect(begin(**kw), GS_ERR_ARG, "null pointer argument")
+    expect(begin(rects=ARENA + 4), GS_ERR_ALIGN, "rects must be 16-byte aligned")
+    expect(begin(size=need - 1), GS_ERR_WORKSPACE, f"rect_tiles workspace too small: need {need} bytes")
+    expect(begin(ws=None), GS_ERR_WORKSPACE, "rect_tiles workspace too small")
+    expect(L.gs_rect_tiles_end(None, ctypes.byref(b)), GS_ERR_ARG, "null pointer argument")
+    expect(L.gs_rect_tiles_end(ctypes.byref(m), None), GS_ERR_ARG, "null pointer argument")
+
+
+def test_loss_value_refuses_what_the_loss_refuses():
+    L = _lib.lib()
+    lam = ctypes.c_float(0.2)
+    need = L.gs_l1_ssim_workspace_size(3, 16, 16)
+    expect(L.gs_l1_ssim_fwd_value(None, None, 3, 0, 16, lam, None, None, None, None, 0, None), GS_ERR_ARG,
+           "invalid image size")
+    expect(L.gs_l1_ssim_fwd_value(None, None, 3, 16, 16, lam, None, None, None, None, 0, None), GS_ERR_ARG, "null pointer")
+    expect(L.gs_l1_ssim_fwd_value(ARENA, ARENA, 3, 16, 16, lam, None, ARENA, None, ARENA, need - 1, None),
+           GS_ERR_WORKSPACE, f"workspace too small: need {need} bytes")
+
+
 # ---------------------------------------------------------------------------------------
 # Device-side failures (real buffers of the full size; nothing may be written)
 # ---------------------------------------------------------------------------------------
