@@ -828,8 +828,20 @@ __device__ __forceinline__ void group_totals(S& u0, S& u1) {
   asm volatile("" : "+v"(u0), "+v"(u1));
 }
 
-// Reduction of one bucket-splat step (the 3D backward without the |dL/dmean2d| sums, and the toy2d
-// rules). In: the
+// The columns' two sums of every row (even rows t1 = their first pair's, odd rows their second's), the
+// dx factors of row 0 applied, summed over the row's 16 columns.
+template <typename S>
+__device__ __forceinline__ void reduce_rows(S t0, S t1, S dx, bool row0, S& u0, S& u1) {
+  const S f = row0 ? dx : S(1);
+  const S v0 = t0 * f, v1 = v0 * f, v3 = t1 * f;
+  const bool b3 = (threadIdx.x & 8) != 0;
+  u0 = (b3 ? v1 : v0) + dpp<0x128>(b3 ? v0 : v1);  // row_ror:8 = partner lane ^ 8
+  u1 = (b3 ? v3 : t1) + dpp<0x128>(b3 ? t1 : v3);
+  group_totals(u0, u1);
+}
+
+// Reduction of one bucket-splat step (the 3D backward without the |dL/dmean2d| sums, and, with
+// another sum, the toy2d rules). In: the
 // lane's sums over its 4 pixels (one column) of h, h dy, h dy^2 and the three colour sums, and
 // the column's dx. The 4 lanes of a column (lane ^ 16, ^ 32) are summed first, transposing: xor
 // 32 with v_permlane32_swap over the pairs (h, red), (h dy, green), (h dy^2, blue), leaving the
@@ -845,29 +857,30 @@ __device__ __forceinline__ void group_totals(S& u0, S& u1) {
 template <typename S>
 __device__ __forceinline__ void wave_reduce_cols(S sh, S shy, S shyy, S cr, S cg, S cb, S dx, bool row0, S& u0,
                                                  S& u1) {
-  const int lane = threadIdx.x & 63;
   const S s0 = swap32_add(sh, cr), s1 = swap32_add(shy, cg), s2 = swap32_add(shyy, cb);
   const S t0 = swap16_add(s0, s0);  // every row: its quarter's first sum
-  const S t1 = swap16_add(s1, s2);  // even rows s1, odd rows s2
-  const S f = row0 ? dx : S(1);
-  const S v0 = t0 * f, v1 = v0 * f, v3 = t1 * f;
-  const bool b3 = (lane & 8) != 0;
-  u0 = (b3 ? v1 : v0) + dpp<0x128>(b3 ? v0 : v1);  // row_ror:8 = partner lane ^ 8
-  u1 = (b3 ? v3 : t1) + dpp<0x128>(b3 ? t1 : v3);
-  group_totals(u0, u1);
+  reduce_rows(t0, swap16_add(s1, s2), dx, row0, u0, u1);
+}
+
+// The same with a sum of its own for the opacity (toy2d), so, in place of group 2's sum h.
+template <typename S>
+__device__ __forceinline__ void wave_reduce_cols_op(S sh, S shy, S shyy, S so, S cr, S cg, S cb, S dx, bool row0, S& u0,
+                                                    S& u1) {
+  const S s0 = swap32_add(sh, cr), so0 = swap32_add(so, cr), s1 = swap32_add(shy, cg), s2 = swap32_add(shyy, cb);
+  reduce_rows(swap16_add(s0, so0), swap16_add(s1, s2), dx, row0, u0, u1);
 }
 
 // The same of the phase0 rules, whose shape and mean gradients are sums of h a and h b (a = l0 dx +
 // l1 dy, b = l2 dy, formed at each pixel): xor 32 over the pairs (h a, red), (h a dy, green),
-// (h b, blue), (h b dy, h), xor 16 over the pairs of those, the dx factor on the columns' h a. On return
+// (h b, blue), (h b dy, G dL/dalpha), xor 16 over the pairs of those, the dx factor on the columns' h a. On return
 //   g 0: (sum h a, sum h b)            g 1: (sum h a dx, sum h b)
-//   g 2: (sum h a dy, sum h b dy)      g 4: (red, blue)        g 6: (green, sum h)
+//   g 2: (sum h a dy, sum h b dy)      g 4: (red, blue)        g 6: (green, sum G dL/dalpha)
 // (g 3, 5, 7 hold repeats).
 template <typename S>
-__device__ __forceinline__ void wave_reduce_cols_chol(S sha, S shay, S shb, S shby, S sh, S cr, S cg, S cb, S dx,
+__device__ __forceinline__ void wave_reduce_cols_chol(S sha, S shay, S shb, S shby, S so, S cr, S cg, S cb, S dx,
                                                       bool row0, S& u0, S& u1) {
   const int lane = threadIdx.x & 63;
-  const S s0 = swap32_add(sha, cr), s1 = swap32_add(shay, cg), s2 = swap32_add(shb, cb), s3 = swap32_add(shby, sh);
+  const S s0 = swap32_add(sha, cr), s1 = swap32_add(shay, cg), s2 = swap32_add(shb, cb), s3 = swap32_add(shby, so);
   const S t0 = swap16_add(s0, s1), t1 = swap16_add(s2, s3);
   const S v1 = t0 * (row0 ? dx : S(1));
   const bool b3 = (lane & 8) != 0;
@@ -1249,7 +1262,7 @@ __device__ __forceinline__ Staged2D<S> stage2d(const Staged<S>& r, S cut) {
   if constexpr (R == kRulesPhase0) {
     // power = -(a^2 + b^2) / 2, a = l0 dx + l1 dy, b = l2 dy, d = pixel - mean: the mean's gradient is
     // (l0 sum h a, l1 sum h a + l2 sum h b), that of l0 -sum h a dx, of l1 -sum h a dy, of l2
-    // -sum h b dy; the opacity logit's dL/do o (1 - o) = (1 - o) sum h. (Along an elongated rotated
+    // -sum h b dy; the opacity logit's dL/do o (1 - o), dL/do = sum G dL/dalpha. (Along an elongated rotated
     // splat l0 dx and l1 dy cancel: sums of h dx and h dy combined with Q = L L^T afterwards lose what
     // their sizes differ from the gradients'. Error of the mean's gradient against float64 at standard
     // deviations 2:10 / 0.6:60 px: 1.0e-5 / 2.2e-4 with them, so
@@ -1257,15 +1270,14 @@ __device__ __forceinline__ Staged2D<S> stage2d(const Staged<S>& r, S cut) {
     c[0] = -r.s0; c[1] = S(0); c[2] = -r.s1; c[3] = -r.s2;
     c[4] = S(1); c[5] = S(0);
     c[6] = S(0); c[7] = S(1);
-    c[8] = S(0); c[9] = -(S(1) - r.o);
+    c[8] = S(0); c[9] = -(r.o * (S(1) - r.o));
     c[10] = S(-1); c[11] = S(0);
   } else {
-    // power = -1/2 (A dx^2 + 2 B dx dy + C dy^2), d = mean - pixel; dL/do = (sum h) / o, since
-    // h = alpha dL/dalpha and alpha = o G wherever it is not clamped (there h is 0)
+    // power = -1/2 (A dx^2 + 2 B dx dy + C dy^2), d = mean - pixel; dL/do = sum G dL/dalpha
     c[0] = r.s0; c[1] = r.s1; c[2] = r.s1; c[3] = r.s2;
     c[4] = S(0.5); c[5] = S(0);
     c[6] = S(0); c[7] = S(1);
-    c[8] = S(-1) / r.o; c[9] = S(0);
+    c[8] = S(-1); c[9] = S(0);
     c[10] = S(0); c[11] = S(0.5);
   }
   c[12] = S(-1); c[13] = S(0); c[14] = S(0); c[15] = S(-1);
@@ -1319,7 +1331,7 @@ __device__ __forceinline__ double div_unit(double a, double b) { return a / b; }
 // pixel, wave_reduce_cols) with the rule sets' own arithmetic, so that T replays the forward's bits;
 // a row whose lanes' exponents are all at or below the splat's cut skips the exponential.
 // VALU bound. Against a loop that evaluated every row of every entry and reduced twelve sums per
-// splat with wave_reduce12: toy2d 1024^2, 200k splats 192 -> 104 us; phase0 1080p, 50k splats
+// splat with wave_reduce12: toy2d 1024^2, 200k splats 192 -> 105 us; phase0 1080p, 50k splats
 // 247 -> 149 us without the counts, 572 -> 150 + 6.5 us with them.
 // kCount: the bucket's reduced steps and its splat-pixel evaluations (a pixel evaluates every list
 // entry up to its stop) are added, as integers, to slots 9 and 10 of its first splat's gradient
@@ -1432,6 +1444,7 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
       k1 = s1 * dx;
     }
     S sh = S(0), shy = S(0), shyy = S(0), cr = S(0), cg = S(0), cb = S(0);
+    S so = S(0);                // G dL/dalpha: (sum h) / o, less its roundings
     S sha = S(0), shay = S(0);  // (phase0; there shy and shyy sum h b and h b dy)
     uint64_t used = 0;
 #pragma unroll
@@ -1450,7 +1463,8 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
       }
       const bool reach = j < lim[r] && Ru::in_domain(power) && power > cut;
       if (__ballot(reach ? 1 : 0) == 0ull) continue;  // wave-uniform
-      const S raw = o * exp_t(power);
+      const S G = exp_t(power);
+      const S raw = o * G;
       const bool clamped = raw > S(0.99);
       const S alpha = clamped ? S(0.99) : raw;
       const bool take = reach && alpha >= Ru::alpha_min();
@@ -1463,8 +1477,9 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
         cb = fma(w, Gb[r], cb);
         rho[r] = fma(-w, dot, rho[r]);
         const S oma = S(1) - alpha;
-        const S dLda = T[r] * dot - div_unit(rho[r], oma);
-        const S h = clamped ? S(0) : alpha * dLda;  // dL/dpower
+        const S dLda = clamped ? S(0) : T[r] * dot - div_unit(rho[r], oma);
+        const S h = alpha * dLda;  // dL/dpower
+        so = fma(G, dLda, so);
         S hy;
         if constexpr (R == kRulesPhase0) {
           const S ha = h * pa;
@@ -1486,9 +1501,9 @@ __device__ __forceinline__ void bwd_bucket_2d(const BlendArgs<S>& a, int64_t b, 
     ++steps;
     S u0, u1;
     if constexpr (R == kRulesPhase0)
-      wave_reduce_cols_chol(sha, shay, shy, shyy, sh, cr, cg, cb, dx, row0, u0, u1);
+      wave_reduce_cols_chol(sha, shay, shy, shyy, so, cr, cg, cb, dx, row0, u0, u1);
     else
-      wave_reduce_cols(sh, shy, shyy, cr, cg, cb, dx, row0, u0, u1);
+      wave_reduce_cols_op(sh, shy, shyy, so, cr, cg, cb, dx, row0, u0, u1);
     const S g = fma(-sp.co[2 * pair], u0, -(sp.co[2 * pair + 1] * u1));
     if (owner) atomic_add_grad(a.grad_rec + static_cast<int64_t>(s_id[j]) * kGrad2D + slot, g);
   }

@@ -602,3 +602,33 @@ def test_phase0_backward_of_rotated_splats(s1, s2, dtype, exact):
     print(f"phase0 {s1}:{s2} {dtype.__name__}: mean {e[0]:.2e} (plain {e_plain[0]:.2e}), shape {e[1]:.2e} "
           f"(plain {e_plain[1]:.2e})")
     assert (e <= 3 * e_plain + 2 * np.finfo(dtype).eps).all()
+
+
+@pytest.mark.parametrize("dtype,exact", [(np.float32, np.float64), (np.float64, np.longdouble)])
+def test_toy2d_opacity_gradient_of_small_splats(dtype, exact):
+    """dL/do = sum G dL/dalpha of small toy2d splats, each alone, of opacities whose reciprocals round
+    worst: the root mean square error of that sum in the same type, whose exponential is no better than
+    the kernel's, and not that of sum alpha dL/dalpha divided by o."""
+    W = H = 16
+    rng = np.random.default_rng(3)
+    o = rng.uniform(0.236, 0.25, 40_000).astype(dtype)
+    o = o[np.argsort(np.abs((dtype(1) / o).astype(exact) * o.astype(exact) - 1))[-96:]]
+    err = []
+    for op in o:
+        mx, my = (dtype(x) for x in rng.uniform(6, 10, 2))
+        A = dtype(rng.uniform(0.5, 2))
+        col, gi = rng.uniform(0.2, 1, 3).astype(dtype), rng.uniform(0, 1, (3, H, W)).astype(dtype)
+        t = [cuda(np.array(x, dtype)) for x in ([[mx, my]], [[A, 0, A]], [col], [op])]
+        rec = R2.pack(R2.TOY2D, *t)
+        rg, ids, bo = (cuda(np.array(x, np.int32)) for x in ([[0, 1]], [0], [0, 1]))
+        image, _, nc, _, tmax, ckpt = R2.blend_fwd(R2.TOY2D, rec, rg, 2, ids, bo, 1, W, H)
+        g = R2.blend_bwd_bucket(R2.TOY2D, rec, rg, 2, ids, bo, bo[:1].contiguous(), 1, W, H, image, cuda(gi), nc, tmax, ckpt)
+        y, x = np.nonzero(nc.cpu().numpy())
+        ref, plain = (
+            (np.exp(dt(-0.5) * (A.astype(dt) * (mx.astype(dt) - x.astype(dt)) ** 2 + A.astype(dt) *
+                                (my.astype(dt) - y.astype(dt)) ** 2)) *
+             (gi[:, y, x].astype(dt) * col.astype(dt)[:, None]).sum(0)).sum() for dt in (exact, dtype))
+        err.append([float(abs(exact(v) - ref) / ref) for v in (R2.split_grads(g)[2].cpu().numpy()[0], plain)])
+    e, e_plain = np.sqrt(np.mean(np.square(err), 0))
+    print(f"toy2d opacity {dtype.__name__}: {e:.2e} (plain {e_plain:.2e})")
+    assert e <= e_plain
