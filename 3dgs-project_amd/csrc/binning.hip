@@ -5,10 +5,10 @@
 // instances emitted in Gaussian-index order, obtained in two levels: a stable 32-bit sort of
 // the Gaussians by depth (N keys), emission of the instances in that order, and a stable sort
 // of the instances by tile (M keys, ceil(log2 T) bits). The first is a bucket sort up to 1M keys
-// (gs_sample_sort.h); otherwise each sort is LSD radix, reduce-then-scan per digit: a histogram kernel, a device-wide exclusive scan of the
-// digit-major histogram table, and a scatter kernel that ranks keys stably inside its
-// workgroup. No kernel waits on another workgroup, so there is no forward-progress
-// requirement.
+// (gs_sample_sort.h); otherwise each sort is LSD radix, reduce-then-scan per digit: a histogram
+// kernel, a device-wide exclusive scan of the digit-major histogram table, and a scatter kernel that
+// ranks keys stably inside its workgroup. No kernel waits on another workgroup, so there is no
+// forward-progress requirement.
 #include "gs_host.h"
 
 namespace gs {
@@ -866,7 +866,7 @@ __global__ __launch_bounds__(256) void tile_bounds_kernel(const uint32_t* __rest
 }
 
 // One workgroup of kBoThreads: the exclusive scans of the tiles' instance counts (count_of(t)) and of
-// their bucket counts ceil(len / 32); put(t, len, instances before, buckets before) for every tile.
+// their bucket counts ceil(len / 32); put(t, len, instances before) for every tile.
 // A wavefront takes 512 consecutive tiles in rounds of 64, so that reads and writes are coalesced
 // (with eight consecutive tiles per thread the writes of 8160 tiles took 20 us of one CU).
 constexpr int kBoThreads = 1024;
@@ -1000,19 +1000,18 @@ __global__ void rect_counts_kernel(const int4* __restrict__ rects, int64_t n, in
 // The tile lists in (tile, depth) order without sorting the M instances. A Gaussian's tiles
 // in one tile row form a run of columns, its row span (tx0, nt); two counting passes over the
 // spans place every instance once:
-//   rows     the Gaussians in depth order, kRowChunk per wavefront: each chunk counts its
-//            non-empty (Gaussian, tile row) items per row (span_rows_kernel<count>), a scan of
-//            each row over the chunks gives every chunk its offsets (rs_rowscan_kernel), and
-//            each chunk writes its spans there (span_rows_kernel<write>): the spans of one row
-//            are contiguous and in depth order. Each row's spans start at a multiple of
-//            kSpanChunk.
-//   columns  kSpanChunk spans per wavefront, all of one row: each chunk counts its instances
-//            per column with a difference array over the columns (span_col_count_kernel); a
-//            scan of every (row, column) over the row's chunks gives every chunk its offsets
-//            and the tile counts, and the last workgroup to finish scans the tile counts into
-//            ranges and bucket offsets (span_col_scan_kernel); each chunk expands its spans into
-//            instances and writes the Gaussian of each at its tile's start + the chunk's offset
-//            + its rank among the chunk's instances in that column (span_col_write_kernel).
+//   rows     the Gaussians in depth order, kRowChunk per workgroup: each chunk gathers its
+//            non-empty (Gaussian, tile row) spans and counts them per row (span_gather_kernel), a
+//            scan of each row over the chunks gives every chunk its offsets (rs_rowscan_kernel), and
+//            each chunk writes its spans there (span_place_kernel): the spans of one row are
+//            contiguous and in depth order. Each row's spans start at a multiple of kSpanChunk.
+//   columns  kSpanChunk spans per workgroup, all of one row: each chunk counts its instances per
+//            column with a difference array over the columns (span_col_count_kernel); a workgroup
+//            per row scans its columns over the row's chunks: every chunk's offsets and the tile
+//            counts (span_col_scan_kernel); one workgroup scans the tile counts into ranges and
+//            bucket offsets (tile_scan_kernel); each chunk sorts its instances by column in LDS, a
+//            batch at a time, and writes every column's run at its tile's start + the chunk's
+//            offset + the batch's (span_col_write_kernel).
 // Ranks inside a chunk come from coverage masks (of a row, of a column) whose bits are in item
 // order, and chunks keep their order through the scans, so both passes are stable and a tile's list
 // holds its Gaussians in depth order: the order of a stable sort by tile of the instances
@@ -1027,7 +1026,7 @@ constexpr int kRowChunk = 256;     // depth positions per workgroup in the row p
 constexpr int kRowBand = 16;
 constexpr int kSpanChunk = 1024;   // spans per workgroup in the column pass
 constexpr int kSpanWaves = 4;      // wavefronts per workgroup (256 threads)
-constexpr int kColScanThreads = kBoThreads;  // the last workgroup runs tile_scan_block
+constexpr int kColScanThreads = kBoThreads;
 
 __device__ __forceinline__ int align4i(int v) { return (v + 3) & ~3; }
 
@@ -1556,8 +1555,12 @@ __global__ __launch_bounds__(kBoThreads) void tile_scan_kernel(const uint32_t* _
 // count where that word is set.
 constexpr int kDiffThreads = 1024;
 constexpr int64_t kDiffMax = 16000;       // array entries (below 64 KB of LDS): canvases up to 2000 x 2000
-constexpr int64_t kDiffDirect = 8192;     // rectangles one workgroup takes alone
-constexpr int64_t kDiffPer = 16384;       // rectangles per workgroup beyond
+// Rectangles that one workgroup takes alone, rectangles per workgroup beyond, and the most workgroups.
+// Both kernels, 64 x 64 tiles: 2048 rectangles 14.8 us alone (17.8 with workgroups), 8192 16.5 (19.0),
+// 16384 18.6 (21.2), 32768 23.2 (21.8), 200k 70 (25): the two cross between 16384 and 32768. With 16
+// workgroups of 8192 instead: 16384 19.9, 200k 22.8, 1M 36 (8 of 16384: 52).
+constexpr int64_t kDiffDirect = 8192;
+constexpr int64_t kDiffPer = 16384;
 constexpr int kDiffGroups = 8;
 constexpr unsigned long long kDiffOther = ~0ull;
 
@@ -1896,11 +1899,13 @@ static EmitLayout emit_layout(int64_t m, int n_tiles) {
 static bool span_binning(int tiles_x, int tiles_y) { return tiles_x <= kSpanMaxDim && tiles_y <= kSpanMaxDim; }
 
 // Which fill a canvas and Gaussian count take: the span binning on canvases of at most
-// kSpanMaxDim tiles per side from kSpanMinGaussians Gaussians on (below that, the radix path was
-// measured faster: 1M Gaussians at 1297x840 bin in 127 us by radix and 152 us by spans, 3M at
-// 1957x1091 in 1.01 ms by radix and 0.81 ms by spans), unless flags force a path. The choice
-// needs no instance count, so the depth ordering knows beforehand whether the fill needs the
-// instance offsets.
+// kSpanMaxDim tiles per side from kSpanMinGaussians Gaussians on, unless flags force a path. The
+// choice needs no instance count, so the depth ordering knows beforehand whether the fill needs the
+// instance offsets. The line lies where the radix path was the faster one when it was drawn (1M
+// Gaussians at 1297x840: 127 us by radix, 152 by spans); with today's kernels it lies too high. Whole
+// inference forwards, us by radix / by spans: 100k at 800x800 176 / 163, 300k at 1001x667 209 / 200 to
+// 227, 700k at 1297x840 294 / 292, 1M there 348 / 343, 1.5M 465 / 444, 1M at 1957x1091 700 / 507, 2M
+// 1226 / 814, 3M 1708 / 1074.
 constexpr int64_t kSpanMinGaussians = 2000000;
 
 static bool use_spans(int64_t n, int tiles_x, int tiles_y, int flags) {

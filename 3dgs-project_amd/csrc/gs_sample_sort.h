@@ -24,7 +24,8 @@
 // against 169 without equal keys), so it is taken beyond kSsMaxKeys. Reserving bucket space
 // by atomics instead of count and rowscan was slower (one kernel of 46 us for count, rowscan and
 // scatter together at 1M: a returning atomic per workgroup and bucket). No workgroup waits on
-// another.
+// another. Over other distributions (a third culled, 37 or 1000 distinct depths, tight clusters,
+// sorted; 2k to 1M keys) it is between 0.14 and 1.05 times the radix sort's time.
 #pragma once
 
 namespace gs {
@@ -36,15 +37,19 @@ constexpr int kSsBits = 9;
 constexpr int kSsMaxBuckets = 1 << kSsBits;
 constexpr int kSsOver = 8;      // samples per bucket
 constexpr int kSsSmall = 4096;  // keys sorted by one workgroup
-// Keys per bucket aimed at: a quarter of the LDS capacity of its workgroup. A bucket beyond the
-// capacity (once in 1e4 sorts, for any input, since the sampled positions are hashed) is sorted
-// through global memory. Larger buckets cost less per key, but fewer workgroups than CUs would
-// leave the chip idle.
+// Keys per bucket aimed at: a quarter of the LDS capacity of its workgroup. Larger buckets cost less
+// per key, but fewer workgroups than CUs would leave the chip idle. A bucket beyond the capacity is
+// sorted by its workgroup through global memory, at about 10 us per 1000 keys. The sampled positions
+// are hashed from n alone: an input that does not follow them (whatever its order and its values'
+// distribution) has such a bucket, slightly beyond the capacity, once in 1e4 inputs, but then on every
+// sort of that input; one made against the positions can bring nearly all keys into one bucket (30k
+// keys 0.35 ms, 100k 1.1, 1M 10.7; the radix sort takes 0.05 to 0.08).
 constexpr int64_t kSsLargeFrom = int64_t(512) << 10;
 static int ss_mean(int64_t n) { return n < kSsLargeFrom ? 1024 : 2048; }
 constexpr int64_t kSsMaxKeys = int64_t(1) << 20;
 
-__device__ __forceinline__ uint32_t ss_hash(uint32_t x) {  // (any mixing of the bits serves)
+// The published integer mixer lowbias32 (C. Wellons); any mixing of the bits would serve.
+__device__ __forceinline__ uint32_t ss_hash(uint32_t x) {
   x ^= x >> 16;
   x *= 0x7feb352du;
   x ^= x >> 15;
